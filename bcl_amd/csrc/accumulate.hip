@@ -2,10 +2,18 @@
 // SparseHashAccumulator::get_matrix (bcl/containers/sequential/SparseHashAccumulator.hpp:101-182) and of the
 // pairwise sum_tiles_cusparse fold (bcl/containers/experimental/cuda/sequential/cusparse_util.cuh:251-265).
 //
-// The sum is computed as one SpGEMM: C = [T_1 T_2 ... T_K] * [I; I; ...; I], where the left operand stacks the tiles
-// side by side (row i of it is the concatenation of row i of every tile, tile t's columns shifted by t * n) and the
-// right operand stacks K identities. Every product is x * 1 (exact), so the two-phase SpGEMM returns exactly the
-// union pattern, sorted, with each entry summed in float64 and rounded once.
+// The tiles' rows are sorted, so the sum is a K-way merge. The rows are cut into pieces of at most kAccCap entries
+// (whole short rows, or a column range of a long row); one workgroup loads a piece into LDS, merges its K sorted runs
+// as a tree of merge-path merges, and equal (row, column) pairs, now adjacent and in tile order, are summed in
+// float64 and rounded once. A counting merge sizes the rows, a scan places them, a second merge writes them.
+//
+// Measured: eight R-MAT scale 16 tiles (11.2 M entries, fp32) 11.0 ms through the general path, 0.91 ms here.
+//
+// Tiles whose columns are not strictly increasing within each row, and sums of more than kAccMaxTiles tiles (one lane
+// per tile sets a piece up), take the general path: one SpGEMM [T_1 T_2 ... T_K] * [I; I; ...; I], where the left operand stacks the tiles side by side
+// (row i of it is the concatenation of row i of every tile, tile t's columns shifted by t * n) and the right operand
+// stacks K identities. Every product is x * 1 (exact), so the two-phase SpGEMM returns exactly the union pattern,
+// sorted, with each entry summed in float64 and rounded once.
 #include <algorithm>
 
 #include "spgemm.hpp"
@@ -57,7 +65,7 @@ __global__ void k_ident_stack(int64_t rows, int64_t n, int64_t* rp, int* col, T*
 }
 
 template <typename T, typename RP>
-static void accumulate_impl(bclx_handle* h, int K, const bclx_csr* tiles, bclx_csr* C) {
+static void accumulate_spgemm(bclx_handle* h, int K, const bclx_csr* tiles, bclx_csr* C) {
   const int64_t m = tiles[0].m, n = tiles[0].n;
   hipStream_t s = h->stream;
   std::vector<TileIn<T, RP>> tin(K);
@@ -65,7 +73,6 @@ static void accumulate_impl(bclx_handle* h, int K, const bclx_csr* tiles, bclx_c
     tin[t] = {static_cast<const RP*>(tiles[t].row_ptr), tiles[t].col_idx, static_cast<const T*>(tiles[t].vals)};
   int64_t total_in = 0;
   for (int t = 0; t < K; t++) total_in += tiles[t].nnz;
-  BCLX_REQUIRE(K * n < INT32_MAX, BCLX_ERR_OVERFLOW, "K * n must fit int32 (stacked column index)");
   // workspace: tile table, counts, stacked A (int64 row_ptr), stacked identity B
   DevBuf tin_d(sizeof(TileIn<T, RP>) * K), cnt(sizeof(int32_t) * (m + 1)), srp(sizeof(int64_t) * (m + 1));
   DevBuf scol(sizeof(int) * std::max<int64_t>(total_in, 1)), sval(sizeof(T) * std::max<int64_t>(total_in, 1));
@@ -116,6 +123,461 @@ static void accumulate_impl(bclx_handle* h, int K, const bclx_csr* tiles, bclx_c
     C->nnz = nnz;
   }
   BCLX_HIP(hipStreamSynchronize(s));  // the workspace above is released on return
+}
+
+// ------------------------------------------------------------------------------------------------------------
+// merge path
+// ------------------------------------------------------------------------------------------------------------
+
+constexpr int kAccThreads = 256;
+constexpr int kAccItems = 9;                       // merged entries per thread (odd: LDS bank spread)
+constexpr int kAccCap = kAccThreads * kAccItems;   // 2304 entries per piece
+constexpr int kAccTarget = 1024;                   // a piece holds the rows whose weight offset lies in one such span
+constexpr int kAccMaxTiles = 64;                   // one lane per tile in the setup of a piece
+constexpr int kAccSlotBits = 12;                   // key = local row << 43 | column << 12 | slot
+static_assert(kAccCap <= (1 << kAccSlotBits) && 2 * kAccTarget <= kAccCap && kAccTarget + kAccMaxTiles + 1 <= kAccCap,
+              "a piece fits its slots");
+static_assert(kAccTarget <= 1024, "a local row fits 10 bits beside the tile number in a mark");
+
+// A piece of a long row: entries q of its npieces; bounds of piece p at bound[p * K + t].
+struct AccPiece {
+  int32_t row, q, npieces;
+};
+
+template <typename T, typename RP>
+struct AccDev {
+  TileIn<T, RP> tile[kAccMaxTiles];
+  int32_t K;
+  int64_t m, n;
+  int64_t* woff;         // m + 1: offset of each row in units of entries + 1 per row
+  int32_t* cnt;          // m: row weights, then entries of each row of C
+  int64_t* off;          // m + 1: row offsets of C
+  int64_t nchunks;       // spans of kAccTarget weight
+  int32_t* chunk;        // 2 * nchunks: first row and end row of the short rows that start in each span
+  AccPiece* piece;       // pieces of rows longer than kAccTarget
+  int32_t max_pieces;
+  int64_t* bound;        // max_pieces * K: first position of each piece in each tile
+  int32_t* piece_cnt;    // entries of C per piece
+  int32_t* npieces;      // pieces in use
+  int32_t* bad;          // [0] set by the cut (descriptors disagree with the row_ptrs: nothing may use the pieces),
+                         // [1] set by the merge (columns not strictly increasing): the general path takes the sum
+};
+
+// row weights: entries over all tiles, plus one (so a span of weights holds a bounded number of empty rows too)
+template <typename T, typename RP>
+__global__ __launch_bounds__(256) void k_acc_weight(AccDev<T, RP> D) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i == 0) {
+    *D.npieces = 0;
+    D.bad[0] = D.bad[1] = 0;
+  }
+  for (int64_t c = i; c < 2 * D.nchunks; c += (int64_t)gridDim.x * 256) D.chunk[c] = 0;
+  if (i >= D.m) return;
+  long long c = 1;
+  for (int t = 0; t < D.K; t++) c += (long long)(D.tile[t].rp[i + 1] - D.tile[t].rp[i]);
+  D.cnt[i] = (int32_t)c;
+}
+
+// Cuts the rows into pieces: span c of weights [c * kAccTarget, (c + 1) * kAccTarget) owns the rows that start in it
+// (together at most 2 * kAccTarget - 1 entries: all but the last end inside the span), except a last row of more than
+// kAccTarget entries, which is listed as pieces of its own. One thread per row.
+template <typename T, typename RP>
+__global__ __launch_bounds__(256) void k_acc_chunks(AccDev<T, RP> D) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i > D.m) return;
+  const int64_t w = D.woff[i];
+  const int64_t c = w / kAccTarget;
+  if (i > 0) {
+    const int64_t pw = D.woff[i - 1], pc = pw / kAccTarget;
+    if ((i == D.m || pc != c) && pc < D.nchunks) D.chunk[2 * pc + 1] = (int32_t)(w - pw - 1 > kAccTarget ? i - 1 : i);
+  }
+  if (i == D.m) return;
+  D.cnt[i] = 0;
+  if (i == 0 || D.woff[i - 1] / kAccTarget != c) {
+    if (c < D.nchunks) D.chunk[2 * c] = (int32_t)i;
+    else D.bad[0] = 1;  // more entries than the descriptors say
+  }
+  const int64_t len = D.woff[i + 1] - w - 1;
+  if (len > kAccTarget) {
+    const int P = (int)((len + kAccTarget - 1) / kAccTarget);
+    const int base = atomicAdd(D.npieces, P);
+    if (base < 0 || base + P > D.max_pieces) {
+      D.bad[0] = 1;
+      return;
+    }
+    for (int q = 0; q < P; q++) D.piece[base + q] = AccPiece{(int32_t)i, q, P};
+  }
+}
+
+// First positions of a long row's pieces: piece q starts at the largest column c before which the row has at most
+// q * ceil(len / P) entries. One wavefront per piece, one tile per lane: a binary search over the columns, each step
+// a binary search of every tile's row within the bounds the earlier steps left. A piece then holds at most
+// ceil(len / P) + K entries.
+template <typename T, typename RP>
+__global__ __launch_bounds__(256) void k_acc_split(AccDev<T, RP> D) {
+  const int lane = threadIdx.x & 63;
+  if (D.bad[0]) return;
+  const int np = *D.npieces;
+  for (int p = blockIdx.x * 4 + (threadIdx.x >> 6); p < np; p += gridDim.x * 4) {  // wave-uniform
+    const AccPiece pc = D.piece[p];
+    const bool live = lane < D.K;
+    const int* col = live ? D.tile[lane].col : nullptr;
+    int64_t lo = live ? (int64_t)D.tile[lane].rp[pc.row] : 0;
+    int64_t hi = live ? (int64_t)D.tile[lane].rp[pc.row + 1] : 0;
+    const int64_t first = lo;
+    const int64_t len = wave_sum<long long>(hi - lo);
+    const int64_t want = pc.q * ((len + pc.npieces - 1) / pc.npieces);
+    int64_t clo = 0, chi = pc.q == 0 ? 1 : D.n;
+    while (chi - clo > 1) {
+      const int64_t mid = (clo + chi) >> 1;
+      int64_t a = lo, b = hi;  // first position with column >= mid
+      while (a < b) {
+        const int64_t x = (a + b) >> 1;
+        if ((int64_t)col[x] < mid) a = x + 1;
+        else b = x;
+      }
+      if (wave_sum<long long>(a - first) <= want) {
+        clo = mid;
+        lo = a;
+      } else {
+        chi = mid;
+        hi = a;
+      }
+    }
+    if (live) D.bound[(int64_t)p * D.K + lane] = lo;
+  }
+}
+
+// One workgroup per piece (blocks below nlong: long-row pieces, strided; then one block per span of short rows).
+// NUM false: entries of C per row (cnt) and per long-row piece; NUM true: the entries, at off[].
+// Bound by LDS reads of the merge tree (log2 K levels, about two 8-byte reads per entry and level) and the latency of
+// the piece's loads; five workgroups per CU (fp32) cover each other's.
+template <bool NUM, typename T, typename RP>
+__global__ __launch_bounds__(kAccThreads) void k_acc_merge(AccDev<T, RP> D, int nlong, int* c_col, T* c_val) {
+  __shared__ unsigned long long s_key[kAccCap];
+  __shared__ T s_val[NUM ? kAccCap : 1];
+  __shared__ unsigned s_mark[kAccCap];  // tile << 10 | local row of each slot; then entries per local row
+  __shared__ int s_seg[kAccMaxTiles + 1];
+  __shared__ int64_t s_beg[kAccMaxTiles];
+  __shared__ const int* s_tcol[kAccMaxTiles];
+  __shared__ const T* s_tval[kAccMaxTiles];
+  __shared__ unsigned s_scan[kAccThreads / 64 + 1];
+  __shared__ long long s_base;
+  const int tid = threadIdx.x, K = D.K;
+  if (D.bad[0]) return;  // written by an earlier kernel only
+  const bool is_long = (int)blockIdx.x < nlong;
+  const int np = is_long ? *D.npieces : 1;
+  for (int p = is_long ? (int)blockIdx.x : 0; p < np; p += nlong > 0 && is_long ? nlong : 1) {
+    // the piece's K runs: [beg, beg + len) of each tile, laid out one after the other in the slots
+    int row0, nrows;
+    AccPiece pc{0, 0, 0};
+    if (is_long) {
+      pc = D.piece[p];
+      row0 = pc.row;
+      nrows = 1;
+    } else {
+      const int64_t c = (int64_t)blockIdx.x - nlong;
+      row0 = D.chunk[2 * c];
+      nrows = D.chunk[2 * c + 1] - row0;
+      if (nrows <= 0) return;
+    }
+    if (tid < 64) {
+      int64_t beg = 0, end = 0;
+      if (tid < K) {
+        if (is_long) {
+          beg = D.bound[(int64_t)p * K + tid];
+          end = pc.q + 1 < pc.npieces ? D.bound[(int64_t)(p + 1) * K + tid] : (int64_t)D.tile[tid].rp[row0 + 1];
+        } else {
+          beg = (int64_t)D.tile[tid].rp[row0];
+          end = (int64_t)D.tile[tid].rp[row0 + nrows];
+        }
+        s_beg[tid] = beg;
+        s_tcol[tid] = D.tile[tid].col;
+        if (NUM) s_tval[tid] = D.tile[tid].val;
+      }
+      const bool back = end < beg;  // only possible when the row is not sorted
+      const int len = back ? 0 : (int)(end - beg < kAccCap ? end - beg : kAccCap);
+      const int inc = wave_incl_scan(len);
+      if (__ballot(back) != 0ull && tid == 0) D.bad[1] = 1;
+      if (tid < K) s_seg[tid] = inc - len;
+      if (tid == 63) s_seg[K] = inc;
+      if (NUM && is_long) {  // entries of the row's earlier pieces
+        long long before = 0;
+        for (int q = tid; q < pc.q; q += 64) before += D.piece_cnt[p - pc.q + q];
+        before = wave_sum<long long>(before);
+        if (tid == 0) s_base = D.off[row0] + before;
+      } else if (NUM && tid == 0) {
+        s_base = D.off[row0];
+      }
+    }
+    for (int s = tid; s < kAccCap; s += kAccThreads) s_mark[s] = 0;
+    __syncthreads();
+    const int E = s_seg[K];
+    if (E > kAccCap) {  // only possible when a row is not sorted or a row_ptr changed meanwhile
+      if (tid == 0) D.bad[1] = 1;
+      return;
+    }
+    // the first slot of every (tile, row) run is marked; a running maximum gives each slot its tile and row
+    for (int x = tid; x < K * nrows; x += kAccThreads) {
+      const int t = x / nrows, r = x - t * nrows;
+      if (is_long) {
+        if (s_seg[t + 1] > s_seg[t]) s_mark[s_seg[t]] = (unsigned)t << 10;
+      } else {
+        const RP* rp = D.tile[t].rp + row0 + r;
+        const int64_t a = (int64_t)rp[0] - s_beg[t], b = (int64_t)rp[1] - s_beg[t];
+        if (b > a && a >= 0 && s_seg[t] + a < E) s_mark[s_seg[t] + a] = (unsigned)t << 10 | (unsigned)r;
+      }
+    }
+    __syncthreads();
+    int vt = (E + kAccThreads - 1) / kAccThreads;
+    vt |= 1;
+    const int s0 = tid * vt;
+    {
+      unsigned run = 0;
+      for (int v = 0; v < vt; v++) run = max(run, s_mark[s0 + v]);
+      unsigned inc = run;
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const unsigned t = __shfl_up(inc, d, 64);
+        if ((tid & 63) >= d) inc = max(inc, t);
+      }
+      if ((tid & 63) == 63) s_scan[tid >> 6] = inc;
+      unsigned before = __shfl_up(inc, 1, 64);
+      if ((tid & 63) == 0) before = 0;
+      __syncthreads();
+      for (int w = 0; w < (tid >> 6); w++) before = max(before, s_scan[w]);
+      for (int v = 0; v < vt; v++) {
+        before = max(before, s_mark[s0 + v]);
+        s_mark[s0 + v] = before;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < kAccItems; v++) {
+      const int s = v * kAccThreads + tid;
+      if (s < E) {
+        const unsigned mk = s_mark[s];
+        const int t = (int)(mk >> 10);
+        const int64_t q = s_beg[t] + (s - s_seg[t]);
+        const int c = s_tcol[t][q];
+        if (is_long && s == s_seg[t] && q > (int64_t)D.tile[t].rp[row0] && s_tcol[t][q - 1] >= c) D.bad[1] = 1;
+        s_key[s] = (unsigned long long)(mk & 1023u) << (31 + kAccSlotBits) |
+                   (unsigned long long)((unsigned)c & 0x7fffffffu) << kAccSlotBits | (unsigned)s;
+        if (NUM) s_val[s] = s_tval[t][q];
+      }
+    }
+    __syncthreads();
+    if (!NUM) {  // each run must be strictly increasing in (row, column)
+#pragma unroll
+      for (int v = 0; v < kAccItems; v++) {
+        const int s = v * kAccThreads + tid;
+        if (s > 0 && s < E && (s_mark[s] >> 10) == (s_mark[s - 1] >> 10) &&
+            (s_key[s] >> kAccSlotBits) <= (s_key[s - 1] >> kAccSlotBits))
+          D.bad[1] = 1;
+      }
+    }
+    // merge tree: at width w, runs of w tiles are merged pairwise; thread tid produces slots [s0, s0 + vt)
+    for (int w = 1; w < K; w *= 2) {
+      unsigned long long out[kAccItems];
+      int a = 0, a1 = 0, b = 0, b1 = -1;  // next positions and ends of the two runs being merged
+#pragma unroll
+      for (int v = 0; v < kAccItems; v++) {
+        const int s = s0 + v;
+        if (v < vt && s < E) {
+          if (s >= b1) {  // the pair of runs holding slot s, and how much of each comes before s (merge path)
+            int t = 0;    // last tile whose first slot is at or before s
+            for (int step = kAccMaxTiles / 2; step > 0; step >>= 1)
+              if (t + step < K && s_seg[t + step] <= s) t += step;
+            const int t0 = t / (2 * w) * (2 * w);
+            const int a0 = s_seg[t0];
+            a1 = s_seg[t0 + w < K ? t0 + w : K];
+            b1 = s_seg[t0 + 2 * w < K ? t0 + 2 * w : K];
+            const int d = s - a0;
+            int lo = d > b1 - a1 ? d - (b1 - a1) : 0, hi = d < a1 - a0 ? d : a1 - a0;
+            while (lo < hi) {
+              const int mid = (lo + hi) >> 1;
+              if (s_key[a0 + mid] < s_key[a1 + d - 1 - mid]) lo = mid + 1;
+              else hi = mid;
+            }
+            a = a0 + lo;
+            b = a1 + d - lo;
+          }
+          const unsigned long long ka = a < a1 ? s_key[a] : ~0ull, kb = b < b1 ? s_key[b] : ~0ull;
+          out[v] = ka < kb ? ka : kb;
+          if (ka < kb) a++;
+          else b++;
+        }
+      }
+      __syncthreads();
+#pragma unroll
+      for (int v = 0; v < kAccItems; v++)
+        if (v < vt && s0 + v < E) s_key[s0 + v] = out[v];
+      __syncthreads();
+    }
+    // compress: an entry of C starts where the (row, column) changes
+    unsigned heads = 0;
+#pragma unroll
+    for (int v = 0; v < kAccItems; v++) {
+      const int s = s0 + v;
+      if (v < vt && s < E && (s == 0 || (s_key[s - 1] >> kAccSlotBits) != (s_key[s] >> kAccSlotBits))) heads |= 1u << v;
+    }
+    unsigned total;
+    const unsigned before = block_excl_scan<kAccThreads, unsigned>((unsigned)__popc(heads), &total, s_scan);
+    if constexpr (!NUM) {
+      if (is_long) {
+        if (tid == 0) {
+          D.piece_cnt[p] = (int)total;
+          atomicAdd(&D.cnt[row0], (int)total);
+        }
+      } else {
+        for (int r = tid; r < nrows; r += kAccThreads) s_mark[r] = 0;
+        __syncthreads();
+        int r = -1, c = 0;
+#pragma unroll
+        for (int v = 0; v < kAccItems; v++) {
+          if (heads >> v & 1u) {
+            const int rr = (int)(s_key[s0 + v] >> (31 + kAccSlotBits));
+            if (rr != r) {
+              if (c) atomicAdd(&s_mark[r], (unsigned)c);
+              r = rr;
+              c = 0;
+            }
+            c++;
+          }
+        }
+        if (c) atomicAdd(&s_mark[r], (unsigned)c);
+        __syncthreads();
+        for (int x = tid; x < nrows; x += kAccThreads) D.cnt[row0 + x] = (int)s_mark[x];
+      }
+    } else {
+      double sum[kAccItems];
+      int col[kAccItems];
+#pragma unroll
+      for (int v = 0; v < kAccItems; v++) {
+        if (heads >> v & 1u) {
+          const unsigned long long k = s_key[s0 + v];
+          const unsigned long long rc = k >> kAccSlotBits;
+          col[v] = (int)(rc & 0x7fffffffu);
+          sum[v] = (double)s_val[k & ((1u << kAccSlotBits) - 1u)];
+          for (int q = s0 + v + 1; q < E; q++) {  // the same entry in later tiles, in tile order
+            const unsigned long long kq = s_key[q];
+            if ((kq >> kAccSlotBits) != rc) break;
+            sum[v] += (double)s_val[kq & ((1u << kAccSlotBits) - 1u)];
+          }
+        }
+      }
+      __syncthreads();
+      // staged by rank in LDS, then stored with unit stride
+      int* s_col = reinterpret_cast<int*>(s_key);
+      int r = (int)before;
+#pragma unroll
+      for (int v = 0; v < kAccItems; v++)
+        if (heads >> v & 1u) {
+          s_col[r] = col[v];
+          s_val[r] = (T)sum[v];
+          r++;
+        }
+      __syncthreads();
+      const long long base = s_base;
+      for (int x = tid; x < (int)total; x += kAccThreads) {
+        __builtin_nontemporal_store(s_col[x], &c_col[base + x]);
+        __builtin_nontemporal_store(s_val[x], &c_val[base + x]);
+      }
+    }
+    __syncthreads();  // the next piece reuses the LDS
+  }
+}
+
+// row_ptr of C from the row offsets
+static void write_rowptr(hipStream_t s, const int64_t* off, int64_t m, void* row_ptr, int ptr_width) {
+  const unsigned g = div_up(m + 1, 256);
+  if (ptr_width == 8)
+    hipLaunchKernelGGL(k_rowptr<int64_t>, dim3(g), dim3(256), 0, s, off, (int64_t)0, m, static_cast<int64_t*>(row_ptr));
+  else
+    hipLaunchKernelGGL(k_rowptr<int32_t>, dim3(g), dim3(256), 0, s, off, (int64_t)0, m, static_cast<int32_t*>(row_ptr));
+  BCLX_HIP(hipGetLastError());
+}
+
+// The merge path; false when the tiles need the general path (nothing of C is written then).
+template <typename T, typename RP>
+static bool accumulate_merge(bclx_handle* h, int K, const bclx_csr* tiles, bclx_csr* C) {
+  const int64_t m = tiles[0].m, n = tiles[0].n;
+  if (K > kAccMaxTiles || m == 0) return false;
+  int64_t total_in = 0;
+  for (int t = 0; t < K; t++) total_in += tiles[t].nnz;
+  const int64_t max_pieces = 2 * (total_in / kAccTarget) + 1;
+  if (m >= INT32_MAX || max_pieces >= INT32_MAX / 2) return false;
+  hipStream_t s = h->stream;
+  AccDev<T, RP> D;
+  for (int t = 0; t < K; t++)
+    D.tile[t] = {static_cast<const RP*>(tiles[t].row_ptr), tiles[t].col_idx, static_cast<const T*>(tiles[t].vals)};
+  D.K = K;
+  D.m = m;
+  D.n = n;
+  D.nchunks = (total_in + m) / kAccTarget + 1;
+  D.max_pieces = (int32_t)max_pieces;
+  Arena ws;  // in the handle's scratch: this call waits for the stream before it returns
+  const size_t o_woff = ws.reserve(sizeof(int64_t) * (m + 4)), o_cnt = ws.reserve(sizeof(int32_t) * (m + 4)),
+               o_off = ws.reserve(sizeof(int64_t) * (m + 4)), o_chunk = ws.reserve(sizeof(int32_t) * 2 * D.nchunks),
+               o_piece = ws.reserve(sizeof(AccPiece) * max_pieces), o_bound = ws.reserve(sizeof(int64_t) * max_pieces * K),
+               o_pcnt = ws.reserve(sizeof(int32_t) * max_pieces), o_part = ws.reserve(sizeof(long long) * scan_partials(m)),
+               o_flag = ws.reserve(2 * sizeof(int64_t) + sizeof(int32_t));
+  h->scratch.reserve(ws.used);
+  ws.use_external(h->scratch.p, h->scratch.bytes);
+  D.woff = ws.at<int64_t>(o_woff);
+  D.cnt = ws.at<int32_t>(o_cnt);
+  D.off = ws.at<int64_t>(o_off);
+  D.chunk = ws.at<int32_t>(o_chunk);
+  D.piece = ws.at<AccPiece>(o_piece);
+  D.bound = ws.at<int64_t>(o_bound);
+  D.piece_cnt = ws.at<int32_t>(o_pcnt);
+  long long* part = ws.at<long long>(o_part);
+  int64_t* total = ws.at<int64_t>(o_flag);  // nnz(C), and beside it the two flags: the host reads them together
+  D.bad = reinterpret_cast<int32_t*>(total + 1);
+  D.npieces = D.bad + 2;
+  const unsigned grow = div_up(m + 1, 256);
+  hipLaunchKernelGGL((k_acc_weight<T, RP>), dim3(grow), dim3(256), 0, s, D);
+  scan_counts(s, D.cnt, m, D.woff, part, nullptr);
+  hipLaunchKernelGGL((k_acc_chunks<T, RP>), dim3(grow), dim3(256), 0, s, D);
+  const int nlong = total_in > kAccTarget ? (int)std::min<int64_t>(max_pieces, (int64_t)h->num_cus * 8) : 0;
+  if (nlong > 0) hipLaunchKernelGGL((k_acc_split<T, RP>), dim3(nlong), dim3(256), 0, s, D);
+  const unsigned grid = (unsigned)(D.nchunks + nlong);
+  hipLaunchKernelGGL((k_acc_merge<false, T, RP>), dim3(grid), dim3(kAccThreads), 0, s, D, nlong, (int*)nullptr,
+                     (T*)nullptr);
+  BCLX_HIP(hipGetLastError());
+  scan_counts(s, D.cnt, m, D.off, part, total);
+  int64_t got[2] = {0, 0};
+  BCLX_HIP(hipMemcpyAsync(got, total, sizeof(got), hipMemcpyDeviceToHost, s));
+  BCLX_HIP(hipStreamSynchronize(s));
+  if (got[1] != 0) return false;
+  const int64_t nnz = got[0];
+  if (C->col_idx == nullptr) {
+    if (C->row_ptr) {
+      BCLX_REQUIRE(C->ptr_width == 8 || nnz <= INT32_MAX, BCLX_ERR_OVERFLOW, "nnz does not fit an int32 row_ptr");
+      write_rowptr(s, D.off, m, C->row_ptr, C->ptr_width);
+    }
+  } else {
+    BCLX_REQUIRE(C->row_ptr && C->vals, BCLX_ERR_INVALID, "C->row_ptr / C->vals are null");
+    BCLX_REQUIRE(C->dtype == tiles[0].dtype, BCLX_ERR_INVALID, "C dtype must match the tiles");
+    BCLX_REQUIRE(C->nnz >= nnz, BCLX_ERR_INVALID, "C arrays smaller than the sum's entries");
+    BCLX_REQUIRE(C->ptr_width == 8 || nnz <= INT32_MAX, BCLX_ERR_OVERFLOW,
+                 "nnz(C) = " + std::to_string(nnz) + " does not fit an int32 row_ptr; request ptr_width 8");
+    hipLaunchKernelGGL((k_acc_merge<true, T, RP>), dim3(grid), dim3(kAccThreads), 0, s, D, nlong, C->col_idx,
+                       static_cast<T*>(C->vals));
+    BCLX_HIP(hipGetLastError());
+    write_rowptr(s, D.off, m, C->row_ptr, C->ptr_width);
+  }
+  C->m = m;
+  C->n = n;
+  C->nnz = nnz;
+  BCLX_HIP(hipStreamSynchronize(s));  // C is complete, and the handle's scratch free, on return
+  return true;
+}
+
+template <typename T, typename RP>
+static void accumulate_impl(bclx_handle* h, int K, const bclx_csr* tiles, bclx_csr* C) {
+  BCLX_REQUIRE(K * tiles[0].n < INT32_MAX, BCLX_ERR_OVERFLOW, "K * n must fit int32 (stacked column index)");
+  if (!accumulate_merge<T, RP>(h, K, tiles, C)) accumulate_spgemm<T, RP>(h, K, tiles, C);
 }
 
 }  // namespace bclx
