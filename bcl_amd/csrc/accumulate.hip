@@ -522,8 +522,7 @@ static bool accumulate_merge(bclx_handle* h, int K, const bclx_csr* tiles, bclx_
                o_piece = ws.reserve(sizeof(AccPiece) * max_pieces), o_bound = ws.reserve(sizeof(int64_t) * max_pieces * K),
                o_pcnt = ws.reserve(sizeof(int32_t) * max_pieces), o_part = ws.reserve(sizeof(long long) * scan_partials(m)),
                o_flag = ws.reserve(2 * sizeof(int64_t) + sizeof(int32_t));
-  h->scratch.reserve(ws.used);
-  ws.use_external(h->scratch.p, h->scratch.bytes);
+  ScratchUse use(h, ws);
   D.woff = ws.at<int64_t>(o_woff);
   D.cnt = ws.at<int32_t>(o_cnt);
   D.off = ws.at<int64_t>(o_off);

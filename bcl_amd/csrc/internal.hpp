@@ -153,6 +153,23 @@ inline void set_device(bclx_handle* h) {
 
 inline unsigned div_up(int64_t a, int64_t b) { return (unsigned)((a + b - 1) / b); }
 
+// The handle's scratch for a call that waits for its stream before it returns: grown on demand, and given back at the
+// end of a call that grew it beyond kScratchKeep (so one large call does not hold its memory until bclx_destroy).
+constexpr size_t kScratchKeep = size_t(1) << 30;
+struct ScratchUse {
+  bclx_handle* h;
+  size_t before;
+  ScratchUse(bclx_handle* h_, Arena& ws) : h(h_), before(h_->scratch.bytes) {
+    h->scratch.reserve(ws.used);
+    ws.use_external(h->scratch.p, h->scratch.bytes);
+  }
+  ~ScratchUse() {
+    if (h->scratch.bytes <= kScratchKeep || h->scratch.bytes <= before) return;
+    (void)hipStreamSynchronize(h->stream);
+    h->scratch.release();
+  }
+};
+
 // Looks up, once per device and with that device current, the address of the fixed scratch array that
 // bclx_spgemm_noalloc works in.
 void init_noalloc_scratch(int device);

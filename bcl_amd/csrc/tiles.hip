@@ -7,12 +7,15 @@
 // entries in their order in A. With 288 GB of HBM a whole matrix fits next to its tiles, so the cut is two passes over
 // A on the GPU instead of one host slice per tile:
 //   1. count: one thread per (row, tile column) finds where the tile column's segment of the row starts (binary
-//      search; A's columns are sorted within each row) and writes the segment length;
-//   2. one scan per tile column over all rows turns the lengths into offsets; a tile's row_ptr is that scan
-//      restricted to its rows, minus the value at its first row;
-//   3. copy: one wavefront per row; each lane takes entries of the row, finds its tile column from the segment
-//      starts staged in LDS, and writes the entry to its tile at (row offset + position in the segment).
-// Bytes: A's row_ptr and col_idx are read twice (count, copy) and its values once; every tile is written once.
+//      search; A's columns are sorted within each row) and writes that start and the segment length;
+//   2. one scan over the lengths of all tile columns, one column after the other, turns them into offsets; a tile's
+//      row_ptr is that scan restricted to its rows, minus the value at its first row;
+//   3. copy: work is split by entries (kSplitChunk per workgroup), so hub rows and short rows cost the same; a lane
+//      finds its entry's row in a window of row offsets in LDS, its tile column by a division, and writes the entry to
+//      its tile at (row offset + position in the segment).
+// Bytes: A's row_ptr and col_idx are read twice (count, copy) and its values once; every tile is written once. Measured
+// on R-MAT scale 20 (15.7 M entries, 4 x 4 tiles), sizes and copy together: 1.82 ms with one wavefront per row and
+// one scan per tile column, 0.51 ms this way.
 //
 // bclx_dense_binary_op is DMatrix's elementwise arithmetic on a tile (DMatrix::binary_op / binary_op_inplace,
 // bcl/containers/DMatrix.hpp:319-366, with operator+, -, *, / and += at :368-386): C = A op B per element, rows of
@@ -26,28 +29,43 @@
 
 namespace bclx {
 
-constexpr int kSplitMaxGridN = 256;  // tile columns of one split (LDS of the copy kernel)
+constexpr int kSplitMaxGridN = 256;            // tile columns of one split
+constexpr int kSplitChunk = 4096;              // entries of A per copying workgroup
 
-// cnt[tj * cstride + i] = entries of row i in tile column tj.
+// Row i's segment of tile column tj: seg[tj * stride + i] = its first position within the row, cnt[...] its length.
+// A block takes 256 / gn whole rows, so a segment's end is its neighbour's start. Also clears the counts that pad a
+// tile column to the stride.
 template <typename RP>
 __global__ __launch_bounds__(256) void k_split_count(const RP* rp, const int32_t* col, int64_t m, int64_t tile_n,
-                                                     int gn, int32_t* cnt, int64_t cstride) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= m * gn) return;
-  const int64_t i = t / gn;
-  const int tj = (int)(t - i * gn);
-  const int64_t a0 = (int64_t)rp[i], a1 = (int64_t)rp[i + 1];
-  // first position with col >= bound, for the tile column's two bounds
-  auto lower = [&](int64_t bound) {
-    int64_t lo = a0, hi = a1;
+                                                     int gn, int32_t* cnt, int32_t* seg, int64_t stride,
+                                                     int32_t* bad) {
+  __shared__ int s_lo[257];
+  const int rows = 256 / gn;
+  const int r = (int)threadIdx.x / gn, tj = (int)threadIdx.x - r * gn;
+  const int64_t i = (int64_t)blockIdx.x * rows + r;
+  const bool live = r < rows && i < m;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *bad = 0;
+  int len = 0;
+  if (live) {
+    const int64_t a0 = (int64_t)rp[i], a1 = (int64_t)rp[i + 1];
+    len = (int)(a1 - a0);
+    int lo = 0, hi = tj == 0 ? 0 : len;  // first position with column >= tj * tile_n
+    const int64_t bound = (int64_t)tj * tile_n;
     while (lo < hi) {
-      const int64_t mid = (lo + hi) >> 1;
-      if ((int64_t)col[mid] < bound) lo = mid + 1;
+      const int mid = lo + (hi - lo) / 2;
+      if ((int64_t)col[a0 + mid] < bound) lo = mid + 1;
       else hi = mid;
     }
-    return lo;
-  };
-  cnt[(int64_t)tj * cstride + i] = (int32_t)(lower((int64_t)(tj + 1) * tile_n) - lower((int64_t)tj * tile_n));
+    s_lo[threadIdx.x] = lo;
+  }
+  __syncthreads();
+  if (live) {
+    const int lo = s_lo[threadIdx.x], end = tj + 1 < gn ? s_lo[threadIdx.x + 1] : len;
+    seg[(int64_t)tj * stride + i] = lo;
+    cnt[(int64_t)tj * stride + i] = end > lo ? end - lo : 0;  // shorter than 0 only when the row is not sorted
+    if (i == m - 1)
+      for (int64_t q = m; q < stride; q++) cnt[(int64_t)tj * stride + q] = 0;
+  }
 }
 
 struct SplitTile {
@@ -58,69 +76,112 @@ struct SplitTile {
   int32_t ptr_width;
 };
 
-// One wavefront per row of A: row_ptr entries of its tiles, then its entries copied to their tiles. An entry that
-// would land outside its tile (columns of A not sorted within the row, or not below n) is not written and sets *bad.
-template <typename RP, typename T>
-__global__ __launch_bounds__(256) void k_split_copy(const RP* rp, const int32_t* col, const T* val, int64_t m,
-                                                    int64_t n, int64_t tile_m, int64_t tile_n, int gn,
-                                                    const int64_t* off, int64_t ostride, const SplitTile* tiles,
-                                                    int32_t* bad) {
-  __shared__ int64_t s_seg[4][kSplitMaxGridN + 1];
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int64_t i = (int64_t)blockIdx.x * 4 + w;
-  const bool live = i < m;
-  const int64_t a0 = live ? (int64_t)rp[i] : 0, a1 = live ? (int64_t)rp[i + 1] : 0;
-  const int64_t ti = live ? i / tile_m : 0, li = i - ti * tile_m;
-  const int64_t first = ti * tile_m;
-  const int64_t rows = (m - first) < tile_m ? (m - first) : tile_m;
-  // segment starts of the row's tile columns (positions in A), and the tiles' row_ptr entries of this row
-  for (int tj = lane; live && tj <= gn; tj += 64) {
-    int64_t lo = a0, hi = a1;
-    const int64_t bound = (int64_t)tj * tile_n;
-    while (lo < hi) {
-      const int64_t mid = (lo + hi) >> 1;
-      if ((int64_t)col[mid] < bound) lo = mid + 1;
-      else hi = mid;
-    }
-    s_seg[w][tj] = tj == gn ? a1 : lo;
-    if (tj < gn) {
-      const int64_t* o = off + (int64_t)tj * ostride;
-      const SplitTile& t = tiles[ti * gn + tj];
-      const int64_t base = o[first];
-      const int64_t v = o[i] - base;
-      if (t.ptr_width == 8) static_cast<int64_t*>(t.rp)[li] = v;
-      else static_cast<int32_t*>(t.rp)[li] = (int32_t)v;
-      if (li == rows - 1) {  // the row that closes its tile row also writes the tile's last row_ptr entry
-        const int64_t e = o[first + rows] - base;
-        if (t.ptr_width == 8) static_cast<int64_t*>(t.rp)[rows] = e;
-        else static_cast<int32_t*>(t.rp)[rows] = (int32_t)e;
-      }
-    }
+// i / d, in 32 bits where the rows fit them
+__device__ inline int64_t row_div(int64_t i, int64_t d, int64_t m) {
+  return m <= (int64_t)UINT32_MAX && d <= (int64_t)UINT32_MAX ? (int64_t)((uint32_t)i / (uint32_t)d) : i / d;
+}
+
+// The tiles' row_ptrs from the scanned offsets: one thread per (tile column, row). The threads of tile column 0 also
+// list, for each chunk of kSplitChunk entries of A, the row holding its first entry.
+template <typename RP>
+__global__ __launch_bounds__(256) void k_split_rowptr(const RP* rp, const int64_t* off, int64_t stride, int64_t m,
+                                                      int64_t tile_m, int gn, const SplitTile* tiles,
+                                                      int64_t* chunk_row) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int tj = blockIdx.y;
+  if (i >= m) return;
+  if (tj == 0) {
+    const int64_t a0 = (int64_t)rp[i], a1 = (int64_t)rp[i + 1];
+    for (int64_t c = (a0 + kSplitChunk - 1) / kSplitChunk; c * kSplitChunk < a1; c++) chunk_row[c] = i;
   }
-  __syncthreads();
-  for (int64_t p = a0 + lane; p < a1; p += 64) {
-    const int64_t c = col[p];
-    const int64_t tj = c / tile_n;
-    if (c < 0 || c >= n || tj >= gn) {
-      *bad = 1;
-      continue;
-    }
-    const SplitTile& t = tiles[ti * gn + tj];
-    const int64_t* o = off + tj * ostride;
-    const int64_t dst = (o[i] - o[first]) + (p - s_seg[w][tj]);
-    if (p < s_seg[w][tj] || p >= s_seg[w][tj + 1] || dst < 0 || dst >= t.nnz) {
-      *bad = 1;
-      continue;
-    }
-    t.col[dst] = (int32_t)(c - tj * tile_n);
-    static_cast<T*>(t.val)[dst] = val[p];
+  const int64_t ti = row_div(i, tile_m, m), first = ti * tile_m, li = i - first;
+  const int64_t rows = (m - first) < tile_m ? (m - first) : tile_m;
+  const int64_t* o = off + (int64_t)tj * stride;
+  const SplitTile t = tiles[ti * gn + tj];
+  const int64_t base = o[first], v = o[i] - base;
+  if (t.ptr_width == 8) static_cast<int64_t*>(t.rp)[li] = v;
+  else static_cast<int32_t*>(t.rp)[li] = (int32_t)v;
+  if (li == rows - 1) {  // the row that closes its tile row also writes the tile's last row_ptr entry
+    const int64_t e = o[first + rows] - base;
+    if (t.ptr_width == 8) static_cast<int64_t*>(t.rp)[rows] = e;
+    else static_cast<int32_t*>(t.rp)[rows] = (int32_t)e;
   }
 }
 
-// tot[ti * gn + tj] = entries of tile (ti, tj).
-__global__ void k_split_totals(const int64_t* off, int64_t ostride, int64_t m, int64_t tile_m, int gm, int gn,
-                               int64_t* tot) {
+// Copies A's entries [blockIdx * kSplitChunk, ...) to their tiles, walking windows of 256 row offsets from the chunk's
+// first row; unit-stride loads, four entries in flight per thread. An entry that would land outside its tile (columns
+// of A not sorted within the row, or not below n) is not written and sets *bad.
+template <typename RP, typename T>
+__global__ __launch_bounds__(256) void k_split_copy(const RP* rp, const int32_t* col, const T* val, int64_t m,
+                                                    int64_t n, int64_t tile_m, uint32_t tile_n, int gn,
+                                                    const int64_t* off, const int32_t* seg, int64_t stride,
+                                                    const SplitTile* tiles, const int64_t* chunk_row, int64_t total,
+                                                    int32_t* bad) {
+  __shared__ int64_t s_rp[257];
+  const int tid = threadIdx.x;
+  const int64_t c0 = (int64_t)blockIdx.x * kSplitChunk;
+  if (c0 >= total) return;
+  const int64_t c1 = c0 + kSplitChunk < total ? c0 + kSplitChunk : total;
+  int64_t r0 = chunk_row[blockIdx.x];
+  int64_t e = c0;
+  while (e < c1 && r0 < m) {
+    const int64_t r = r0 + tid;
+    s_rp[tid] = (int64_t)rp[r < m ? r : m];
+    if (tid == 0) s_rp[256] = (int64_t)rp[r0 + 256 < m ? r0 + 256 : m];
+    __syncthreads();
+    const int64_t we = s_rp[256] < c1 ? s_rp[256] : c1;
+    for (int64_t x0 = e; x0 < we; x0 += 4 * 256) {
+      int a[4];  // largest a with s_rp[a] <= x: four branchless searches in lockstep
+#pragma unroll
+      for (int q = 0; q < 4; q++) a[q] = 0;
+#pragma unroll
+      for (int step = 128; step > 0; step >>= 1) {
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+          if (s_rp[a[q] + step] <= x0 + q * 256 + tid) a[q] += step;
+      }
+      int c[4];
+      T v[4];
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const int64_t x = x0 + q * 256 + tid;
+        c[q] = x < we ? __builtin_nontemporal_load(&col[x]) : 0;
+        v[q] = x < we ? __builtin_nontemporal_load(&val[x]) : T(0);
+      }
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const int64_t x = x0 + q * 256 + tid;
+        if (x >= we) continue;
+        const uint32_t tj = (uint32_t)c[q] / tile_n;
+        if (c[q] < 0 || (int64_t)c[q] >= n || tj >= (uint32_t)gn) {
+          *bad = 1;
+          continue;
+        }
+        const int64_t i = r0 + a[q], ti = row_div(i, tile_m, m);
+        const int64_t* o = off + (int64_t)tj * stride;
+        const int64_t at = x - s_rp[a[q]] - seg[(int64_t)tj * stride + i];  // position within the segment
+        const int64_t oi = o[i], dst = oi - o[ti * tile_m] + at;
+        const SplitTile& t = tiles[ti * gn + tj];
+        if (at < 0 || oi + at >= o[i + 1] || dst < 0 || dst >= t.nnz) {
+          *bad = 1;
+          continue;
+        }
+        t.col[dst] = (int32_t)((uint32_t)c[q] - tj * tile_n);
+        static_cast<T*>(t.val)[dst] = v[q];
+      }
+    }
+    e = we > e ? we : e;
+    r0 += 256;
+    __syncthreads();
+  }
+}
+
+// tot[ti * gn + tj] = entries of tile (ti, tj); tot[gm * gn] = entries of A.
+template <typename RP>
+__global__ void k_split_totals(const RP* rp, const int64_t* off, int64_t ostride, int64_t m, int64_t tile_m, int gm,
+                               int gn, int64_t* tot) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t == gm * gn) tot[t] = (int64_t)rp[m];
   if (t >= gm * gn) return;
   const int ti = t / gn, tj = t - ti * gn;
   const int64_t r0 = (int64_t)ti * tile_m, r1 = (r0 + tile_m) < m ? (r0 + tile_m) : m;
@@ -132,28 +193,34 @@ template <typename RP, typename T>
 void split_grid(bclx_handle* h, const bclx_csr* A, int64_t tile_m, int64_t tile_n, int gm, int gn, bclx_csr* tiles) {
   hipStream_t s = h->stream;
   const int64_t m = A->m;
-  const int64_t cstride = (m + 3) / 4 * 4;      // 16-byte aligned count rows
-  const int64_t ostride = (m + 1 + 3) / 4 * 4;  // 16-byte aligned offset rows
-  DevBuf cnt(sizeof(int32_t) * (size_t)(cstride * gn));
-  DevBuf off(sizeof(int64_t) * (size_t)(ostride * gn));
-  DevBuf partial(sizeof(long long) * (size_t)scan_partials(m));
-  DevBuf tot(sizeof(int64_t) * (size_t)(gm * gn));
+  const int64_t stride = m / 4 * 4 + 4;  // a tile column's counts, padded with zeros: off[tj * stride + m] is its end
+  const int64_t L = stride * gn;
+  Arena ws;  // in the handle's scratch: this call waits for the stream before it returns
+  const size_t o_cnt = ws.reserve(sizeof(int32_t) * (size_t)L), o_seg = ws.reserve(sizeof(int32_t) * (size_t)L),
+               o_off = ws.reserve(sizeof(int64_t) * (size_t)(L + 4)),
+               o_part = ws.reserve(sizeof(long long) * (size_t)scan_partials(L)),
+               o_tot = ws.reserve(sizeof(int64_t) * (size_t)(gm * gn + 1)),
+               o_chunk = ws.reserve(sizeof(int64_t) * (size_t)(A->nnz / kSplitChunk + 1)),
+               o_tile = ws.reserve(sizeof(SplitTile) * (size_t)(gm * gn)), o_bad = ws.reserve(sizeof(int32_t));
+  ScratchUse use(h, ws);
+  int32_t* cnt = ws.at<int32_t>(o_cnt);
+  int32_t* seg = ws.at<int32_t>(o_seg);
+  int64_t* off = ws.at<int64_t>(o_off);
+  int64_t* tot = ws.at<int64_t>(o_tot);
+  int32_t* bad = ws.at<int32_t>(o_bad);
   const RP* rp = static_cast<const RP*>(A->row_ptr);
+  std::vector<int64_t> nnz((size_t)gm * gn + 1);
   if (m > 0) {
-    const int64_t nt = m * gn;
-    hipLaunchKernelGGL((k_split_count<RP>), dim3(div_up(nt, 256)), dim3(256), 0, s, rp, A->col_idx, m, tile_n, gn,
-                       cnt.as<int32_t>(), cstride);
+    hipLaunchKernelGGL((k_split_count<RP>), dim3(div_up(m, 256 / gn)), dim3(256), 0, s, rp, A->col_idx, m, tile_n, gn,
+                       cnt, seg, stride, bad);
     BCLX_HIP(hipGetLastError());
+    scan_counts(s, cnt, L, off, ws.at<long long>(o_part), nullptr);
+    hipLaunchKernelGGL((k_split_totals<RP>), dim3(div_up((int64_t)gm * gn + 1, 256)), dim3(256), 0, s, rp, off, stride, m,
+                       tile_m, gm, gn, tot);
+    BCLX_HIP(hipGetLastError());
+    BCLX_HIP(hipMemcpyAsync(nnz.data(), tot, sizeof(int64_t) * nnz.size(), hipMemcpyDeviceToHost, s));
+    BCLX_HIP(hipStreamSynchronize(s));
   }
-  for (int tj = 0; tj < gn; tj++)
-    scan_counts(s, cnt.as<int32_t>() + (int64_t)tj * cstride, m, off.as<int64_t>() + (int64_t)tj * ostride,
-                partial.as<long long>(), nullptr);
-  hipLaunchKernelGGL(k_split_totals, dim3(div_up((int64_t)gm * gn, 256)), dim3(256), 0, s, off.as<int64_t>(), ostride,
-                     m, tile_m, gm, gn, tot.as<int64_t>());
-  BCLX_HIP(hipGetLastError());
-  std::vector<int64_t> nnz((size_t)gm * gn);
-  BCLX_HIP(hipMemcpyAsync(nnz.data(), tot.p, sizeof(int64_t) * nnz.size(), hipMemcpyDeviceToHost, s));
-  BCLX_HIP(hipStreamSynchronize(s));
   bool sizes_only = true;
   for (int t = 0; t < gm * gn; t++) sizes_only = sizes_only && tiles[t].row_ptr == nullptr;
   for (int t = 0; t < gm * gn; t++) {
@@ -180,21 +247,31 @@ void split_grid(bclx_handle* h, const bclx_csr* A, int64_t tile_m, int64_t tile_
   std::vector<SplitTile> st((size_t)gm * gn);
   for (int t = 0; t < gm * gn; t++)
     st[t] = SplitTile{tiles[t].row_ptr, tiles[t].col_idx, tiles[t].vals, nnz[t], tiles[t].ptr_width};
-  DevBuf dt(sizeof(SplitTile) * st.size() + sizeof(int32_t));
-  int32_t* bad = reinterpret_cast<int32_t*>(dt.as<char>() + sizeof(SplitTile) * st.size());
-  BCLX_HIP(hipMemcpyAsync(dt.p, st.data(), sizeof(SplitTile) * st.size(), hipMemcpyHostToDevice, s));
-  BCLX_HIP(hipMemsetAsync(bad, 0, sizeof(int32_t), s));
+  int32_t h_bad = 0;
+  const int64_t entries = nnz.back();
+  DevBuf more_chunks;
   if (m > 0) {
-    hipLaunchKernelGGL((k_split_copy<RP, T>), dim3(div_up(m, 4)), dim3(256), 0, s, rp, A->col_idx,
-                       static_cast<const T*>(A->vals), m, A->n, tile_m, tile_n, gn, off.as<int64_t>(), ostride,
-                       dt.as<SplitTile>(), bad);
+    int64_t* chunk_row = ws.at<int64_t>(o_chunk);
+    if (entries > A->nnz) {  // the descriptor's nnz is not what row_ptr says
+      more_chunks.alloc(sizeof(int64_t) * (size_t)(entries / kSplitChunk + 1));
+      chunk_row = more_chunks.as<int64_t>();
+    }
+    SplitTile* dt = ws.at<SplitTile>(o_tile);
+    BCLX_HIP(hipMemcpyAsync(dt, st.data(), sizeof(SplitTile) * st.size(), hipMemcpyHostToDevice, s));
+    hipLaunchKernelGGL((k_split_rowptr<RP>), dim3(div_up(m, 256), (unsigned)gn), dim3(256), 0, s, rp, off, stride, m,
+                       tile_m, gn, dt, chunk_row);
     BCLX_HIP(hipGetLastError());
+    if (entries > 0) {
+      hipLaunchKernelGGL((k_split_copy<RP, T>), dim3(div_up(entries, kSplitChunk)), dim3(256), 0, s, rp, A->col_idx,
+                         static_cast<const T*>(A->vals), m, A->n, tile_m, (uint32_t)std::min<int64_t>(tile_n, UINT32_MAX),
+                         gn, off, seg, stride, dt, chunk_row, entries, bad);
+      BCLX_HIP(hipGetLastError());
+    }
+    BCLX_HIP(hipMemcpyAsync(&h_bad, bad, sizeof(int32_t), hipMemcpyDeviceToHost, s));
   } else {  // one row of tiles with no rows: each row_ptr is {0}
     for (int t = 0; t < gm * gn; t++) BCLX_HIP(hipMemsetAsync(tiles[t].row_ptr, 0, (size_t)tiles[t].ptr_width, s));
   }
-  int32_t h_bad = 0;
-  BCLX_HIP(hipMemcpyAsync(&h_bad, bad, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-  BCLX_HIP(hipStreamSynchronize(s));  // the scratch buffers are released on return
+  BCLX_HIP(hipStreamSynchronize(s));  // the tiles are complete, and the handle's scratch free, on return
   BCLX_REQUIRE(h_bad == 0, BCLX_ERR_INVALID, "A's columns must be sorted within each row and below A->n");
 }
 
