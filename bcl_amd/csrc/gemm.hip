@@ -8,13 +8,19 @@
 //   2  split-BF16 3-term: x = x_hi + x_lo with x_hi = bf16(x), x_lo = bf16(x - x_hi); a*b is taken as
 //      a_lo*b_hi + a_hi*b_lo + a_hi*b_hi (the a_lo*b_lo term, below 2^-16 relative, is dropped), fp32 accumulation
 //
-// Pipeline: a pack pass writes op(A) as Ap[M'][K'] and op(B) as Bp[N'][K'] (K contiguous, zero-padded to the block
-// tile, converted / split for the bf16 modes), then the MFMA kernel runs on the packed operands with no bounds checks
-// in its main loop. Block tile 128 x 128, four wavefronts of 64 x 64 (2 x 2 MFMA tiles of 32 x 32), the next K tile
-// is loaded into registers while the current one is multiplied out of LDS. Blocks are ordered so that each XCD
+// Two pipelines (gemm_impl chooses by predicted time):
+//   packed, for large fp32-operand products: a pack pass writes op(A) as Ap[M'][K'] and op(B) as Bp[N'][K'] (K
+//     contiguous, zero-padded to the block tile, converted / split for the bf16 modes), then the MFMA kernel runs on
+//     the packed operands with no bounds checks in its main loop. Block tile 128 x 128, four wavefronts of 64 x 64 (2 x
+//     2 MFMA tiles of 32 x 32);
+//   direct, for the others and for fp64: one kernel reads the caller's arrays, 64 x 64 tiles, K split over blocks
+//     where the tiles alone leave CUs idle.
+// In both the next K tile is loaded into registers while the current one is multiplied out of LDS, and blocks are
+// ordered so that each XCD
 // (blocks are dealt round-robin over the 8 XCDs) works on a compact patch of C tiles and shares their A and B panels
 // in its L2.
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "internal.hpp"
@@ -33,6 +39,9 @@ __device__ inline void static_for(F&& f) {
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+typedef double f64x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kGThreads = 256;
 
@@ -278,115 +287,285 @@ __global__ __launch_bounds__(kGThreads, TM * TN > 4 ? 2 : 1) void k_gemm(const t
     }
 }
 
-// ---- FP64 GEMM on the matrix cores (cblas_gemm_wrapper_'s double overload -> cblas_dgemm,
-// bcl/containers/algorithms/cblas_wrapper.hpp:29-40) ------------------------------------------------------------
-// Packed operands as above (op(A) as [M'][K'], op(B) as [N'][K'], K contiguous, zero-padded), block tile 128 x 128
-// of four wavefronts (2 x 2), each owning 4 x 4 tiles of 16 x 16 computed by v_mfma_f64_16x16x4f64 (fp64 products
-// and sums). K tiles of 16 doubles are staged through LDS; the next one is loaded into registers meanwhile.
+// ---- direct kernels: operands read from the caller's arrays ----------------------------------------------------
+// Sizes at which a pack pass (two more launches, each operand read and written once more) costs more than it saves,
+// and every fp32 and fp64 product: the block reads its A and B tiles straight from the caller's row-major arrays into
+// registers (bounds-checked at the edges, the next K tile while the current one is multiplied), converts / splits them
+// for the bf16 modes and stores them to LDS with K contiguous. A thread moves micro-tiles of 4 x 4 (fp32) or 2 x 2
+// (fp64) elements: one 16-byte load per source line of the micro-tile, along K or along the rows, whichever the source
+// has contiguous, and one K-contiguous LDS store per row. Loads need only the element's own alignment.
+// K is split over gridDim.z where the C tiles alone leave CUs idle: each split writes its partial sums to a workspace
+// and k_gemm_reduce adds them in order.
 
-__global__ __launch_bounds__(256) void k_pack_f64(const double* __restrict__ src, int64_t R, int64_t K, int64_t rs,
-                                                  int64_t cs, double* dst, int64_t Rp, int64_t Kp) {
-  __shared__ double tile[32][33];
-  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-  const int64_t r0 = (int64_t)blockIdx.y * 32, c0 = (int64_t)blockIdx.x * 32;
-  const bool rows_contig = cs != 1;
-  for (int q = ty; q < 32; q += 8) {
-    int64_t r, c;
-    if (rows_contig) { r = r0 + tx; c = c0 + q; }
-    else { r = r0 + q; c = c0 + tx; }
-    const double v = (r < R && c < K) ? src[r * rs + c * cs] : 0.0;
-    if (rows_contig) tile[tx][q] = v;
-    else tile[q][tx] = v;
+// Micro-tiles of one operand's block tile, and their way to LDS. Operand element (r, k), r < R, k < K, at
+// src[r * ld + k] (KC: contiguous along K) or src[k * ld + r].
+template <typename T, int Q, int ROWS, int BK, bool KC>
+struct MicroTiles {
+  static constexpr int COUNT = ROWS * BK / (Q * Q) / kGThreads;  // per thread
+  static constexpr int KQ = BK / Q;                              // micro-tiles along K
+  static_assert(ROWS * BK % (Q * Q * kGThreads) == 0, "whole micro-tiles per thread");
+  typedef T line_t __attribute__((ext_vector_type(Q)));
+  typedef T line_u __attribute__((ext_vector_type(Q), aligned(sizeof(T))));  // element-aligned in memory
+  line_t x[COUNT][Q];  // [micro-tile][source line]
+  int row[COUNT];      // first row of each micro-tile within the block tile
+  bool inside;         // every micro-tile lies inside the operand's rows
+
+  // Neighbouring lanes run along the contiguous direction (all of a K row of the tile, or 8 micro-tiles of rows). A
+  // micro-tile that would reach past the operand's last row is moved back to end there: it stores the rows it shares
+  // with its neighbour a second time (the same values), and the block's rows past the end stay unset (their products
+  // are not stored). Fewer than Q rows left in the whole block: the guarded path.
+  __device__ inline void init(int64_t r0, int64_t R) {
+    const int last = (int)(R - r0 < ROWS ? R - r0 - Q : ROWS - Q);
+    inside = last >= 0;
+    static_for<0, COUNT>([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      const int q = (int)threadIdx.x + i * kGThreads;
+      const int r = KC ? q / KQ * Q : (q % 8 + q / (8 * KQ) * 8) * Q;
+      row[i] = inside && r > last ? last : r;
+    });
+  }
+  static __device__ inline int k_of(int i) {
+    const int q = (int)threadIdx.x + i * kGThreads;
+    return (KC ? q % KQ : q / 8 % KQ) * Q;
+  }
+  // rows r0.. and K positions k0.. of the operand; k_whole: the K tile lies wholly inside it
+  __device__ inline void load(const T* src, int64_t ld, int64_t r0, int64_t k0, int64_t R, int64_t K, bool k_whole) {
+    const bool whole = inside && k_whole;
+    static_for<0, COUNT>([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      const int64_t line0 = KC ? r0 + row[i] : k0 + k_of(i), elem0 = KC ? k0 + k_of(i) : r0 + row[i];
+      const T* p = src + line0 * ld + elem0;
+      if (whole) {
+        static_for<0, Q>([&](auto jc) {
+          constexpr int j = decltype(jc)::value;
+          x[i][j] = *reinterpret_cast<const line_u*>(p + j * ld);
+        });
+      } else {
+        const int64_t nl = (KC ? R : K) - line0, ne = (KC ? K : R) - elem0;
+        static_for<0, Q>([&](auto jc) {
+          constexpr int j = decltype(jc)::value;
+          static_for<0, Q>([&](auto ec) {
+            constexpr int e = decltype(ec)::value;
+            x[i][j][e] = (j < nl && e < ne) ? p[j * ld + e] : T(0);
+          });
+        });
+      }
+    });
+  }
+  // f(row, k, values of k .. k + Q - 1) for each row of each micro-tile
+  template <typename F>
+  __device__ inline void rows(F&& f) const {
+    static_for<0, COUNT>([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      static_for<0, Q>([&](auto jc) {
+        constexpr int j = decltype(jc)::value;
+        line_t v;
+        static_for<0, Q>([&](auto ec) {
+          constexpr int e = decltype(ec)::value;
+          v[e] = x[i][KC ? j : e][KC ? e : j];
+        });
+        f(row[i] + j, k_of(i), v);
+      });
+    });
+  }
+};
+
+// C tile of this block, its K tiles, and where its result goes.
+struct DirectArgs {
+  int64_t M, N, K, lda, ldb, ldc;
+  int32_t tiles_m, tiles_n;
+  int32_t kt_per_split;      // K tiles per split
+  int64_t split_stride;      // elements between the splits' copies of C
+};
+
+constexpr int kDirectTile = 64;   // C tile of a block: 64 x 64, four wavefronts (2 x 2) of 32 x 32 each
+constexpr int kDirectBK = 64;     // K per LDS tile (fp32 operands)
+constexpr int kDirectBK64 = 16;   // K per LDS tile (fp64)
+
+template <int MODE, bool AKC, bool BKC>
+__global__ __launch_bounds__(kGThreads, 2) void k_gemm_direct(DirectArgs D, const float* __restrict__ A,
+                                                              const float* __restrict__ B, float alpha, float beta,
+                                                              float* C) {
+  using E = typename GemmCfg<MODE>::E;
+  constexpr int BK = kDirectBK, LDK = BK + GemmCfg<MODE>::PAD;
+  constexpr int BM = kDirectTile, BN = kDirectTile;
+  constexpr int NSPLIT = MODE == 2 ? 2 : 1;
+  __shared__ __align__(16) E As[NSPLIT][BM * LDK];
+  __shared__ __align__(16) E Bs[NSPLIT][BN * LDK];
+  int tm, tn;
+  gemm_tile_of<true>(blockIdx.x, D.tiles_m, D.tiles_n, tm, tn);
+  const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wm = wave >> 1, wn = wave & 1;
+  const int nk = (int)((D.K + BK - 1) / BK);
+  const int kt0 = (int)blockIdx.z * D.kt_per_split;
+  const int kt1 = min(nk, kt0 + D.kt_per_split);
+  C += (int64_t)blockIdx.z * D.split_stride;
+  MicroTiles<float, 4, BM, BK, AKC> ma;
+  MicroTiles<float, 4, BN, BK, BKC> mb;
+  ma.init(m0, D.M);
+  mb.init(n0, D.N);
+  auto gload = [&](int kt) {
+    const int64_t k0 = (int64_t)kt * BK;
+    const bool k_whole = k0 + BK <= D.K;
+    ma.load(A, D.lda, m0, k0, D.M, D.K, k_whole);
+    mb.load(B, D.ldb, n0, k0, D.N, D.K, k_whole);
+  };
+  auto put = [&](E* hi, E* lo, int r, int k, f32x4 v) {
+    if constexpr (MODE == 0) {
+      *reinterpret_cast<f32x4*>(hi + r * LDK + k) = v;
+    } else {
+      typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+      uint32_t h[4], l[4];
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        h[e] = f32_to_bf16_rne(v[e]);
+        if constexpr (MODE == 2) l[e] = f32_to_bf16_rne(v[e] - bf16_bits_to_f32((uint16_t)h[e]));
+      }
+      *reinterpret_cast<u32x2*>(hi + r * LDK + k) = u32x2{h[0] | h[1] << 16, h[2] | h[3] << 16};
+      if constexpr (MODE == 2) *reinterpret_cast<u32x2*>(lo + r * LDK + k) = u32x2{l[0] | l[1] << 16, l[2] | l[3] << 16};
+    }
+  };
+  auto lstore = [&]() {
+    ma.rows([&](int r, int k, f32x4 v) { put(As[0], As[NSPLIT - 1], r, k, v); });
+    mb.rows([&](int r, int k, f32x4 v) { put(Bs[0], Bs[NSPLIT - 1], r, k, v); });
+  };
+
+  f32x16 acc;
+#pragma unroll
+  for (int v = 0; v < 16; v++) acc[v] = 0.f;
+
+  const int fr = lane & 31, fk = lane >> 5;
+  const int oa = (wm * 32 + fr) * LDK, ob = (wn * 32 + fr) * LDK;
+  if (kt0 < kt1) {
+    gload(kt0);
+    lstore();
   }
   __syncthreads();
-  for (int q = ty; q < 32; q += 8) {
-    const int64_t r = r0 + q, c = c0 + tx;
-    if (r < Rp && c < Kp) dst[r * Kp + c] = tile[q][tx];
+  for (int kt = kt0; kt < kt1; kt++) {
+    if (kt + 1 < kt1) gload(kt + 1);
+    if constexpr (MODE == 0) {
+      // a lane's fragments of four K steps are one 16-byte read: half fk takes k = ks + 4 fk + q at step q
+#pragma unroll
+      for (int ks = 0; ks < BK; ks += 8) {
+        const f32x4 af = *reinterpret_cast<const f32x4*>(&As[0][oa + ks + 4 * fk]);
+        const f32x4 bf = *reinterpret_cast<const f32x4*>(&Bs[0][ob + ks + 4 * fk]);
+#pragma unroll
+        for (int q = 0; q < 4; q++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(af[q], bf[q], acc, 0, 0, 0);
+      }
+    } else {
+#pragma unroll
+      for (int ks = 0; ks < BK; ks += 16) {
+        const bf16x8 ah = *reinterpret_cast<const bf16x8*>(&As[0][oa + ks + fk * 8]);
+        const bf16x8 bh = *reinterpret_cast<const bf16x8*>(&Bs[0][ob + ks + fk * 8]);
+        if constexpr (MODE == 2) {
+          const bf16x8 al = *reinterpret_cast<const bf16x8*>(&As[NSPLIT - 1][oa + ks + fk * 8]);
+          const bf16x8 bl = *reinterpret_cast<const bf16x8*>(&Bs[NSPLIT - 1][ob + ks + fk * 8]);
+          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, bh, acc, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bl, acc, 0, 0, 0);
+        }
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bh, acc, 0, 0, 0);
+      }
+    }
+    __syncthreads();
+    if (kt + 1 < kt1) {
+      lstore();
+      __syncthreads();
+    }
+  }
+  // accumulator layout of a 32 x 32 MFMA tile: lane l holds column l % 32, rows 8 * (v / 4) + 4 * (l / 32) + v % 4
+  const int64_t col = n0 + wn * 32 + fr;
+  if (col >= D.N) return;
+#pragma unroll
+  for (int v = 0; v < 16; v++) {
+    const int64_t row = m0 + wm * 32 + 8 * (v / 4) + 4 * fk + (v % 4);
+    if (row < D.M) {
+      float* p = C + row * D.ldc + col;
+      *p = beta == 0.f ? alpha * acc[v] : fmaf(beta, *p, alpha * acc[v]);
+    }
   }
 }
 
-typedef double f64x4 __attribute__((ext_vector_type(4)));
-typedef double f64x2 __attribute__((ext_vector_type(2)));
-constexpr int kG64BK = 16;                // K per LDS tile
-constexpr int kG64LDK = kG64BK + 2;       // padded row (bank spread)
-constexpr int kG64T = 4;                  // 16 x 16 MFMA tiles per wavefront side
-constexpr int kG64BM = 2 * 16 * kG64T;    // 128
-
-__global__ __launch_bounds__(kGThreads) void k_gemm_f64(const double* __restrict__ Ap, const double* __restrict__ Bp,
-                                                        int64_t M, int64_t N, int64_t Kp, double alpha, double beta,
-                                                        double* C, int64_t ldc, int tiles_m, int tiles_n) {
-  __shared__ __align__(16) double As[kG64BM * kG64LDK];
-  __shared__ __align__(16) double Bs[kG64BM * kG64LDK];
-  int tm, tn;  // row-major: the fp64 product is bound by its matrix-core rate, and the grouped order measured 4% slower
-  gemm_tile_of<false>(blockIdx.x, tiles_m, tiles_n, tm, tn);
-  const int64_t m0 = (int64_t)tm * kG64BM, n0 = (int64_t)tn * kG64BM;
+// fp64 (cblas_gemm_wrapper_'s double overload -> cblas_dgemm, bcl/containers/algorithms/cblas_wrapper.hpp:29-40):
+// each wavefront owns 2 x 2 tiles of 16 x 16 computed by v_mfma_f64_16x16x4f64 (fp64 products and sums). Blocks of
+// 128 x 128 (two per CU at most) were slower at every size from 64 to 4096 (4096^3: 2.47 ms against 2.27).
+template <bool AKC, bool BKC>
+__global__ __launch_bounds__(kGThreads, 3) void k_gemm_f64_direct(DirectArgs D, const double* __restrict__ A,
+                                                               const double* __restrict__ B, double alpha, double beta,
+                                                               double* C) {
+  constexpr int TT = 2, BK = kDirectBK64, LDK = BK + 2, BM = kDirectTile;
+  __shared__ __align__(16) double As[BM * LDK];
+  __shared__ __align__(16) double Bs[BM * LDK];
+  int tm, tn;
+  gemm_tile_of<true>(blockIdx.x, D.tiles_m, D.tiles_n, tm, tn);
+  const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BM;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
-  constexpr int VPR = kG64BK / 2;                 // 16-byte vectors per tile row
-  constexpr int VPT = kG64BM * VPR / kGThreads;   // per thread, per operand
-  const double* __restrict__ Ag = Ap + m0 * Kp;
-  const double* __restrict__ Bg = Bp + n0 * Kp;
-  f64x2 ra[VPT], rb[VPT];
-  auto gload = [&](int64_t k0) {
-    static_for<0, VPT>([&](auto ic) {
-      constexpr int i = decltype(ic)::value;
-      const int v = tid + i * kGThreads;
-      const int64_t o = (int64_t)(v / VPR) * Kp + k0 + (v % VPR) * 2;
-      ra[i] = *reinterpret_cast<const f64x2*>(Ag + o);
-      rb[i] = *reinterpret_cast<const f64x2*>(Bg + o);
-    });
+  const int nk = (int)((D.K + BK - 1) / BK);
+  const int kt0 = (int)blockIdx.z * D.kt_per_split;
+  const int kt1 = min(nk, kt0 + D.kt_per_split);
+  C += (int64_t)blockIdx.z * D.split_stride;
+  MicroTiles<double, 2, BM, BK, AKC> ma;
+  MicroTiles<double, 2, BM, BK, BKC> mb;
+  ma.init(m0, D.M);
+  mb.init(n0, D.N);
+  auto gload = [&](int kt) {
+    const int64_t k0 = (int64_t)kt * BK;
+    const bool k_whole = k0 + BK <= D.K;
+    ma.load(A, D.lda, m0, k0, D.M, D.K, k_whole);
+    mb.load(B, D.ldb, n0, k0, D.N, D.K, k_whole);
   };
   auto lstore = [&]() {
-    static_for<0, VPT>([&](auto ic) {
-      constexpr int i = decltype(ic)::value;
-      const int v = tid + i * kGThreads;
-      const int o = (v / VPR) * kG64LDK + (v % VPR) * 2;
-      *reinterpret_cast<f64x2*>(&As[o]) = ra[i];
-      *reinterpret_cast<f64x2*>(&Bs[o]) = rb[i];
-    });
+    ma.rows([&](int r, int k, f64x2 v) { *reinterpret_cast<f64x2*>(&As[r * LDK + k]) = v; });
+    mb.rows([&](int r, int k, f64x2 v) { *reinterpret_cast<f64x2*>(&Bs[r * LDK + k]) = v; });
   };
-  f64x4 acc[kG64T][kG64T];
+  f64x4 acc[TT][TT];
 #pragma unroll
-  for (int a = 0; a < kG64T; a++)
+  for (int a = 0; a < TT; a++)
 #pragma unroll
-    for (int c = 0; c < kG64T; c++) acc[a][c] = f64x4{0.0, 0.0, 0.0, 0.0};
-  const int nk = (int)(Kp / kG64BK);
-  gload(0);
-  lstore();
-  __syncthreads();
+    for (int c = 0; c < TT; c++) acc[a][c] = f64x4{0.0, 0.0, 0.0, 0.0};
   const int fr = lane & 15, fk = lane >> 4;  // operand lane layout: row (or column) fr, k offset fk
-  for (int kt = 0; kt < nk; kt++) {
-    if (kt + 1 < nk) gload((int64_t)(kt + 1) * kG64BK);
+  if (kt0 < kt1) {
+    gload(kt0);
+    lstore();
+  }
+  __syncthreads();
+  for (int kt = kt0; kt < kt1; kt++) {
+    if (kt + 1 < kt1) gload(kt + 1);
+    // a lane's fragments of two K steps are one 16-byte read: lane group fk takes k = ks + 2 fk + q at step q
 #pragma unroll
-    for (int ks = 0; ks < kG64BK; ks += 4) {
-      double af[kG64T], bf[kG64T];
+    for (int ks = 0; ks < BK; ks += 8) {
+      f64x2 af[TT], bf[TT];
 #pragma unroll
-      for (int t = 0; t < kG64T; t++) {
-        af[t] = As[(wm * 16 * kG64T + t * 16 + fr) * kG64LDK + ks + fk];
-        bf[t] = Bs[(wn * 16 * kG64T + t * 16 + fr) * kG64LDK + ks + fk];
+      for (int t = 0; t < TT; t++) {
+        af[t] = *reinterpret_cast<const f64x2*>(&As[(wm * 16 * TT + t * 16 + fr) * LDK + ks + 2 * fk]);
+        bf[t] = *reinterpret_cast<const f64x2*>(&Bs[(wn * 16 * TT + t * 16 + fr) * LDK + ks + 2 * fk]);
       }
 #pragma unroll
-      for (int a = 0; a < kG64T; a++)
+      for (int q = 0; q < 2; q++)
 #pragma unroll
-        for (int c = 0; c < kG64T; c++) acc[a][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[a], bf[c], acc[a][c], 0, 0, 0);
+        for (int a = 0; a < TT; a++)
+#pragma unroll
+          for (int c = 0; c < TT; c++)
+            acc[a][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[a][q], bf[c][q], acc[a][c], 0, 0, 0);
     }
     __syncthreads();
-    if (kt + 1 < nk) {
+    if (kt + 1 < kt1) {
       lstore();
       __syncthreads();
     }
   }
   // accumulator layout of a 16 x 16 fp64 tile: lane l holds column l % 16, rows l / 16 + 4 * v
-  static_for<0, kG64T>([&](auto ac) {
+  static_for<0, TT>([&](auto ac) {
     constexpr int a = decltype(ac)::value;
-    static_for<0, kG64T>([&](auto cc) {
+    static_for<0, TT>([&](auto cc) {
       constexpr int c = decltype(cc)::value;
-      const int64_t col = n0 + wn * 16 * kG64T + c * 16 + fr;
+      const int64_t col = n0 + wn * 16 * TT + c * 16 + fr;
       static_for<0, 4>([&](auto vc) {
         constexpr int v = decltype(vc)::value;
-        const int64_t row = m0 + wm * 16 * kG64T + a * 16 + fk + 4 * v;
-        if (row < M && col < N) {
-          double* p = C + row * ldc + col;
+        const int64_t row = m0 + wm * 16 * TT + a * 16 + fk + 4 * v;
+        if (row < D.M && col < D.N) {
+          double* p = C + row * D.ldc + col;
           *p = beta == 0.0 ? alpha * acc[a][c][v] : fma(beta, *p, alpha * acc[a][c][v]);
         }
       });
@@ -394,25 +573,93 @@ __global__ __launch_bounds__(kGThreads) void k_gemm_f64(const double* __restrict
   });
 }
 
-static void gemm_f64_run(bclx_handle* h, bool ta, bool tb, int64_t m, int64_t n, int64_t k, double alpha,
-                         const double* A, int64_t lda, const double* B, int64_t ldb, double beta, double* C,
-                         int64_t ldc) {
-  const int64_t Mp = (m + kG64BM - 1) / kG64BM * kG64BM, Np = (n + kG64BM - 1) / kG64BM * kG64BM;
-  const int64_t Kp = std::max<int64_t>(32, (k + 31) / 32 * 32);  // whole pack tiles and whole K tiles
-  const size_t a_bytes = (size_t)Mp * Kp * 8, off_b = (a_bytes + 255) / 256 * 256;
-  h->scratch.reserve(off_b + (size_t)Np * Kp * 8 + 256);
-  double* Ap = h->scratch.as<double>();
-  double* Bp = reinterpret_cast<double*>(h->scratch.as<char>() + off_b);
-  hipLaunchKernelGGL(k_pack_f64, dim3((unsigned)(Kp / 32), (unsigned)(Mp / 32)), dim3(256), 0, h->stream, A, m, k,
-                     ta ? (int64_t)1 : lda, ta ? lda : (int64_t)1, Ap, Mp, Kp);
+// C = beta * C + alpha * (sum of the splits' partial products, in order)
+template <typename T>
+__global__ __launch_bounds__(256) void k_gemm_reduce(const T* ws, int splits, int64_t M, int64_t N, T alpha, T beta,
+                                                     T* C, int64_t ldc) {
+  const int64_t total = M * N;
+  for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < total; t += (int64_t)gridDim.x * 256) {
+    T sum = ws[t];
+    for (int z = 1; z < splits; z++) sum += ws[(int64_t)z * total + t];
+    T* p = C + t / N * ldc + t % N;
+    *p = beta == T(0) ? alpha * sum : fma(beta, *p, alpha * sum);
+  }
+}
+
+template <typename T>
+static void reduce_splits(bclx_handle* h, const T* ws, int splits, int64_t M, int64_t N, T alpha, T beta, T* C,
+                          int64_t ldc) {
+  const unsigned g = (unsigned)std::min<int64_t>(div_up(M * N, 256), (int64_t)h->num_cus * 8);
+  hipLaunchKernelGGL((k_gemm_reduce<T>), dim3(g), dim3(256), 0, h->stream, ws, splits, M, N, alpha, beta, C, ldc);
   BCLX_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_pack_f64, dim3((unsigned)(Kp / 32), (unsigned)(Np / 32)), dim3(256), 0, h->stream, B, n, k,
-                     tb ? ldb : (int64_t)1, tb ? (int64_t)1 : ldb, Bp, Np, Kp);
-  BCLX_HIP(hipGetLastError());
-  const int tiles_m = (int)(Mp / kG64BM), tiles_n = (int)(Np / kG64BM);
-  hipLaunchKernelGGL(k_gemm_f64, dim3((unsigned)(tiles_m * tiles_n)), dim3(kGThreads), 0, h->stream, Ap, Bp, m, n, Kp,
-                     alpha, beta, C, ldc, tiles_m, tiles_n);
-  BCLX_HIP(hipGetLastError());
+}
+
+// Do the rows x cols elements of C (leading dimension ldc) share memory with an operand's?
+template <typename T>
+static bool overlaps(const T* C, int64_t rows, int64_t cols, int64_t ldc, const T* X, int64_t xrows, int64_t xcols,
+                     int64_t ldx) {
+  if (xrows <= 0 || xcols <= 0) return false;
+  const uintptr_t c0 = reinterpret_cast<uintptr_t>(C), c1 = c0 + sizeof(T) * (size_t)((rows - 1) * ldc + cols);
+  const uintptr_t x0 = reinterpret_cast<uintptr_t>(X), x1 = x0 + sizeof(T) * (size_t)((xrows - 1) * ldx + xcols);
+  return c0 < x1 && x0 < c1;
+}
+
+// K tiles of bk in about `splits` equal parts, one grid layer each; launch(D, grid, alpha, beta, C). `apart`: C may
+// share memory with an operand, so no block may write it while others read.
+template <typename T, typename LAUNCH>
+static void direct_run(bclx_handle* h, DirectArgs D, int bk, int splits, bool apart, T alpha, T beta, T* C,
+                       LAUNCH&& launch) {
+  D.tiles_m = (int)((D.M + kDirectTile - 1) / kDirectTile);
+  D.tiles_n = (int)((D.N + kDirectTile - 1) / kDirectTile);
+  const int64_t nk = (D.K + bk - 1) / bk;
+  D.kt_per_split = (int)std::max<int64_t>(1, (nk + splits - 1) / splits);
+  splits = (int)std::max<int64_t>(1, (nk + D.kt_per_split - 1) / D.kt_per_split);
+  const dim3 grid((unsigned)(D.tiles_m * D.tiles_n), 1, (unsigned)splits);
+  if (splits > 1 || apart) {  // partial products into the workspace, scaled and added to C afterwards
+    h->scratch.reserve(sizeof(T) * (size_t)splits * (size_t)(D.M * D.N));
+    T* ws = h->scratch.as<T>();
+    const int64_t ldc = D.ldc;
+    D.ldc = D.N;
+    D.split_stride = D.M * D.N;
+    launch(D, grid, T(1), T(0), ws);
+    BCLX_HIP(hipGetLastError());
+    reduce_splits<T>(h, ws, splits, D.M, D.N, alpha, beta, C, ldc);
+  } else {
+    launch(D, grid, alpha, beta, C);
+    BCLX_HIP(hipGetLastError());
+  }
+}
+
+// f(A contiguous along K, B contiguous along K) as compile-time constants
+template <typename F>
+static void with_layout(bool ta, bool tb, F&& f) {
+  if (!ta && !tb) f(std::true_type{}, std::false_type{});
+  else if (!ta) f(std::true_type{}, std::true_type{});
+  else if (!tb) f(std::false_type{}, std::false_type{});
+  else f(std::false_type{}, std::true_type{});
+}
+
+template <int MODE>
+static void gemm_direct(bclx_handle* h, const DirectArgs& D, bool ta, bool tb, int splits, float alpha, const float* A,
+                        const float* B, float beta, float* C) {
+  direct_run<float>(h, D, kDirectBK, splits, false, alpha, beta, C,
+                    [&](const DirectArgs& d, dim3 grid, float al, float be, float* out) {
+    with_layout(ta, tb, [&](auto ac, auto bc) {
+      hipLaunchKernelGGL((k_gemm_direct<MODE, decltype(ac)::value, decltype(bc)::value>), grid, dim3(kGThreads), 0,
+                         h->stream, d, A, B, al, be, out);
+    });
+  });
+}
+
+static void gemm_f64_direct(bclx_handle* h, const DirectArgs& D, bool ta, bool tb, int splits, bool apart, double alpha,
+                            const double* A, const double* B, double beta, double* C) {
+  direct_run<double>(h, D, kDirectBK64, splits, apart, alpha, beta, C,
+                     [&](const DirectArgs& d, dim3 grid, double al, double be, double* out) {
+    with_layout(ta, tb, [&](auto ac, auto bc) {
+      hipLaunchKernelGGL((k_gemm_f64_direct<decltype(ac)::value, decltype(bc)::value>), grid, dim3(kGThreads), 0,
+                         h->stream, d, A, B, al, be, out);
+    });
+  });
 }
 
 // FP64 reference: C += A * B (fp32 inputs widened exactly), 16 x 16 tiles, row-major. Error oracle only.
@@ -433,8 +680,7 @@ __global__ __launch_bounds__(256) void k_gemm_f64_ref(int64_t M, int64_t N, int6
   if (row < M && col < N) C[row * ldc + col] += s;
 }
 
-// Wavefront tile (TM x TN MFMA tiles) per mode: BF16 uses 4 x 2 (block 256 x 128) when M is large enough to fill the
-// GPU with such blocks; FP32 and split-BF16 (twice the LDS) keep 2 x 2 (block 128 x 128).
+// Pack both operands, then the packed kernel.
 template <int MODE, int TM, int TN>
 static void gemm_run(bclx_handle* h, bool ta, bool tb, int64_t m, int64_t n, int64_t k, float alpha, const float* A,
                      int64_t lda, const float* B, int64_t ldb, float beta, float* C, int64_t ldc) {
@@ -466,12 +712,80 @@ static void gemm_run(bclx_handle* h, bool ta, bool tb, int64_t m, int64_t n, int
   BCLX_HIP(hipGetLastError());
 }
 
+// Predicted microseconds of a kernel: `packed` (with its two pack passes) or direct, C tiles of bm x bn, `per` and
+// `per_block` = a K tile of 64 on one CU: fixed and for each block that shares the CU. The constants are fitted to
+// square, ragged, flat and deep products from 64 to 8192 (within about 15%): what decides is how many blocks a CU
+// gets, what a K tile costs a block alone (its load latency) and what the pack passes or the K splits' sum cost.
+struct GemmCost {
+  bool packed;
+  int bm, bn;
+  double per, per_block;
+};
+struct GemmPlan {
+  double us;
+  int splits;
+};
+// w: bytes of an element of C; pack_bytes: read and written per packed element
+static GemmPlan gemm_cost(const bclx_handle* h, const GemmCost& c, int64_t m, int64_t n, int64_t k, int w,
+                          int pack_bytes) {
+  const double nk = std::max<double>(1.0, std::ceil((double)k / 64));
+  const double tiles = std::ceil((double)m / c.bm) * std::ceil((double)n / c.bn);
+  GemmPlan best{0, 0};
+  for (int s = 1; s <= 64 && (s == 1 || (!c.packed && 2 * s <= nk)); s *= 2) {
+    const double load = tiles * s / h->num_cus;
+    // the fullest CU decides; the packed bf16 kernels wait more for memory, which the emptier CUs leave to them
+    const double blocks = c.packed ? 0.5 * (std::ceil(load) + std::max(1.0, load)) : std::ceil(load);
+    double us = 3 + std::ceil(nk / s) * (c.per + c.per_block * blocks);
+    if (s > 1) us += 3 + (2 * s + 2) * (double)m * (double)n * w / 5e6;
+    if (c.packed) us += 6 + (double)(m + n) * (double)k * pack_bytes / 4e6;
+    if (best.splits == 0 || us < 0.95 * best.us) best = {us, s};
+  }
+  return best;
+}
+
+// Direct kernels where they are predicted faster, and smaller packed tiles where 128 x 128 leave CUs idle. The
+// 128 x 128 (bf16: 256 x 128) packed kernel is the one for large products; the others have to beat it by 10%.
+// Measured, us, packed 128 x 128 against the choice made here: fp32 2000 x 1500 x 3001 255 -> 174 (direct), 489 x 93 x
+// 3552 268 -> 16 (direct, K split), 4096^3 1108 (packed; direct 1200); bf16 1500^3 46 -> 39 (packed 64 x 64), 512^3
+// 24 -> 11 (direct); split-bf16 947 x 1486 x 2519 102 -> 61 (packed 64 x 64).
 template <int MODE>
 static void gemm_impl(bclx_handle* h, bool ta, bool tb, int64_t m, int64_t n, int64_t k, float alpha, const float* A,
                       int64_t lda, const float* B, int64_t ldb, float beta, float* C, int64_t ldc) {
-  const bool big = MODE == 1 && ((m + 255) / 256) * ((n + 127) / 128) >= 2 * (int64_t)h->num_cus;
-  if (big) gemm_run<MODE, 4, 2>(h, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
-  else gemm_run<MODE, 2, 2>(h, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
+  constexpr int pack_bytes = MODE == 1 ? 6 : 8;
+  constexpr GemmCost large{true, 128, 128, MODE == 0 ? 0.6 : MODE == 1 ? 0.55 : 0.35,
+                           MODE == 0 ? 3.9 : MODE == 1 ? 0.56 : 1.45};
+  constexpr GemmCost small{true, 64, 64, MODE == 1 ? 0.3 : 0.1, MODE == 1 ? 0.225 : 0.46};
+  constexpr GemmCost direct{false, 64, 64, MODE == 0 ? 0.4 : MODE == 1 ? 0.85 : 1.45,
+                            MODE == 0 ? 1.1 : MODE == 1 ? 0.5 : 0.95};
+  const DirectArgs D{m, n, k, lda, ldb, ldc, 0, 0, 0, 0};
+  const double us_large = gemm_cost(h, large, m, n, k, 4, pack_bytes).us;
+  GemmPlan d = gemm_cost(h, direct, m, n, k, 4, pack_bytes);
+  // the packed kernels read only their copies of A and B, so C may share memory with them
+  if (overlaps(C, m, n, ldc, A, ta ? k : m, ta ? m : k, lda) || overlaps(C, m, n, ldc, B, tb ? n : k, tb ? k : n, ldb))
+    d.us = HUGE_VAL;
+  if constexpr (MODE == 0) {
+    if (d.us < 0.98 * us_large) gemm_direct<0>(h, D, ta, tb, d.splits, alpha, A, B, beta, C);
+    else gemm_run<0, 2, 2>(h, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
+  } else {
+    const bool big = MODE == 1 && ((m + 255) / 256) * ((n + 127) / 128) >= 2 * (int64_t)h->num_cus;
+    const double us_small = gemm_cost(h, small, m, n, k, 4, pack_bytes).us;
+    if (big) gemm_run<1, 4, 2>(h, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
+    else if (d.us < 0.9 * us_large && d.us < us_small) gemm_direct<MODE>(h, D, ta, tb, d.splits, alpha, A, B, beta, C);
+    else if (us_small < 0.9 * us_large) gemm_run<MODE, 1, 1>(h, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
+    else gemm_run<MODE, 2, 2>(h, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
+  }
+}
+
+// fp64, us, against packed operands and 128 x 128 blocks: 512^3 103 -> 17, 1234 x 2048 x 1777 355 -> 181, 4096^3 2940 ->
+// 2175 (63 TFLOP/s of the 72.6 that the vendor library reaches at 8192^3).
+static void gemm_f64_run(bclx_handle* h, bool ta, bool tb, int64_t m, int64_t n, int64_t k, double alpha,
+                         const double* A, int64_t lda, const double* B, int64_t ldb, double beta, double* C,
+                         int64_t ldc) {
+  constexpr GemmCost direct{false, 64, 64, 1.56, 1.72};
+  const GemmPlan d = gemm_cost(h, direct, m, n, k, 8, 0);
+  const bool apart = overlaps(C, m, n, ldc, A, ta ? k : m, ta ? m : k, lda) ||
+                     overlaps(C, m, n, ldc, B, tb ? n : k, tb ? k : n, ldb);
+  gemm_f64_direct(h, DirectArgs{m, n, k, lda, ldb, ldc, 0, 0, 0, 0}, ta, tb, d.splits, apart, alpha, A, B, beta, C);
 }
 
 }  // namespace bclx
