@@ -52,6 +52,7 @@ bclx_status bclx_create(int device, void* stream, bclx_handle** out) {
     h->num_cus = cus > 0 ? cus : 256;
     h->lds_per_block = lds > 0 ? (size_t)lds : 65536;
     init_noalloc_scratch(device);
+    BCLX_HIP(hipHostMalloc(reinterpret_cast<void**>(&h->h_pinned), sizeof(int64_t) * kPinnedCounts, hipHostMallocDefault));
     *out = h.release();
   });
 }
@@ -77,6 +78,7 @@ bclx_status bclx_set_allocator(bclx_handle* h, bclx_alloc_fn alloc, bclx_free_fn
 bclx_status bclx_set_stream(bclx_handle* h, void* stream) {
   return guarded([&] {
     BCLX_REQUIRE(h != nullptr, BCLX_ERR_INVALID, "null handle");
+    if (h->stream != static_cast<hipStream_t>(stream)) h->stream_changes++;
     h->stream = static_cast<hipStream_t>(stream);
   });
 }

@@ -122,11 +122,20 @@ struct bclx_handle {
   bclx::DevBuf dense_slots;  // heavy-row dense accumulators, kept zeroed between uses
   size_t dense_slot_doubles = 0;
   int dense_nslots = 0;
-  bclx::DevBuf pinned_dummy;
-  int64_t* h_pinned = nullptr;  // small pinned host buffer for counts
+  int64_t* h_pinned = nullptr;  // kPinnedCounts values in pinned host memory, written by k_report
+  // workspace of the last spgemm plan, kept for the next one (at most kPlanKeep bytes; hipMalloc'd handles only)
+  bclx::DevBuf plan_ws;
+  bool plan_ws_busy = false;
+  unsigned stream_changes = 0;  // bclx_set_stream calls that changed the stream
+  ~bclx_handle() {
+    if (h_pinned) (void)hipHostFree(h_pinned);
+  }
 };
 
 namespace bclx {
+
+constexpr size_t kPlanKeep = size_t(4) << 30;
+constexpr int kPinnedCounts = 64;
 
 // Wraps a C-ABI body: converts exceptions to status codes and records the message.
 template <typename F>

@@ -53,22 +53,7 @@ void ensure_dense_slots(bclx_handle* h, int nslots, size_t ndoubles) {
 // ---------------------------------------------------------------------------------------------------------------
 
 template <typename T, typename RP>
-void FlatRows<T, RP>::setup(bclx_handle* h_, const std::vector<TileDev<T, RP>>& tiles_in, bool with_cap) {
-  h = h_;
-  tiles = tiles_in;
-  ntiles = (int)tiles.size();
-  nflat = 0;
-  max_n = 1;
-  std::vector<uint16_t> blk;
-  for (int t = 0; t < ntiles; t++) {
-    tiles[t].flat0 = nflat;
-    int64_t pm = ((int64_t)tiles[t].m + kRowBlock - 1) / kRowBlock * kRowBlock;
-    if (pm == 0) pm = kRowBlock;  // every product owns at least one block
-    for (int64_t b = 0; b < pm / kRowBlock; b++) blk.push_back((uint16_t)t);
-    nflat += pm;
-    max_n = std::max<int64_t>(max_n, tiles[t].n);
-  }
-  BCLX_REQUIRE(ntiles <= 65535, BCLX_ERR_INVALID, "at most 65535 products per batch");
+void FlatRows<T, RP>::layout(bool with_cap, bool pooled, bool* from_pool) {
   BCLX_REQUIRE(nflat < INT32_MAX, BCLX_ERR_OVERFLOW, "too many rows in one batch (flat rows must fit int32)");
   nblocks = nflat / kRowBlock;
   Arena& A = arena;
@@ -90,6 +75,12 @@ void FlatRows<T, RP>::setup(bclx_handle* h_, const std::vector<TileDev<T, RP>>& 
   size_t nsb = (size_t)((nflat + kScanTile - 1) / kScanTile) + 1;
   size_t o_part = A.reserve(sizeof(long long) * nsb);
   size_t o_tot = A.reserve(sizeof(int64_t) * 2);
+  if (pooled && !A.ext && !h->alloc.alloc && !h->plan_ws_busy && A.used <= kPlanKeep) {
+    h->plan_ws.reserve(A.used);
+    A.use_external(h->plan_ws.p, h->plan_ws.bytes);
+    h->plan_ws_busy = true;
+    *from_pool = true;
+  }
   A.commit();
   R.tiles = A.at<TileDev<T, RP>>(o_tiles);
   R.blk_tile = A.at<uint16_t>(o_blk);
@@ -111,6 +102,46 @@ void FlatRows<T, RP>::setup(bclx_handle* h_, const std::vector<TileDev<T, RP>>& 
   R.stats = A.at<unsigned long long>(o_stats);
   scan_partial = A.at<long long>(o_part);
   scan_total = A.at<int64_t>(o_tot);
+}
+
+template <typename T, typename RP>
+bool FlatRows<T, RP>::setup_one(bclx_handle* h_, const TileDev<T, RP>& tile, bool pooled) {
+  h = h_;
+  tiles.assign(1, tile);
+  tiles[0].flat0 = 0;
+  ntiles = 1;
+  nflat = std::max<int64_t>(1, ((int64_t)tile.m + kRowBlock - 1) / kRowBlock) * kRowBlock;
+  max_n = std::max<int64_t>(1, tile.n);
+  bool from_pool = false;
+  layout(false, pooled, &from_pool);
+  return from_pool;
+}
+
+template <typename T, typename RP>
+void FlatRows<T, RP>::prepare_one(hipStream_t s) {
+  const unsigned grid = (unsigned)std::max<int64_t>(3, std::min<int64_t>(div_up(nblocks, 256), h->num_cus));
+  hipLaunchKernelGGL((k_prepare_one<T, RP>), dim3(grid), dim3(256), 0, s, tiles[0], R, nblocks);
+  BCLX_HIP(hipGetLastError());
+}
+
+template <typename T, typename RP>
+void FlatRows<T, RP>::setup(bclx_handle* h_, const std::vector<TileDev<T, RP>>& tiles_in, bool with_cap) {
+  h = h_;
+  tiles = tiles_in;
+  ntiles = (int)tiles.size();
+  nflat = 0;
+  max_n = 1;
+  std::vector<uint16_t> blk;
+  for (int t = 0; t < ntiles; t++) {
+    tiles[t].flat0 = nflat;
+    int64_t pm = ((int64_t)tiles[t].m + kRowBlock - 1) / kRowBlock * kRowBlock;
+    if (pm == 0) pm = kRowBlock;  // every product owns at least one block
+    for (int64_t b = 0; b < pm / kRowBlock; b++) blk.push_back((uint16_t)t);
+    nflat += pm;
+    max_n = std::max<int64_t>(max_n, tiles[t].n);
+  }
+  BCLX_REQUIRE(ntiles <= 65535, BCLX_ERR_INVALID, "at most 65535 products per batch");
+  layout(with_cap, false, nullptr);
   BCLX_HIP(hipMemcpyAsync(const_cast<TileDev<T, RP>*>(R.tiles), tiles.data(), sizeof(TileDev<T, RP>) * ntiles,
                           hipMemcpyHostToDevice, h->stream));
   BCLX_HIP(hipMemcpyAsync(const_cast<uint16_t*>(R.blk_tile), blk.data(), sizeof(uint16_t) * nblocks,
@@ -132,13 +163,18 @@ void FlatRows<T, RP>::reset_counters(hipStream_t s) {
 }
 
 template <typename T, typename RP>
-void FlatRows<T, RP>::analyze(hipStream_t s, bool do_bin, long long pred_min, bool with_stats) {
-  const unsigned grid = (unsigned)((nblocks + kAnaSub - 1) / kAnaSub);
-  fill_i32(s, R.long_count, 1, 0);
-  hipLaunchKernelGGL((k_analyze<T, RP>), dim3(grid), dim3(kRowBlock), 0, s, R, (int64_t)nblocks, do_bin ? 1 : 0,
-                     pred_min, with_stats ? 1 : 0);
+void FlatRows<T, RP>::analyze(hipStream_t s, bool do_bin, long long pred_min, bool with_stats, bool cleared) {
+  if (!cleared) fill_i32(s, R.long_count, 1, 0);
+  if (nblocks >= 2 * kAnaSubLarge * (int64_t)h->num_cus)
+    hipLaunchKernelGGL((k_analyze<kAnaSubLarge, T, RP>), dim3(div_up(nblocks, kAnaSubLarge)), dim3(kRowBlock), 0, s, R,
+                       (int64_t)nblocks, do_bin ? 1 : 0, pred_min, with_stats ? 1 : 0);
+  else
+    hipLaunchKernelGGL((k_analyze<1, T, RP>), dim3((unsigned)nblocks), dim3(kRowBlock), 0, s, R, (int64_t)nblocks,
+                       do_bin ? 1 : 0, pred_min, with_stats ? 1 : 0);
   BCLX_HIP(hipGetLastError());
-  hipLaunchKernelGGL((k_analyze_long<T, RP>), dim3((unsigned)h->num_cus * 8), dim3(kRowBlock), 0, s, R,
+  // at most one wavefront per row
+  const unsigned lg = (unsigned)std::min<int64_t>((int64_t)h->num_cus * 8, nflat / (kRowBlock / 64));
+  hipLaunchKernelGGL((k_analyze_long<T, RP>), dim3(lg), dim3(kRowBlock), 0, s, R,
                      do_bin ? 1 : 0, pred_min, with_stats ? 1 : 0);
   BCLX_HIP(hipGetLastError());
 }
@@ -152,6 +188,11 @@ void FlatRows<T, RP>::bin(hipStream_t s, int src) {
 
 template <typename T, typename RP>
 void FlatRows<T, RP>::scan(hipStream_t s, const int32_t* cnt, int64_t* off, int64_t off_add) {
+  if (nflat <= kScanOneMax) {
+    hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(kScanBlock), 0, s, cnt, nflat, off, off_add, scan_total);
+    BCLX_HIP(hipGetLastError());
+    return;
+  }
   const int64_t nb = (nflat + kScanTile - 1) / kScanTile;
   hipLaunchKernelGGL(k_scan_reduce, dim3((unsigned)nb), dim3(kScanBlock), 0, s, cnt, nflat, scan_partial);
   BCLX_HIP(hipGetLastError());
@@ -191,6 +232,11 @@ void scan_counts(hipStream_t s, const int32_t* cnt, int64_t n, int64_t* off, lon
   if (n == 0) {
     hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, s, reinterpret_cast<unsigned long long*>(off), (int64_t)1, 0ull);
     if (total) hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, s, reinterpret_cast<unsigned long long*>(total), (int64_t)1, 0ull);
+    BCLX_HIP(hipGetLastError());
+    return;
+  }
+  if (n <= kScanOneMax) {
+    hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(kScanBlock), 0, s, cnt, n, off, (int64_t)0, total);
     BCLX_HIP(hipGetLastError());
     return;
   }
@@ -236,8 +282,9 @@ void FlatRows<T, RP>::run_bin(hipStream_t s, int mode, int b, int64_t count_hint
   // rows of at most 32 products (bin 18) and of 33-64 (ESC bin 11): sorted in registers by groups of G lanes
   auto launch_small = [&](auto g_tag, auto n_tag) {
     constexpr int G = decltype(g_tag)::value, N = decltype(n_tag)::value;
-    unsigned grid = count_hint >= 0 ? (unsigned)std::max<int64_t>(1, div_up(count_hint, (64 / G) * kSmallWaves))
-                                    : (unsigned)(h->num_cus * 8);
+    constexpr int rows = (64 / G) * kSmallWaves;  // per block and step
+    unsigned grid = count_hint >= 0 ? (unsigned)std::max<int64_t>(1, div_up(count_hint, rows))
+                                    : (unsigned)std::min<int64_t>(div_up(nflat, rows), (int64_t)h->num_cus * 8);
     grid = std::min<unsigned>(grid, 1u << 20);
 #define BCLX_SMALL(M, ONE) \
   hipLaunchKernelGGL((k_esc_small<M, ONE, G, N, T, RP>), dim3(grid), dim3(64 * kSmallWaves), 0, s, R, b)
@@ -360,6 +407,16 @@ void FlatRows<T, RP>::read_counts(hipStream_t s, int32_t* dst) {
 }
 
 template <typename T, typename RP>
+int64_t FlatRows<T, RP>::report(hipStream_t s, int32_t* counts) {
+  static_assert(kNumBins + 1 <= kPinnedCounts && kNumBins < 64, "one value per lane");
+  hipLaunchKernelGGL((k_report<T, RP>), dim3(1), dim3(64), 0, s, R, (const int64_t*)scan_total, h->h_pinned);
+  BCLX_HIP(hipGetLastError());
+  BCLX_HIP(hipStreamSynchronize(s));
+  for (int b = 0; b < kNumBins; b++) counts[b] = (int32_t)h->h_pinned[b];
+  return h->h_pinned[kNumBins];
+}
+
+template <typename T, typename RP>
 int64_t FlatRows<T, RP>::read_stat(int q) {
   unsigned long long v = 0;
   BCLX_HIP(hipMemcpyAsync(&v, R.stats + q, sizeof(v), hipMemcpyDeviceToHost, h->stream));
@@ -451,18 +508,33 @@ template TileDev<double, int64_t> make_tile<double, int64_t>(const bclx_csr*, co
 template <typename T, typename RP>
 int64_t TwoPhase<T, RP>::symbolic() {
   hipStream_t s = h->stream;
-  F.reset_counters(s);
-  F.analyze(s, true);
+  F.prepare_one(s);
+  F.analyze(s, true, -1, true, true);
   int32_t* counts = sym_counts;
-  F.read_counts(s, counts);
+  // Where the average row has few products, most rows are in the two register-sorted bins: they and the scan are
+  // launched before the counts are known, and when no other bin holds rows the host waits once instead of twice.
+  const TileDev<T, RP>& t = F.tiles[0];
+  const bool small_rows = (double)t.avg_a * (double)t.avg_b <= 2 * kSmallMax;
+  if (small_rows) {
+    F.run_bin(s, 0, kSmallBin, -1);
+    F.run_bin(s, 0, kEscBin0, -1);
+    F.scan(s, F.R.nnz, F.R.off, 0);
+  }
+  int64_t tot = F.report(s, counts);
   if (counts[kHeavyBin] > 0) F.prepare_heavy();
   reuse_bins = true;  // the hash bins and the heavy bin are chosen by the row's size bound, which the count replaces
   for (int b = 1; b <= kHeavyBin; b++) reuse_bins = reuse_bins && counts[b] == 0;
-  for (int b = 1; b < kNumBins; b++) F.run_bin(s, 0, b, counts[b]);
-  F.scan(s, F.R.nnz, F.R.off, 0);
-  int64_t tot = 0;
-  BCLX_HIP(hipMemcpyAsync(&tot, F.scan_total, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-  BCLX_HIP(hipStreamSynchronize(s));
+  bool more = !small_rows;
+  for (int b = 1; b < kNumBins; b++) {
+    if (counts[b] == 0 || (small_rows && (b == kSmallBin || b == kEscBin0))) continue;
+    F.run_bin(s, 0, b, counts[b]);
+    more = true;
+  }
+  if (more) {
+    F.scan(s, F.R.nnz, F.R.off, 0);
+    int32_t again[kNumBins];
+    tot = F.report(s, again);
+  }
   nnz_c = tot;
   return tot;
 }
@@ -474,11 +546,16 @@ void TwoPhase<T, RP>::numeric(int* c_col, T* c_val, int64_t c_cap, void* row_ptr
   BCLX_REQUIRE(ptr_width == 8 || nnz_c <= INT32_MAX, BCLX_ERR_OVERFLOW,
                "nnz(C) = " + std::to_string(nnz_c) + " does not fit an int32 row_ptr; request ptr_width 8");
   hipStream_t s = h->stream;
-  if (F.tiles[0].c_col != c_col || F.tiles[0].c_val != c_val) {
-    F.tiles[0].c_col = c_col;
-    F.tiles[0].c_val = c_val;
-    F.upload_tiles();
-  }
+  F.tiles[0].c_col = c_col;
+  F.tiles[0].c_val = c_val;
+  const unsigned g = div_up(m + 1, 256);
+  if (ptr_width == 8)
+    hipLaunchKernelGGL((k_begin_numeric<int64_t, T, RP>), dim3(g), dim3(256), 0, s, F.R, m, static_cast<int64_t*>(row_ptr),
+                       c_col, c_val);
+  else
+    hipLaunchKernelGGL((k_begin_numeric<int32_t, T, RP>), dim3(g), dim3(256), 0, s, F.R, m, static_cast<int32_t*>(row_ptr),
+                       c_col, c_val);
+  BCLX_HIP(hipGetLastError());
   F.R.out_limit = c_cap;
   int32_t counts[kNumBins];
   if (reuse_bins) {
@@ -488,14 +565,6 @@ void TwoPhase<T, RP>::numeric(int* c_col, T* c_val, int64_t c_cap, void* row_ptr
     F.read_counts(s, counts);
   }
   for (int b = 1; b < kNumBins; b++) F.run_bin(s, 1, b, counts[b]);
-  const unsigned g = div_up(m + 1, 256);
-  if (ptr_width == 8)
-    hipLaunchKernelGGL(k_rowptr<int64_t>, dim3(g), dim3(256), 0, s, F.R.off, (int64_t)0, m,
-                       static_cast<int64_t*>(row_ptr));
-  else
-    hipLaunchKernelGGL(k_rowptr<int32_t>, dim3(g), dim3(256), 0, s, F.R.off, (int64_t)0, m,
-                       static_cast<int32_t*>(row_ptr));
-  BCLX_HIP(hipGetLastError());
 }
 
 template struct TwoPhase<float, int32_t>;
@@ -513,7 +582,7 @@ struct PlanBase {
 template <typename T, typename RP>
 struct TwoPhasePlan : PlanBase {
   TwoPhase<T, RP> tp;
-  TwoPhasePlan(bclx_handle* h, const bclx_csr* A, const bclx_csr* B) : tp(h, make_tile<T, RP>(A, B), BinTuning{}) {}
+  TwoPhasePlan(bclx_handle* h, const bclx_csr* A, const bclx_csr* B) : tp(h, make_tile<T, RP>(A, B), BinTuning{}, nullptr, 0, true) {}
   int64_t symbolic() override { return tp.symbolic(); }
   void numeric(bclx_csr* C) override {
     BCLX_REQUIRE(C && C->row_ptr, BCLX_ERR_INVALID, "C or C->row_ptr is null");

@@ -35,11 +35,16 @@ struct FlatRows {
   DevBuf gbits;  // per-workgroup column bitmaps of the wide-tile heavy kernel (kept zeroed between rows)
 
   void setup(bclx_handle* h, const std::vector<TileDev<T, RP>>& tiles, bool with_cap);
+  // the same for one product, without any GPU work: prepare_one() writes its tables. pooled: the workspace may be the
+  // handle's (then it is given back by the owner)
+  bool setup_one(bclx_handle* h, const TileDev<T, RP>& tile, bool pooled);
+  void prepare_one(hipStream_t s);
   void upload_tiles();
   void reset_counters(hipStream_t s);
   // pred_min >= 0 (learned path): also write cap = min(prod, n) and list the rows with more than pred_min products
   // with_stats: also count products (stats[0]) and rows bound for the heavy bin (stats[5])
-  void analyze(hipStream_t s, bool do_bin, long long pred_min = -1, bool with_stats = true);
+  // cleared: the counters (the long-row count among them) are zero already
+  void analyze(hipStream_t s, bool do_bin, long long pred_min = -1, bool with_stats = true, bool cleared = false);
   void bin(hipStream_t s, int src);
   // exclusive scan of cnt over all flat rows into off (nflat + 1 entries), plus off_add; total -> *scan_total
   void scan(hipStream_t s, const int32_t* cnt, int64_t* off, int64_t off_add);
@@ -52,6 +57,10 @@ struct FlatRows {
   bool heavy_lds_bitmap() const;  // wide-tile heavy kernel: bitmap in LDS (else per-workgroup global bitmaps)
   int64_t read_stat(int q);
   void read_counts(hipStream_t s, int32_t* dst);  // kNumBins bin counts (synchronises s)
+  int64_t report(hipStream_t s, int32_t* counts);  // the bin counts and the last scan's total (synchronises s)
+
+ private:
+  void layout(bool with_cap, bool pooled, bool* from_pool);
 };
 
 // The two-phase product C = A * B of one tile pair (symbolic, then numeric into caller-allocated C).
@@ -65,16 +74,29 @@ struct TwoPhase {
   // products alone)
   int32_t sym_counts[kNumBins] = {0};
   bool reuse_bins = false;
-  // scratch / scratch_bytes: device memory the workspace is laid out in instead of being allocated
+  bool from_pool = false;        // the workspace is the handle's
+  unsigned stream_changes = 0;   // of the handle, when the workspace was taken
+  // scratch / scratch_bytes: device memory the workspace is laid out in instead of being allocated. pooled: the handle's
+  // workspace may be taken (by one product at a time)
   TwoPhase(bclx_handle* h_, const TileDev<T, RP>& tile, const BinTuning& tn, void* scratch = nullptr,
-           size_t scratch_bytes = 0)
+           size_t scratch_bytes = 0, bool pooled = false)
       : h(h_) {
-    std::vector<TileDev<T, RP>> tiles{tile};
     if (scratch) F.arena.use_external(scratch, scratch_bytes);
-    F.setup(h, tiles, false);
+    from_pool = F.setup_one(h, tile, pooled);
+    stream_changes = h->stream_changes;
     F.R.tn = tn;
     m = tile.m;
   }
+  // The handle's workspace goes back once nothing uses it: the work of this product is on the handle's stream, or on an
+  // earlier one where bclx_set_stream was called in between.
+  ~TwoPhase() {
+    if (!from_pool) return;
+    if (stream_changes == h->stream_changes) (void)hipStreamSynchronize(h->stream);
+    else (void)hipDeviceSynchronize();
+    h->plan_ws_busy = false;
+  }
+  TwoPhase(const TwoPhase&) = delete;
+  TwoPhase& operator=(const TwoPhase&) = delete;
   int64_t symbolic();
   // writes col/val into c_col/c_val (capacity c_cap entries) and row_ptr (m+1 entries of 4 or 8 bytes)
   void numeric(int* c_col, T* c_val, int64_t c_cap, void* row_ptr, int ptr_width);

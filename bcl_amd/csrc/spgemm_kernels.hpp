@@ -187,9 +187,11 @@ __device__ inline V block_sum(V v, V* smem) {
 
 // 256-row blocks of flat rows per analysis workgroup: each thread analyzes one row of each, with the loads of its
 // rows issued together, and the workgroup takes its bin and list positions with one global atomic per bin.
-constexpr int kAnaSub = 4;
+// Four blocks where that still fills the GPU; one where it does not (16384 rows of 8 entries: 18 us with four, 8 us with
+// one).
+constexpr int kAnaSubLarge = 4;
 
-template <typename T, typename RP>
+template <int kAnaSub, typename T, typename RP>
 __global__ __launch_bounds__(kRowBlock) void k_analyze(RowsDev<T, RP> R, int64_t nblocks, int do_bin,
                                                        long long pred_min, int with_stats) {
   __shared__ int s_nlong, s_lbase;
@@ -2074,6 +2076,63 @@ __global__ __launch_bounds__(kRowBlock) void k_compact(RowsDev<T, RP> R, const i
     e = we;
     r0 += kRowBlock;
     __syncthreads();
+  }
+}
+
+// Scan of at most kScanOneMax counts by one workgroup: one launch instead of three (500 rows 2.7 us, 16384 rows 9.4 us;
+// the three took 6.7 and 8.3 us and two more gaps between launches).
+constexpr int64_t kScanOneMax = 8 * kScanTile;
+static __global__ __launch_bounds__(kScanBlock) void k_scan_one(const int32_t* cnt, int64_t n, int64_t* off,
+                                                                int64_t off_add, int64_t* total_out) {
+  __shared__ long long sm[kScanBlock / 64 + 1];
+  long long base = 0;
+  for (int64_t b = 0; b < n; b += kScanTile) {
+    const int64_t r0 = b + (int64_t)threadIdx.x * kScanPer;
+    long long v[kScanPer];
+    scan_load4(cnt, n, r0, v);
+    long long tot;
+    long long run = base + off_add + block_excl_scan<kScanBlock, long long>(v[0] + v[1] + v[2] + v[3], &tot, sm);
+#pragma unroll
+    for (int q = 0; q < kScanPer; q++) {
+      if (r0 + q < n) off[r0 + q] = run;
+      run += v[q];
+    }
+    base += tot;
+  }
+  if (threadIdx.x == 0) {
+    off[n] = base + off_add;
+    if (total_out) *total_out = base;
+  }
+}
+
+// One launch before a product's passes: its tile, the (single) product of every row block, all counters cleared.
+template <typename T, typename RP>
+__global__ __launch_bounds__(256) void k_prepare_one(TileDev<T, RP> tile, RowsDev<T, RP> R, int64_t nblocks) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x, step = (int64_t)gridDim.x * 256;
+  if (i == 0) *const_cast<TileDev<T, RP>*>(R.tiles) = tile;
+  for (int64_t b = i; b < nblocks; b += step) const_cast<uint16_t*>(R.blk_tile)[b] = 0;
+  for (int64_t b = i; b < kNumBins * kCountStride; b += step) R.bin_count[b] = 0;
+  if (i < 3) R.ovf_count[i] = 0;  // overflow, predicted and long rows
+  if (i < 8) R.stats[i] = 0;
+}
+
+// The bin counts and the last scan's total, written to pinned host memory (kNumBins + 1 values): the host waits for the
+// stream and reads them, with no copy in between.
+template <typename T, typename RP>
+__global__ void k_report(RowsDev<T, RP> R, const int64_t* total, int64_t* out) {
+  if (threadIdx.x < kNumBins) out[threadIdx.x] = *R.count_of(threadIdx.x);
+  if (threadIdx.x == kNumBins) out[kNumBins] = *total;
+}
+
+// One launch before the numeric pass: C's row_ptr, and the arrays its entries go to.
+template <typename OUT, typename T, typename RP>
+__global__ void k_begin_numeric(RowsDev<T, RP> R, int64_t m, OUT* rp, int* c_col, T* c_val) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i <= m) rp[i] = (OUT)(R.off[i] - R.off[0]);
+  if (i == 0) {
+    TileDev<T, RP>* t = const_cast<TileDev<T, RP>*>(R.tiles);
+    t->c_col = c_col;
+    t->c_val = c_val;
   }
 }
 

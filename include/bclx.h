@@ -87,7 +87,8 @@ BCLX_API bclx_status bclx_set_allocator(bclx_handle* h, bclx_alloc_fn alloc, bcl
  * symbolic: row analysis (products per row), binning and an exact per-row count of C's pattern; returns
  * nnz(C). numeric: fills caller-allocated C (row_ptr m+1 of C->ptr_width, col_idx/vals of nnz) with sorted
  * columns and values accumulated in float64 and rounded once to C->dtype. A and B must share dtype and
- * ptr_width. C->ptr_width 4 fails with BCLX_ERR_OVERFLOW when nnz(C) > 2^31 - 1. */
+ * ptr_width. C->ptr_width 4 fails with BCLX_ERR_OVERFLOW when nnz(C) > 2^31 - 1. The handle keeps the device workspace
+ * of the last plan (up to 4 GiB) for the next one until bclx_destroy, unless it has a caller's allocator. */
 BCLX_API bclx_status bclx_spgemm_symbolic(bclx_handle* h, const bclx_csr* A, const bclx_csr* B,
                                           bclx_spgemm_plan** plan, int64_t* nnz_c);
 BCLX_API bclx_status bclx_spgemm_numeric(bclx_spgemm_plan* plan, bclx_csr* C);
