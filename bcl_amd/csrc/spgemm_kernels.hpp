@@ -801,6 +801,13 @@ __device__ inline void esc_lookup(const int* pre, int ne, int base, int lane, in
   }
 }
 
+// A pointer read from device memory, as one to global memory: the compiler then emits global loads and stores. Flat ones also
+// count as LDS operations, so that each LDS wait waits for them.
+template <typename P>
+__device__ inline __attribute__((address_space(1))) P* glob(P* p) {
+  return (__attribute__((address_space(1))) P*)p;
+}
+
 // Compare-exchange of one bitonic stage whose partner is `d` lanes away (d < 64): keep min or max of the pair.
 // Value of lane (lane ^ D) of a wavefront. Distances 1, 2 and 8 are one DPP move (quad_perm [1,0,3,2], quad_perm
 // [2,3,0,1], row_ror:8), 4 is two DPP moves (row_shl:4 for lanes with bit 2 clear, row_shr:4 for the others), 16 is
@@ -1017,147 +1024,227 @@ __global__ __launch_bounds__(64 * kEscWaves) void k_esc(RowsDev<T, RP> R, int bi
 }
 
 // ------------------------------------------------------------------------------------------------------------
-// Rows of at most 32 products, half a wavefront each (two rows per wavefront). The products are expanded one per lane
-// as 32-bit keys (column << 5 | product index), sorted by a bitonic network over the 32 lanes (DPP and swizzle
-// exchanges: no LDS, no barrier), and equal columns are summed in product (A-row) order, in float64, rounded once.
+// Rows of at most 32 (64) products, 8 (16) lanes each. The products are expanded four per lane as 32-bit keys (column
+// << 5 (6) | product index), sorted in registers (DPP exchanges: no LDS, no barrier), and equal columns are summed in
+// product (A-row) order, in float64, rounded once.
 // A hash row of this size costs a table clear, LDS atomics and a sort of its table in LDS; a one-wavefront ESC row
 // leaves half the lanes idle. Tiles up to 2^27 - 2 columns wide. Modes as in k_esc.
 // ------------------------------------------------------------------------------------------------------------
 
 constexpr int kSmallWaves = 4;  // wavefronts per block
 
-// One bitonic stage (block size K, partner distance J) over the 32 elements of a row group: element x = s * G + gl
-// sits in slot s of lane gl. Partners J >= G lie in the same lane (another slot); closer ones in lane gl ^ J.
-template <int K, int J, int G, int S>
-__device__ inline void grp_cx(unsigned (&key)[S], int gl) {
-  if constexpr (J >= G) {
-    constexpr int D = J / G;
+// A value moved between the lanes of a 16-lane DPP row, one VALU move (part of the using instruction where that allows
+// it): from lane ^ X (X = 1, 2, 3, 7 or 15), or from the lane D below (above); lanes without one get 0.
+template <int X>
+__device__ inline unsigned dpp_xor(unsigned v) {
+  constexpr int ctrl = X == 1 ? 0xB1 : X == 2 ? 0x4E : X == 3 ? 0x1B : X == 7 ? 0x141 : 0x140;
+  static_assert(X == 1 || X == 2 || X == 3 || X == 7 || X == 15, "a quad permutation or a mirror");
+  return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, 0xF, 0xF, true);
+}
+template <int D>
+__device__ inline unsigned dpp_below(unsigned v) {
+  return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x110 + D, 0xF, 0xF, true);
+}
+template <int D>
+__device__ inline unsigned dpp_above(unsigned v) {
+  return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x100 + D, 0xF, 0xF, true);
+}
+
+// min(a, b) where lim is 0, max(a, b) where it is ~0 (the median of the three: one instruction)
+__device__ inline unsigned min_or_max(unsigned a, unsigned b, unsigned lim) {
+  return max(min(a, b), min(max(a, b), lim));
+}
+
+__device__ inline void cx(unsigned& a, unsigned& b) {
+  const unsigned lo = min(a, b);
+  b = max(a, b);
+  a = lo;
+}
+
+// Ascending sort of the 4 * G keys of each row group (G = 8 or 16 lanes): in, any order; out, element x of the sorted
+// sequence is slot x % 4 of lane x / 4. Bitonic, with every comparator ascending (each merge first meets the mirrored
+// position). Four neighbours per lane put 10 of the 15 stages of 32 keys (11 of 21 of 64) inside a lane at two instructions a
+// pair; the others take a DPP move and a median per key. 82 instructions instead of the 200 that positions
+// spread over the lanes (slot * G + lane: 3 stages inside a lane) took.
+template <int G>
+__device__ inline void grp_sort(unsigned (&key)[4], int gl) {
+  cx(key[0], key[1]);
+  cx(key[2], key[3]);
+  cx(key[0], key[2]);
+  cx(key[1], key[3]);
+  cx(key[1], key[2]);
+  const unsigned l1 = gl & 1 ? ~0u : 0u, l2 = gl & 2 ? ~0u : 0u, l4 = gl & 4 ? ~0u : 0u, l8 = gl & 8 ? ~0u : 0u;
+  auto mirror = [&](auto x, unsigned lim) {
+    constexpr int X = decltype(x)::value;
+    const unsigned o0 = dpp_xor<X>(key[3]), o1 = dpp_xor<X>(key[2]), o2 = dpp_xor<X>(key[1]), o3 = dpp_xor<X>(key[0]);
+    key[0] = min_or_max(key[0], o0, lim);
+    key[1] = min_or_max(key[1], o1, lim);
+    key[2] = min_or_max(key[2], o2, lim);
+    key[3] = min_or_max(key[3], o3, lim);
+  };
+  auto lanes = [&](auto x, unsigned lim) {
+    constexpr int X = decltype(x)::value;
 #pragma unroll
-    for (int s = 0; s < S; s++)
-      if ((s & D) == 0) {
-        const bool asc = ((s * G + gl) & K) == 0;
-        const unsigned a = key[s], b = key[s + D];
-        key[s] = asc ? min(a, b) : max(a, b);
-        key[s + D] = asc ? max(a, b) : min(a, b);
-      }
-  } else {
-#pragma unroll
-    for (int s = 0; s < S; s++) {
-      const unsigned other = lane_xor<J>(key[s], gl);
-      const int x = s * G + gl;
-      const bool lower = (x & J) == 0, asc = (x & K) == 0;
-      key[s] = lower == asc ? min(key[s], other) : max(key[s], other);
+    for (int q = 0; q < 4; q++) {
+      // lane ^ 4 is the mirror of eight, then of four
+      const unsigned o = X == 4 ? dpp_xor<3>(dpp_xor<7>(key[q])) : dpp_xor<X == 4 ? 1 : X>(key[q]);
+      key[q] = min_or_max(key[q], o, lim);
     }
+  };
+  auto inside = [&] {
+    cx(key[0], key[2]);
+    cx(key[1], key[3]);
+    cx(key[0], key[1]);
+    cx(key[2], key[3]);
+  };
+  constexpr std::integral_constant<int, 1> x1{};
+  constexpr std::integral_constant<int, 2> x2{};
+  mirror(x1, l1);
+  inside();
+  mirror(std::integral_constant<int, 3>{}, l2);
+  lanes(x1, l1);
+  inside();
+  mirror(std::integral_constant<int, 7>{}, l4);
+  lanes(x2, l2);
+  lanes(x1, l1);
+  inside();
+  if constexpr (G == 16) {
+    mirror(std::integral_constant<int, 15>{}, l8);
+    lanes(std::integral_constant<int, 4>{}, l4);
+    lanes(x2, l2);
+    lanes(x1, l1);
+    inside();
   }
 }
 
-// ascending over the N elements of each row group (bitonic: block sizes K = 2 .. N, partner distances J = K/2 .. 1)
-template <int K, int J, int G, int S, int N>
-__device__ inline void grp_sort_from(unsigned (&key)[S], int gl) {
-  grp_cx<K, J, G, S>(key, gl);
-  if constexpr (J > 1) grp_sort_from<K, J / 2, G, S, N>(key, gl);
-  else if constexpr (K < N) grp_sort_from<K * 2, K, G, S, N>(key, gl);
-}
-template <int G, int S, int N>
-__device__ inline void grp_sort(unsigned (&key)[S], int gl) {
-  grp_sort_from<2, 1, G, S, N>(key, gl);
-}
-
-// The value of slot-array v at element x of the group (lane x % G, slot x / G). Every lane runs the exchanges.
-template <int G, int S, typename V>
-__device__ inline V grp_at(const V (&v)[S], int x) {
-  V r = V(0);
-#pragma unroll
-  for (int s = 0; s < S; s++) {
-    const V t = __shfl(v[s], x & (G - 1), G);
-    if (x / G == s) r = t;
-  }
-  return r;
-}
-
-// One row per group of G lanes, 32 / G products per lane (G = 8: eight rows per wavefront; measured on the FP64
-// Laplacian square, 16.7 M rows of 25 products: G = 32 9.4 ms, 16 7.5 ms, 8 6.6 ms, 4 8.5 ms): expand, sort,
+// One row per group of G lanes, four products per lane (G = 8 for 32 products: eight rows per wavefront): expand, sort,
 // compress, write. `next` runs once the row's last global loads are issued (the caller's prefetch of its next row
 // overlaps them). Every exchange is executed by all groups of the wavefront.
+// Bound by issued instructions: the VALU, and the LDS pipe that lane exchanges and LDS accesses share (all four SIMDs of a CU
+// use one). So entries are found by a popcount over a bit mask of their first products instead of a search by lane
+// exchanges, prefixes and neighbours move by DPP, runs come from a bit mask of their heads, and products
+// are put in sorted order in LDS and summed from there: about 60 LDS operations per row group instead of 300 and, with the
+// sort above, 400 VALU instructions instead of 590 (numeric pass of the same square 4.26 -> 2.26 ms, symbolic 1.46 -> 0.99 ms).
 template <int MODE, int G, int N, typename T, typename RP, typename NEXT>
 __device__ inline void small_row(const RowsDev<T, RP>& R, const TileDev<T, RP>& tile, int fr, bool active, RP a0,
-                                 RP a1, int grp, int gl, NEXT&& next) {
+                                 RP a1, int grp, int gl, RP* s_delta, T* s_av, double* s_val, unsigned* s_key,
+                                 NEXT&& next) {
   constexpr bool NUM = MODE != 0;
   constexpr int S = N / G;
   constexpr unsigned kShift = N == 32 ? 5 : 6;  // product-index bits of a key
-  static_assert(N == 32 || N == 64, "rows of at most 32 or 64 products");
+  using Bits = std::conditional_t<N == 32, unsigned, unsigned long long>;  // a bit per product position of the row
+  static_assert(S == 4 && (G == 8 || G == 16), "four products per lane, a group inside one 16-lane DPP row");
+  auto wave_sync = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  auto group_bits = [&](bool v) { return (unsigned)(__ballot(v) >> (grp * G)) & ((1u << G) - 1u); };
+  auto count_bits = [](Bits v) { return N == 32 ? __popc((unsigned)v) : __popcll((unsigned long long)v); };
   const int na = (int)(a1 - a0);
-  int na_max = na;
-#pragma unroll
-  for (int d = G; d < 64; d <<= 1) na_max = max(na_max, __shfl_xor(na_max, d, 64));
   // expand: product x (A-row order) goes to slot x / G of lane x % G of the group
   unsigned key[S];
-  double pv[S];
 #pragma unroll
-  for (int q = 0; q < S; q++) {
-    key[q] = kEscPad;
-    pv[q] = 0.0;
-  }
+  for (int q = 0; q < S; q++) key[q] = kEscPad;
   int base = 0;
-  for (int c0 = 0; c0 < na_max; c0 += G) {
-    const int ne = min(max(na - c0, 0), G);
+  for (int c0 = 0; __ballot(c0 < na) != 0ull; c0 += G) {
     int len = 0;
     RP st = 0;
     T av = T(0);
-    if (gl < ne) {
-      const int kk = tile.a_col[a0 + c0 + gl];
-      st = tile.b_rp[kk];
-      len = (int)(tile.b_rp[kk + 1] - st);
-      if (NUM) av = tile.a_val[a0 + c0 + gl];
+    if (c0 + gl < na) {
+      const int kk = glob(tile.a_col)[a0 + c0 + gl];
+      st = glob(tile.b_rp)[kk];
+      len = (int)(glob(tile.b_rp)[kk + 1] - st);
+      if (NUM) av = glob(tile.a_val)[a0 + c0 + gl];
     }
     int inc = len;
-#pragma unroll
-    for (int d = 1; d < G; d <<= 1) {
-      const int t = __shfl_up(inc, d, G);
-      if (gl >= d) inc += t;
+    {
+      int t = (int)dpp_below<1>((unsigned)inc);
+      if (gl >= 1) inc += t;
+      t = (int)dpp_below<2>((unsigned)inc);
+      if (gl >= 2) inc += t;
+      t = (int)dpp_below<4>((unsigned)inc);
+      if (gl >= 4) inc += t;
+      if constexpr (G == 16) inc += (int)dpp_below<8>((unsigned)inc);
     }
     const int ex = inc - len;
     const int total = __shfl(inc, G - 1, G);
+    // the entries that have products, in order, and a bit at each one's first product
+    const int rank = __popc(group_bits(len > 0) & ((1u << gl) - 1u));
+    if (len > 0) {
+      s_delta[rank] = st - (RP)ex;
+      if (NUM) s_av[rank] = av;
+    }
+    auto or_group = [&](unsigned v) {
+      v |= dpp_xor<1>(v);
+      v |= dpp_xor<2>(v);
+      v |= dpp_xor<7>(v);
+      if constexpr (G == 16) v |= dpp_xor<15>(v);
+      return v;
+    };
+    const unsigned lo = or_group(len > 0 && ex < 32 ? 1u << ex : 0u);
+    unsigned hi = 0;
+    if constexpr (N == 64) hi = or_group(len > 0 && ex >= 32 ? 1u << (ex - 32) : 0u);
+    wave_sync();
 #pragma unroll
     for (int q = 0; q < S; q++) {
       const int t = gl + G * q - base;
-      int lo = 0;  // the entry holding product t: the last e < ne with ex[e] <= t
-#pragma unroll
-      for (int step = G / 2; step > 0; step >>= 1) {
-        const int c = lo + step;
-        const int v = __shfl(ex, c < G ? c : G - 1, G);
-        if (c < ne && v <= t) lo = c;
-      }
-      const RP st_e = __shfl(st, lo, G);
-      const int ex_e = __shfl(ex, lo, G);
-      const T av_e = __shfl(av, lo, G);
-      if (t >= 0 && t < total) {  // the row has at most N products, so base + total <= N
-        const RP qb = st_e + (RP)(t - ex_e);
-        key[q] = ((unsigned)tile.b_col[qb] << kShift) | (unsigned)(gl + G * q);
-        if (NUM) pv[q] = (double)av_e * (double)tile.b_val[qb];
+      if ((unsigned)t < (unsigned)total) {  // the row has at most N products, so base + total <= N
+        int e;  // the entry holding product t
+        if constexpr (N == 32) e = __popc(lo & ((2u << t) - 1u)) - 1;
+        else e = (t < 32 ? __popc(lo & ((2u << t) - 1u)) : __popc(lo) + __popc(hi & ((2u << (t - 32)) - 1u))) - 1;
+        const RP qb = s_delta[e] + (RP)t;
+        key[q] = ((unsigned)glob(tile.b_col)[qb] << kShift) | (unsigned)(gl + G * q);
+        if (NUM) s_val[gl + G * q] = (double)s_av[e] * (double)glob(tile.b_val)[qb];
       }
     }
+    wave_sync();
     base += total;
   }
   next();
-  grp_sort<G, S, N>(key, gl);
+  grp_sort<G>(key, gl);
   // compress: a sorted position starts an output entry when its column differs from the previous position's
-  unsigned hm[S];
-  bool head[S];
-  int cnt = 0;
+  if constexpr (MODE == 0) {
+    const unsigned up = dpp_below<1>(key[S - 1]);
+    unsigned cnt = 0;
 #pragma unroll
-  for (int q = 0; q < S; q++) {
-    const unsigned up = __shfl_up(key[q], 1, G);
-    const unsigned wrap = q > 0 ? __shfl(key[q > 0 ? q - 1 : 0], G - 1, G) : 0u;
-    const unsigned prev = gl > 0 ? up : wrap;
-    head[q] = key[q] != kEscPad && (gl + q * G == 0 || (prev >> kShift) != (key[q] >> kShift));
-    hm[q] = (unsigned)((__ballot(head[q]) >> (grp * G)) & (G == 32 ? 0xffffffffull : ((1ull << G) - 1)));
-    cnt += __popc(hm[q]);
-  }
-  if (MODE == 0) {
-    if (active && gl == 0) R.nnz[fr] = cnt;
+    for (int q = 0; q < S; q++) {
+      const unsigned prev = q > 0 ? key[q > 0 ? q - 1 : 0] : up;
+      cnt += key[q] != kEscPad && ((q == 0 && gl == 0) || (prev >> kShift) != (key[q] >> kShift)) ? 1u : 0u;
+    }
+    cnt += dpp_xor<1>(cnt);
+    cnt += dpp_xor<2>(cnt);
+    cnt += dpp_xor<7>(cnt);
+    if constexpr (G == 16) cnt += dpp_xor<15>(cnt);
+    if (active && gl == 0) R.nnz[fr] = (int)cnt;
     return;
   }
+  // from here on position x sits in slot x / G of lane x % G: neighbouring lanes take neighbouring outputs and LDS banks
+#pragma unroll
+  for (int q = 0; q < S; q++) s_key[gl * S + q] = key[q];
+  wave_sync();
+  Bits heads = 0;
+  bool head[S];
+  double sum[S];
+#pragma unroll
+  for (int q = 0; q < S; q++) {
+    key[q] = s_key[gl + G * q];
+    // the pad keys sort last, so the positions before `base` hold the products
+    sum[q] = gl + G * q < base ? s_val[key[q] & (unsigned)(N - 1)] : 0.0;
+  }
+#pragma unroll
+  for (int q = 0; q < S; q++) {
+    const unsigned wrap = q > 0 ? dpp_above<G - 1>(key[q > 0 ? q - 1 : 0]) : 0u;  // lane 0's: of lane G - 1
+    const unsigned up = dpp_below<1>(key[q]);
+    const unsigned prev = gl > 0 ? up : wrap;
+    head[q] = gl + G * q < base && (gl + G * q == 0 || (prev >> kShift) != (key[q] >> kShift));
+    heads |= (Bits)group_bits(head[q]) << (G * q);
+  }
+  const int cnt = count_bits(heads);
+  wave_sync();
+#pragma unroll
+  for (int q = 0; q < S; q++)
+    if (gl + G * q < base) s_val[gl + G * q] = sum[q];
   long long o = 0;
   if (active && gl == 0) {
     if (MODE == 1 || (MODE == 2 && cnt <= R.cap[fr])) {
@@ -1174,58 +1261,51 @@ __device__ inline void small_row(const RowsDev<T, RP>& R, const TileDev<T, RP>& 
     R.nnz[fr] = (o < 0 && MODE != 1) ? 0 : cnt;
   }
   o = __shfl(o, 0, G);
+  wave_sync();
   // sum each run of equal columns in sorted order, i.e. in product order, by the run's first element
-  double mine[S], sum[S];
-  bool run[S];
+  int len[S];
 #pragma unroll
   for (int q = 0; q < S; q++) {
-    const int pidx = (int)(key[q] & (unsigned)(N - 1));
-    double got = 0.0;
-#pragma unroll
-    for (int r = 0; r < S; r++) {
-      const double t = __shfl(pv[r], pidx & (G - 1), G);
-      if (pidx / G == r) got = t;
-    }
-    mine[q] = got;
-    sum[q] = got;
-    run[q] = head[q];
+    const int x = gl + G * q;
+    const Bits later = heads >> x >> 1;
+    len[q] = !head[q] ? 0 : later == 0 ? base - x : (N == 32 ? __ffs((int)later) : __ffsll((long long)later));
   }
-  for (int j = 1; j < N; j++) {
-    bool any = false;
+  for (int j = 1; __ballot(max(max(len[0], len[1]), max(len[2], len[3])) > j) != 0ull; j++) {
 #pragma unroll
-    for (int q = 0; q < S; q++) {
-      const int x = q * G + gl + j;  // the element j places after this one
-      const unsigned kj = grp_at<G, S>(key, x);
-      const double vj = grp_at<G, S>(mine, x);
-      run[q] = run[q] && x < N && kj != kEscPad && (kj >> kShift) == (key[q] >> kShift);
-      if (run[q]) sum[q] += vj;
-      any = any || run[q];
-    }
-    if (__ballot(any) == 0ull) break;
+    for (int q = 0; q < S; q++)
+      if (j < len[q]) sum[q] += s_val[gl + G * q + j];
   }
   if (o >= 0) {
-    int before = 0;
 #pragma unroll
     for (int q = 0; q < S; q++) {
       if (head[q]) {
-        const long long pos = o + before + __popc(hm[q] & ((1u << gl) - 1u));
+        const long long pos = o + count_bits(heads & (((Bits)1 << (gl + G * q)) - 1));
         // plain stores here: rows this small write a fraction of a cache line each, and L2 merges neighbouring
         // rows' pieces before they reach HBM (streaming stores made a 4096^2-grid Laplacian 6.6 -> 7.2 ms)
-        tile.c_col[pos] = (int)(key[q] >> kShift);
-        tile.c_val[pos] = (T)sum[q];
+        glob(tile.c_col)[pos] = (int)(key[q] >> kShift);
+        glob(tile.c_val)[pos] = (T)sum[q];
       }
-      before += __popc(hm[q]);
     }
   }
+  wave_sync();  // the next row reuses the LDS
 }
 
 // ONE: every row belongs to tiles[0] (a single product): the tile is read once, and the next row's bin item and
 // A-row bounds are loaded while the current row runs, so a row waits on three dependent loads (A columns, B-row
-// bounds, B entries) instead of five. G: lanes per row (32 or 16).
+// bounds, B entries) instead of five. G: lanes per row (8 or 16), N: its most products (32 or 64).
 template <int MODE, bool ONE, int G, int N, typename T, typename RP>
-__global__ __launch_bounds__(64 * kSmallWaves) void k_esc_small(RowsDev<T, RP> R, int bin) {
+__global__ __launch_bounds__(64 * kSmallWaves, !ONE ? 6 : N == 32 ? 8 : 7) void k_esc_small(RowsDev<T, RP> R, int bin) {
   constexpr int RW = 64 / G;  // rows per wavefront
+  constexpr bool NUM = MODE != 0;
+  // per row group: the staged A entries (B position of product t of the staged entries, less t), the products' values by
+  // product index, the sorted keys. Strides of N + N / 4 put the rows of a wavefront on different banks.
+  constexpr int GROUPS = kSmallWaves * RW, STRIDE = N + N / 4;
+  __shared__ RP s_delta[GROUPS][G];
+  __shared__ T s_av[NUM ? GROUPS : 1][G];
+  __shared__ double s_val[NUM ? GROUPS : 1][STRIDE];
+  __shared__ __align__(16) unsigned s_key[NUM ? GROUPS : 1][STRIDE];
   const int lane = threadIdx.x & 63, grp = lane / G, gl = lane % G;
+  const int gi = (int)(threadIdx.x >> 6) * RW + grp, gn = NUM ? gi : 0;
   const int count = *R.count_of(bin);
   const int* items = R.bin_items + (int64_t)bin * R.bin_stride;
   const int stride = gridDim.x * kSmallWaves * RW;
@@ -1236,18 +1316,18 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_esc_small(RowsDev<T, RP> R
     int fr = active ? items[p + grp] : 0;
     RP a0 = 0, a1 = 0;
     if (active) {
-      a0 = tile.a_rp[fr - tile.flat0];
-      a1 = tile.a_rp[fr - tile.flat0 + 1];
+      a0 = glob(tile.a_rp)[fr - tile.flat0];
+      a1 = glob(tile.a_rp)[fr - tile.flat0 + 1];
     }
     for (; p < count; p += stride) {
       const int64_t idx_n = p + stride + grp;
       const bool act_n = idx_n < count;
       const int fr_n = act_n ? items[idx_n] : 0;
       RP a0_n = 0, a1_n = 0;
-      small_row<MODE, G, N>(R, tile, fr, active, a0, a1, grp, gl, [&] {
+      small_row<MODE, G, N>(R, tile, fr, active, a0, a1, grp, gl, s_delta[gi], s_av[gn], s_val[gn], s_key[gn], [&] {
         if (act_n) {
-          a0_n = tile.a_rp[fr_n - tile.flat0];
-          a1_n = tile.a_rp[fr_n - tile.flat0 + 1];
+          a0_n = glob(tile.a_rp)[fr_n - tile.flat0];
+          a1_n = glob(tile.a_rp)[fr_n - tile.flat0 + 1];
         }
       });
       active = act_n;
@@ -1265,10 +1345,10 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_esc_small(RowsDev<T, RP> R
       if (active) {
         tile = R.tiles[R.blk_tile[fr >> 8]];
         const int64_t i = fr - tile.flat0;
-        a0 = tile.a_rp[i];
-        a1 = tile.a_rp[i + 1];
+        a0 = glob(tile.a_rp)[i];
+        a1 = glob(tile.a_rp)[i + 1];
       }
-      small_row<MODE, G, N>(R, tile, fr, active, a0, a1, grp, gl, [] {});
+      small_row<MODE, G, N>(R, tile, fr, active, a0, a1, grp, gl, s_delta[gi], s_av[gn], s_val[gn], s_key[gn], [] {});
     }
   }
 }
