@@ -71,6 +71,9 @@ void FlatRows<T, RP>::layout(bool with_cap, bool pooled, bool* from_pool) {
   size_t o_pi = A.reserve(sizeof(int32_t) * (with_cap ? nflat : 1));
   size_t o_cur = A.reserve(sizeof(unsigned long long) * 2);
   size_t o_tmp = A.reserve(sizeof(int32_t) * nflat);
+  size_t o_hh = A.reserve(sizeof(HeavyHead));
+  size_t o_hp = A.reserve(sizeof(HeavyPart) * kMaxHeavyParts);
+  size_t o_hf = A.reserve(sizeof(int32_t) * nflat);
   size_t o_stats = A.reserve(sizeof(unsigned long long) * 8);
   size_t nsb = (size_t)((nflat + kScanTile - 1) / kScanTile) + 1;
   size_t o_part = A.reserve(sizeof(long long) * nsb);
@@ -99,6 +102,9 @@ void FlatRows<T, RP>::layout(bool with_cap, bool pooled, bool* from_pool) {
   R.cursor = A.at<unsigned long long>(o_cur);
   R.heavy_queue = R.cursor + 1;
   R.tmp_items = A.at<int32_t>(o_tmp);
+  R.heavy_head = A.at<HeavyHead>(o_hh);
+  R.heavy_parts = A.at<HeavyPart>(o_hp);
+  R.heavy_first = A.at<int32_t>(o_hf);
   R.stats = A.at<unsigned long long>(o_stats);
   scan_partial = A.at<long long>(o_part);
   scan_total = A.at<int64_t>(o_tot);
@@ -276,7 +282,25 @@ void launch_esc_block(const RowsDev<T, RP>& R, hipStream_t s, int mode, int b, u
 }
 
 template <typename T, typename RP>
-void FlatRows<T, RP>::run_bin(hipStream_t s, int mode, int b, int64_t count_hint) {
+void FlatRows<T, RP>::plan_heavy(hipStream_t s, int mode) {
+  if ((max_n + 31) / 32 > kHRWords) return;  // the wide-tile kernel runs every row whole
+  if (mode == 1) {
+    hipLaunchKernelGGL((k_order_heavy<false, T, RP>), dim3(1), dim3(1024), 0, s, R);  // the symbolic pass split them
+  } else {
+    const unsigned cus = (unsigned)h->num_cus;
+    hipLaunchKernelGGL((k_order_heavy<true, T, RP>), dim3(1), dim3(1024), 0, s, R);
+    hipLaunchKernelGGL((k_heavy_split<T, RP>), dim3(cus), dim3(1024), 0, s, R);
+    if (mode != 0) {
+      hipLaunchKernelGGL((k_heavy_rank<0, T, RP>), dim3(2 * cus), dim3(hr_block<0>()), 0, s, R, kHeavyParts);
+      if (mode == 2) hipLaunchKernelGGL((k_heavy_place<2, T, RP>), dim3(64), dim3(256), 0, s, R);
+      else hipLaunchKernelGGL((k_heavy_place<3, T, RP>), dim3(64), dim3(256), 0, s, R);
+    }
+  }
+  BCLX_HIP(hipGetLastError());
+}
+
+template <typename T, typename RP>
+void FlatRows<T, RP>::run_bin(hipStream_t s, int mode, int b, int64_t count_hint, bool planned) {
   // count_hint >= 0: exact row count known on the host (grid sized to it); < 0: persistent grid.
   if (b == 0 || count_hint == 0) return;
   // rows of at most 32 products (bin 18) and of 33-64 (ESC bin 11): sorted in registers by groups of G lanes
@@ -328,15 +352,18 @@ void FlatRows<T, RP>::run_bin(hipStream_t s, int mode, int b, int64_t count_hint
     return;
   }
   if (b == kHeavyBin && (max_n + 31) / 32 <= kHRWords) {
-    const int64_t resident = (mode == 0 ? 2 : 1) * (int64_t)h->num_cus;
-    const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(count_hint >= 0 ? count_hint : resident, resident));
-    fill_u64(s, R.heavy_queue, 1, 0ull);
-    hipLaunchKernelGGL((k_order_heavy<T, RP>), dim3(1), dim3(1024), 0, s, R);
+    if (!planned) plan_heavy(s, mode);
+    // persistent: the parts of split rows and the whole rows are taken from a queue
+    const unsigned cus = (unsigned)h->num_cus;
     switch (mode) {
-      case 0: hipLaunchKernelGGL((k_heavy_rank<0, T, RP>), dim3(grid), dim3(hr_block<0>()), 0, s, R, kHeavyBin); break;
-      case 1: hipLaunchKernelGGL((k_heavy_rank<1, T, RP>), dim3(grid), dim3(hr_block<1>()), 0, s, R, kHeavyBin); break;
-      case 2: hipLaunchKernelGGL((k_heavy_rank<2, T, RP>), dim3(grid), dim3(hr_block<2>()), 0, s, R, kHeavyBin); break;
-      default: hipLaunchKernelGGL((k_heavy_rank<3, T, RP>), dim3(grid), dim3(hr_block<3>()), 0, s, R, kHeavyBin); break;
+      case 0:
+        hipLaunchKernelGGL((k_heavy_rank<0, T, RP>), dim3(2 * cus), dim3(hr_block<0>()), 0, s, R, kHeavyAll);
+        hipLaunchKernelGGL((k_heavy_place<0, T, RP>), dim3(64), dim3(256), 0, s, R);
+        hipLaunchKernelGGL((k_heavy_rank<0, T, RP>), dim3(2 * cus), dim3(hr_block<0>()), 0, s, R, kHeavyBad);
+        break;
+      case 1: hipLaunchKernelGGL((k_heavy_rank<1, T, RP>), dim3(cus), dim3(hr_block<1>()), 0, s, R, kHeavyAll); break;
+      case 2: hipLaunchKernelGGL((k_heavy_rank<2, T, RP>), dim3(cus), dim3(hr_block<2>()), 0, s, R, kHeavyAll); break;
+      default: hipLaunchKernelGGL((k_heavy_rank<3, T, RP>), dim3(cus), dim3(hr_block<3>()), 0, s, R, kHeavyAll); break;
     }
     BCLX_HIP(hipGetLastError());
     return;

@@ -38,6 +38,12 @@ __host__ __device__ constexpr int bin_group(int b) {
   return b == 1 ? 16 : b == 2 ? 32 : b <= 5 ? 64 : b == 6 ? 256 : b <= 8 ? 512 : 1024;
 }
 
+// Tiles at most 2^19 columns wide: rows of more than 4096 products that need more entries than this run in the
+// rank-slice kernel of the heavy bin, whatever heavy_need allows to hash. 20000 rows of 6400 products: 3190 entries
+// 2.1 ms there and 7.8 ms hashed, 1918 entries 2.1 and 4.3 ms, 998 entries 2.1 and 1.95 ms; rows of 90000 products with
+// 1500 entries 2.3 and 3.3 ms; R-MAT square at scale 16 1.79 and 2.34 ms.
+constexpr int kRankNeed = 1024;
+
 // Tunable binning knobs (chosen by the autotuner; these are the defaults).
 struct BinTuning {
   int32_t work_per_lane = 64;     // a row's group must have >= products / work_per_lane lanes
@@ -61,7 +67,7 @@ __host__ __device__ inline int bin_for(int64_t need, int64_t work, const BinTuni
   if (tn.esc_max > 0 && work <= kSmallMax && n < ((int64_t)1 << kSmallColBits) - 1) return kSmallBin;
   const bool esc_ok = n <= (1 << kEscColBits);
   if (esc_ok && work > tn.esc_min && work <= tn.esc_max && work <= kEscMaxProducts) return esc_bin(work);
-  if (need > tn.heavy_need) return kHeavyBin;
+  if (need > (esc_ok && tn.heavy_need > kRankNeed ? kRankNeed : tn.heavy_need)) return kHeavyBin;
   int64_t slots = need << tn.load_shift;
   int bn = 1;
   while (bn < 9 && bin_table(bn) < slots) bn++;
@@ -99,6 +105,34 @@ struct TileDev {
   int64_t krows;           // rows of B
 };
 
+// A column range of a heavy row (split rows: see k_heavy_split). Bounds are multiples of kHRGroup words of columns.
+struct HeavyPart {
+  int32_t fr, lo, hi;  // row, columns [lo, hi)
+  int32_t parts;       // of a row's first part: its number of parts
+  int32_t nnz;         // the part's output entries
+  int32_t bad;         // of a row's first part: a B row's columns are not sorted, the row runs whole
+  int32_t split_row;   // entry q: first part of the q-th split row
+  int32_t pad;
+  int64_t off;         // output offset: in the row (symbolic), in C (modes 2 and 3; < 0: refused)
+};
+struct HeavyHead {
+  int32_t parts, split_rows;
+  int32_t ordered;  // whole rows in the heavy bin's list
+  int32_t rows;     // with the split rows found bad, appended to the list
+};
+// Products of a part: about an eighth of a compute unit's share of all heavy products, so the last one to finish is short,
+// between 8192 (below, staging a part costs as much as its products) and 2^18, and never so few that more than
+// kMaxHeavyParts parts would be made (a row of P gives ceil(P / size) parts and only rows with more than size are
+// split, so total / (kMaxHeavyParts / 2) is enough).
+constexpr int kMaxHeavyParts = 16384;
+constexpr int kMaxRowParts = 256;
+__host__ __device__ inline long long heavy_part_size(long long total) {
+  const long long share = total / 2048, most = (total + kMaxHeavyParts / 2 - 1) / (kMaxHeavyParts / 2);
+  long long size = share < (1 << 18) ? share : (1 << 18);
+  size = size > 8192 ? size : 8192;
+  return size > most ? size : most;
+}
+
 template <typename T, typename RP>
 struct RowsDev {
   const TileDev<T, RP>* tiles;
@@ -122,10 +156,20 @@ struct RowsDev {
   unsigned long long* cursor;  // bump allocator for rows placed outside their predicted slot
   unsigned long long* heavy_queue;  // next heavy row to take (rows are handed out largest first)
   int32_t* tmp_items;               // scratch list for ordering the heavy bin
+  HeavyHead* heavy_head;
+  HeavyPart* heavy_parts;           // kMaxHeavyParts
+  int32_t* heavy_first;             // per row of the heavy bin: its first part, -1 if it is not split
   unsigned long long* stats;   // [0] products [1] heavy rows [2] overflow rows [3] capacity exceeded [4] predicted
   long long out_limit;         // entries available in the output arrays; writes beyond it are refused
   BinTuning tn;
 };
+
+// A pointer read from device memory, as one to global memory: the compiler then emits global loads and stores. Flat ones also
+// count as LDS operations, so that each LDS wait waits for them.
+template <typename P>
+__device__ inline __attribute__((address_space(1))) P* glob(P* p) {
+  return (__attribute__((address_space(1))) P*)p;
+}
 
 // ------------------------------------------------------------------------------------------------------------
 // reductions / scans
@@ -179,6 +223,32 @@ __device__ inline V block_sum(V v, V* smem) {
   V t;
   (void)block_excl_scan<BLOCK, V>(v, &t, smem);
   return t;
+}
+
+// Inclusive scan of one int per lane of a wavefront, by DPP: six VALU instructions, no LDS.
+__device__ inline int wave_scan_dpp(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, true);   // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2 and 3
+  return v;
+}
+
+// Block-wide exclusive scan of one int per thread with one barrier. `smem` (BLOCK / 64 ints) may be written again only
+// after another barrier.
+template <int BLOCK>
+__device__ inline int block_scan_dpp(int v, int* total, int* smem) {
+  constexpr int NW = BLOCK / 64;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int inc = wave_scan_dpp(v);
+  if (lane == 63) smem[w] = inc;
+  __syncthreads();
+  const int waves = wave_scan_dpp(lane < NW ? smem[lane] : 0);
+  *total = __builtin_amdgcn_readlane(waves, NW - 1);
+  const int before = w > 0 ? __builtin_amdgcn_readlane(waves, w - 1) : 0;
+  return before + inc - v;
 }
 
 // ------------------------------------------------------------------------------------------------------------
@@ -799,13 +869,6 @@ __device__ inline void esc_lookup(const int* pre, int ne, int base, int lane, in
       if (c < ne && pre[c] <= x0 + k * 64 + lane - base) lo[k] = c;
     }
   }
-}
-
-// A pointer read from device memory, as one to global memory: the compiler then emits global loads and stores. Flat ones also
-// count as LDS operations, so that each LDS wait waits for them.
-template <typename P>
-__device__ inline __attribute__((address_space(1))) P* glob(P* p) {
-  return (__attribute__((address_space(1))) P*)p;
 }
 
 // Compare-exchange of one bitonic stage whose partner is `d` lanes away (d < 64): keep min or max of the pair.
@@ -1518,16 +1581,31 @@ __global__ __launch_bounds__(64 * W, 6) void k_esc_block(RowsDev<T, RP> R, int b
 }
 
 // ------------------------------------------------------------------------------------------------------------
-// Heavy rows (more products than the sort-based bins take and more output entries than the largest hash table),
-// rank-slice accumulator: one workgroup per row, everything in LDS.
+// Heavy rows (more products than the sort-based bins take and more output entries than the hash tables are given),
+// rank-slice accumulator: one workgroup per row, or per part of a split row, everything in LDS.
 //   pass 1: LDS bitmap of the row's columns (one atomicOr per product) and prefix counts per group of kHRGroup
-//           words, so every column's output rank is known and nnz(C_i) is exact; the columns are written straight
-//           from the bitmap;
-//   pass 2 (numeric modes), per slice of hr_slice() ranks: the products whose columns fall in the slice's column range
-//           are added in float64 into an LDS array indexed by rank - slice start (ds_add_f64), then written out with
-//           unit stride. Most rows fit one slice; larger rows enumerate their products once per slice.
+//           words, so every column's output rank is known and nnz(C_i) is exact;
+//   pass 2 (numeric modes), per slice of hr_slice() ranks: the slice's columns are written from the bitmap, and the
+//           products whose columns fall in its column range are added in float64 into an LDS array indexed by
+//           rank - slice start (ds_add_f64), then written out with unit stride. Most rows fit one slice; larger
+//           rows enumerate their products once per slice.
 // Modes as in k_hash: 0 symbolic, 1 numeric at off[fr], 2 predicted (slot if nnz <= cap, else bump-allocate),
 // 3 bump-allocate. Needs n <= 32 * kHRWords; wider tiles use k_heavy (global dense accumulator).
+//
+// A row with more products than heavy_part_size() is split by columns into parts of about that many: an R-MAT
+// square at scale 16 has one row of 0.2 % of its products, and the workgroup that ran it alone took 1.6 times the
+// average (19 M cycles of 10 M on average in a stage of 4 x 4 tiles at scale 21). Order of a pass:
+//   k_order_heavy   picks the rows to split and orders the others by size
+//   k_heavy_split   samples a split row's columns and cuts them into ranges with equal samples
+//   k_heavy_rank<0> counts each part's entries (symbolic: and the whole rows')
+//   k_heavy_place   sums a row's parts and, in modes 2 and 3, gives them their places in C
+//   k_heavy_rank    the parts (largest pieces) first, then the whole rows, from one queue
+// A part finds its share of each B row by binary search. Nothing else needs a B row's columns sorted, so the counting pass
+// checks each product's column against the part's range: the parts' shares tile every B row, so if all
+// columns are inside, nothing is missed. Otherwise the row runs whole.
+// R-MAT square at scale 16 (122 M products): symbolic 0.53 -> 0.20 ms, numeric 1.76 -> 0.62 ms with the parts, the
+// product loop of enumerate_waves and a word of the bitmap per lane when the columns are written. Bound now by LDS latency and
+// atomics with one workgroup of 16 wavefronts per CU.
 // ------------------------------------------------------------------------------------------------------------
 
 constexpr int kHRWords = 16384;  // bitmap words: tiles up to 2^19 columns
@@ -1555,9 +1633,9 @@ __device__ inline int hr_rank(const unsigned* bits, const int* gpre, int j) {
          __popc((wi == 0 ? x.x : wi == 1 ? x.y : wi == 2 ? x.z : x.w) & below);
 }
 
-// Column of output rank r (0 <= r < number of set bits): the r-th set bit. One thread.
-__device__ inline int hr_select(const unsigned* bits, const int* gpre, int ng, int r) {
-  int lo = 0, hi = ng;  // last group with gpre <= r
+// Column of output rank r (0 <= r < number of set bits): the r-th set bit of groups [g0, g1). One thread.
+__device__ inline int hr_select(const unsigned* bits, const int* gpre, int g0, int g1, int r) {
+  int lo = g0, hi = g1;  // last group with gpre <= r
   while (hi - lo > 1) {
     const int mid = (lo + hi) >> 1;
     if (gpre[mid] <= r) lo = mid; else hi = mid;
@@ -1586,69 +1664,366 @@ __device__ inline RP hr_lower_bound(const int* b_col, RP st, RP lo0, RP len, int
   return lo;
 }
 
-// Orders the heavy bin by decreasing products (classes of equal floor(log2 P)), so that the dynamic queue of
-// k_heavy_rank starts the largest rows first and the small ones fill in behind them. One block.
-template <typename T, typename RP>
+// [lo, hi) of the B row at st of len entries whose columns are in [c_lo, c_hi) (binary searches in global memory, side by
+// side).
+template <typename RP>
+__device__ inline void hr_column_range(const int* b_col, RP st, RP len, int c_lo, int c_hi, RP* lo, RP* hi) {
+  RP l0 = 0, l1 = len, h0 = 0, h1 = len;
+  while (l0 < l1 || h0 < h1) {
+    const RP lm = (l0 + l1) >> 1, hm = (h0 + h1) >> 1;
+    const int lc = l0 < l1 ? glob(b_col)[st + lm] : 0, hc = h0 < h1 ? glob(b_col)[st + hm] : 0;
+    if (l0 < l1) {
+      if (lc < c_lo) l0 = lm + 1; else l1 = lm;
+    }
+    if (h0 < h1) {
+      if (hc < c_hi) h0 = hm + 1; else h1 = hm;
+    }
+  }
+  *lo = l0;
+  *hi = h0;
+}
+
+// The heavy bin before its rows run: decides which rows are split (BUILD; the numeric pass that follows a symbolic one
+// keeps that pass's parts) and orders the others by decreasing products (classes of equal floor(log2 P)), so that the
+// queue of k_heavy_rank starts the largest first and the small ones fill in behind them. One block.
+template <bool BUILD, typename T, typename RP>
 __global__ __launch_bounds__(1024) void k_order_heavy(RowsDev<T, RP> R) {
+  constexpr int U = 8;
   __shared__ int s_hist[32], s_next[32];
+  __shared__ int s_parts, s_split;
+  __shared__ long long s_scan[17];
+  const int tid = threadIdx.x;
   const int cnt = *R.count_of(kHeavyBin);
   int* items = R.bin_items + (int64_t)kHeavyBin * R.bin_stride;
-  if (threadIdx.x < 32) s_hist[threadIdx.x] = 0;
-  __syncthreads();
-  auto cls = [&](int fr) {  // 31 - floor(log2 P), clamped to [0, 31]: larger rows first
-    const long long p = R.prod[fr];
+  if (tid < 32) s_hist[tid] = 0;
+  if (tid == 0) {
+    s_parts = 0;
+    s_split = 0;
+    *R.heavy_queue = 0ull;
+  }
+  auto each = [&](auto&& f) {  // f(row, products), U rows in flight per thread
+    for (int q0 = tid; q0 < cnt; q0 += U * 1024) {
+      int fr[U];
+      long long p[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) fr[u] = q0 + u * 1024 < cnt ? items[q0 + u * 1024] : -1;
+#pragma unroll
+      for (int u = 0; u < U; u++) p[u] = fr[u] >= 0 ? R.prod[fr[u]] : 0;
+#pragma unroll
+      for (int u = 0; u < U; u++)
+        if (fr[u] >= 0) f(fr[u], p[u]);
+    }
+  };
+  auto cls = [&](long long p) {  // 31 - floor(log2 P), clamped to [0, 31]: larger rows first
     const int lg = 63 - __clzll((unsigned long long)(p > 1 ? p : 1));
     return 31 - (lg < 31 ? lg : 31);
   };
-  for (int q = threadIdx.x; q < cnt; q += blockDim.x) atomicAdd(&s_hist[cls(items[q])], 1);
+  long long size = LLONG_MAX;
+  if (BUILD) {
+    long long mine = 0;
+    each([&](int, long long p) { mine += p; });
+    size = heavy_part_size(block_sum<1024, long long>(mine, s_scan));
+  }
   __syncthreads();
-  if (threadIdx.x == 0) {
+  each([&](int fr, long long p) {
+    bool split = false;
+    if (BUILD) {
+      int first = -1;
+      if (p > size) {
+        const int n = R.tiles[R.blk_tile[fr >> 8]].n;
+        const int k = (int)min(min((p + size - 1) / size, (long long)kMaxRowParts), (long long)(n / (32 * kHRGroup)));
+        if (k > 1) {
+          first = atomicAdd(&s_parts, k);
+          R.heavy_parts[first].fr = fr;
+          R.heavy_parts[first].parts = k;
+          R.heavy_parts[first].bad = 0;
+          R.heavy_parts[atomicAdd(&s_split, 1)].split_row = first;
+          split = true;
+        }
+      }
+      R.heavy_first[fr] = first;
+    } else {
+      const int first = R.heavy_first[fr];
+      split = first >= 0 && !R.heavy_parts[first].bad;
+    }
+    if (!split) atomicAdd(&s_hist[cls(p)], 1);
+  });
+  __syncthreads();
+  if (tid == 0) {
     int run = 0;
     for (int c = 0; c < 32; c++) {
       s_next[c] = run;
       run += s_hist[c];
     }
+    R.heavy_head->ordered = run;
+    R.heavy_head->rows = run;
+    if (BUILD) {
+      R.heavy_head->parts = s_parts;
+      R.heavy_head->split_rows = s_split;
+    }
   }
   __syncthreads();
-  for (int q = threadIdx.x; q < cnt; q += blockDim.x) {
-    const int fr = items[q];
-    R.tmp_items[atomicAdd(&s_next[cls(fr)], 1)] = fr;
-  }
+  each([&](int fr, long long p) {
+    const int first = R.heavy_first[fr];
+    if (first < 0 || (!BUILD && R.heavy_parts[first].bad)) R.tmp_items[atomicAdd(&s_next[cls(p)], 1)] = fr;
+  });
   __syncthreads();
-  for (int q = threadIdx.x; q < cnt; q += blockDim.x) items[q] = R.tmp_items[q];
+  for (int q = tid; q < s_next[31]; q += 1024) items[q] = R.tmp_items[q];  // s_next[31] is now the end of the list
 }
 
+// Cuts the columns of each split row into ranges of about equal products: a histogram, by groups of kHRGroup words, of the columns
+// of 8192 to 16384 products at equal distances in product order. One workgroup per row.
+template <typename T, typename RP>
+__global__ __launch_bounds__(1024) void k_heavy_split(RowsDev<T, RP> R) {
+  constexpr int kSpan = 32 * kHRGroup;  // columns per group
+  __shared__ int s_hist[kHRWords / kHRGroup];
+  __shared__ RP s_delta[1024];
+  __shared__ int s_pre[1024];
+  __shared__ int s_scan[2][16];
+  const int tid = threadIdx.x;
+  const int nsplit = R.heavy_head->split_rows;
+  for (int q = blockIdx.x; q < nsplit; q += gridDim.x) {
+    const int first = R.heavy_parts[q].split_row;
+    HeavyPart* parts = R.heavy_parts + first;
+    const int fr = parts->fr, k = parts->parts;
+    const TileDev<T, RP> tile = R.tiles[R.blk_tile[fr >> 8]];
+    const RP a0 = tile.a_rp[fr - tile.flat0], a1 = tile.a_rp[fr - tile.flat0 + 1];
+    const long long p = R.prod[fr], stride = p / 8192 > 1 ? p / 8192 : 1;
+    const int groups = (tile.n + kSpan - 1) / kSpan;
+    for (int g = tid; g < groups; g += 1024) s_hist[g] = 0;
+    long long base = 0;  // products of the chunks before
+    for (RP c0 = a0; c0 < a1; c0 += 1024) {
+      const int ne = (int)((a1 - c0) < (RP)1024 ? (a1 - c0) : (RP)1024);
+      RP st = 0;
+      int len = 0;
+      if (tid < ne) {
+        const int kk = tile.a_col[c0 + tid];
+        st = tile.b_rp[kk];
+        len = (int)(tile.b_rp[kk + 1] - st);
+      }
+      int total;
+      const int ex = block_scan_dpp<1024>(len, &total, s_scan[0]);
+      if (tid < ne) {
+        s_delta[tid] = st - (RP)ex;
+        s_pre[tid] = ex;
+      }
+      __syncthreads();
+      int top = 1;
+      while (top < ne) top <<= 1;
+      top >>= 1;
+      for (long long smp = (base + stride - 1) / stride + tid; smp * stride < base + total; smp += 1024) {
+        const int t = (int)(smp * stride - base);
+        int e = 0;
+        for (int step = top; step > 0; step >>= 1)
+          if (e + step < ne && s_pre[e + step] <= t) e += step;
+        atomicAdd(&s_hist[tile.b_col[s_delta[e] + (RP)t] / kSpan], 1);
+      }
+      base += total;
+      __syncthreads();
+    }
+    // part x starts at the end of the group in which the running count passes x / k of the samples
+    constexpr int kPer = kHRWords / kHRGroup / 1024;
+    int mine = 0;
+#pragma unroll
+    for (int u = 0; u < kPer; u++) mine += tid * kPer + u < groups ? s_hist[tid * kPer + u] : 0;
+    int ns;
+    long long run = block_scan_dpp<1024>(mine, &ns, s_scan[1]);
+    for (int u = 0; u < kPer; u++) {
+      const int g = tid * kPer + u;
+      if (g >= groups) break;
+      const long long next = run + s_hist[g];
+      for (long long x = run * k / ns + 1; x < k && x * ns <= next * k; x++) {
+        parts[x].lo = (g + 1) * kSpan;
+        parts[x - 1].hi = (g + 1) * kSpan;
+      }
+      run = next;
+    }
+    if (tid == 0) {
+      parts[0].lo = 0;
+      parts[k - 1].hi = groups * kSpan;
+    }
+    for (int x = tid; x < k; x += 1024) {
+      parts[x].fr = fr;
+      parts[x].nnz = 0;
+    }
+    __syncthreads();
+  }
+}
+
+// After the parts are counted: a split row's entries are their sum; modes 2 and 3 also place it in C. Rows whose parts
+// met unsorted B rows join the list of whole rows. One wavefront per row.
 template <int MODE, typename T, typename RP>
-__global__ __launch_bounds__(hr_block<MODE>()) void k_heavy_rank(RowsDev<T, RP> R, int bin) {
+__global__ __launch_bounds__(256) void k_heavy_place(RowsDev<T, RP> R) {
+  const int lane = threadIdx.x & 63, nwaves = gridDim.x * 4;
+  const int nsplit = R.heavy_head->split_rows;
+  int* items = R.bin_items + (int64_t)kHeavyBin * R.bin_stride;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *R.heavy_queue = 0ull;
+  for (int q = blockIdx.x * 4 + (threadIdx.x >> 6); q < nsplit; q += nwaves) {
+    const int first = R.heavy_parts[q].split_row;
+    HeavyPart* parts = R.heavy_parts + first;
+    const int fr = parts->fr, k = parts->parts;
+    const bool bad = parts->bad != 0;
+    static_assert(kMaxRowParts == 4 * 64, "four parts per lane");
+    int cnt[4], mine = 0;
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      cnt[u] = lane * 4 + u < k ? parts[lane * 4 + u].nnz : 0;
+      mine += cnt[u];
+    }
+    const int inc = wave_scan_dpp(mine);
+    const int total = __builtin_amdgcn_readlane(inc, 63);
+    long long b = 0;
+    if (lane == 0) {
+      if (bad) {
+        items[atomicAdd(&R.heavy_head->rows, 1)] = fr;
+      } else {
+        if (MODE != 0) {
+          if (MODE == 2 && total <= R.cap[fr]) {
+            b = R.off[fr];
+          } else {
+            b = (long long)atomicAdd(R.cursor, (unsigned long long)total);
+            R.off[fr] = b;
+          }
+          if (b + total > R.out_limit) {  // refused, as a whole row is
+            R.stats[3] = 1ull;
+            b = -1;
+            R.off[fr] = 0;
+          }
+        }
+        R.nnz[fr] = b < 0 ? 0 : total;
+        atomicAdd(&R.stats[1], 1ull);
+      }
+    }
+    b = __shfl(b, 0, 64);
+    long long off = b + inc - mine;
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      if (lane * 4 + u < k) parts[lane * 4 + u].off = b < 0 ? -1 : off;
+      off += cnt[u];
+    }
+  }
+}
+
+// The product loop of a staged chunk of A entries, a run of consecutive products per wavefront. Entry e's products are
+// t in [e_pre[e], e_pre[e + 1]) at B positions e_delta[e] + t (e_pre[0] = 0; the last entry ends at `total`). A wavefront keeps
+// the entry of its next product and, for each 64 products, reads the starts of the 64 entries that follow:
+// the few that lie inside are broadcast and counted per lane (a B row of a heavy row is mostly longer than 64), more than
+// eight are searched. A binary search per product over the whole chunk took 5 to 10 dependent LDS reads
+// and more instructions than everything else in the pass. U * 64 products are loaded at a time, ahead of the
+// ones being added. f(column, a, b) per product.
+template <int BLOCK, bool NUM, int U, typename T, typename RP, typename F>
+__device__ inline void enumerate_waves(const TileDev<T, RP>& tile, int ne, int total, int tid, const RP* e_delta,
+                                       const int* e_pre, const T* e_val, F&& f) {
+  static_assert(BLOCK <= 1024, "the entry search takes two steps of 64 for at most 4096 entries");
+  constexpr int NW = BLOCK / 64;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int seg = (total + NW * 64 - 1) / (NW * 64) * 64;
+  const int t_beg = w * seg, t_end = min(total, t_beg + seg);
+  if (t_beg >= t_end) return;
+  int e;  // an entry that starts at or before the next product, with none but empty ones between them
+  {
+    const int step = (ne + 63) >> 6;
+    e = (__popcll(__ballot(lane * step < ne && e_pre[lane * step < ne ? lane * step : 0] <= t_beg)) - 1) * step;
+    const int x = e + lane;
+    e += __popcll(__ballot(lane < step && x < ne && e_pre[x < ne ? x : 0] <= t_beg)) - 1;
+  }
+  struct Batch {
+    int j[U];
+    T a[U], b[U];
+  };
+  auto fetch = [&](int t0, Batch& r) {
+    RP q[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int tu = t0 + 64 * u, t = tu + lane;
+      q[u] = 0;
+      if (tu < t_end) {  // uniform
+        const int x = e + 1 + lane;
+        const int start = x < ne ? e_pre[x] : INT_MAX;
+        const int in = __popcll(__ballot(start <= tu + 63));
+        int c = 0;
+        if (in <= 8) {
+          for (int i = 0; i < in; i++) c += __builtin_amdgcn_readlane(start, i) <= t ? 1 : 0;
+        } else {
+          for (int step = in < 64 ? 32 : 512; step > 0; step >>= 1)
+            if (e + c + step < ne && e_pre[e + c + step] <= t) c += step;
+        }
+        const int et = e + c;
+        q[u] = e_delta[et] + (RP)t;
+        if (NUM) r.a[u] = e_val[et];
+        e = in < 64 ? e + in : __builtin_amdgcn_readlane(et, 63);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      if (t0 + 64 * u + lane < t_end) {
+        r.j[u] = glob(tile.b_col)[q[u]];
+        if (NUM) r.b[u] = glob(tile.b_val)[q[u]];
+      }
+  };
+  auto use = [&](int t0, const Batch& r) {
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      if (t0 + 64 * u + lane < t_end) f(r.j[u], NUM ? r.a[u] : T(0), NUM ? r.b[u] : T(0));
+  };
+  Batch now, next;
+  for (int t0 = t_beg - 64 * U; t0 < t_end; t0 += 64 * U) {
+    if (t0 + 64 * U < t_end) fetch(t0 + 64 * U, next);
+    if (t0 >= t_beg) use(t0, now);
+    now = next;
+  }
+}
+
+// A value that is the same in every lane, in scalar registers.
+template <typename V>
+__device__ inline V uniform(V v) {
+  static_assert(sizeof(V) == 4 || sizeof(V) == 8, "one or two registers");
+  int x[sizeof(V) / 4];
+  __builtin_memcpy(x, &v, sizeof(V));
+#pragma unroll
+  for (unsigned u = 0; u < sizeof(V) / 4; u++) x[u] = __builtin_amdgcn_readfirstlane(x[u]);
+  __builtin_memcpy(&v, x, sizeof(V));
+  return v;
+}
+
+// what k_heavy_rank takes: parts and whole rows; parts only; the rows k_heavy_place appended
+constexpr int kHeavyAll = 0, kHeavyParts = 1, kHeavyBad = 2;
+
+template <int MODE, typename T, typename RP>
+__global__ __launch_bounds__(hr_block<MODE>()) void k_heavy_rank(RowsDev<T, RP> R, int what) {
   constexpr int BLOCK = hr_block<MODE>();
   constexpr bool NUM = MODE != 0;
   constexpr int kHRSlice = hr_slice<T, RP>();
   __shared__ __align__(16) unsigned s_bits[kHRWords];
   __shared__ int s_gpre[NUM ? kHRWords / kHRGroup : 1];  // the symbolic pass needs only the total
   __shared__ __align__(16) double s_acc[NUM ? kHRSlice : 1];  // a slice's columns (as int), then its values
-  __shared__ long long s_scan[BLOCK / 64 + 1];
   __shared__ long long s_base;
   __shared__ int s_crange[2];
-  __shared__ RP s_est[BLOCK];
+  __shared__ RP s_delta[BLOCK];
   // product prefixes of one staged chunk fit 32 bits: at most BLOCK entries, each a B row of at most 2^19 columns
-  __shared__ int s_epre[BLOCK + 1];
-  __shared__ T s_eval[BLOCK];
-  __shared__ long long s_lscan[BLOCK / 64 + 1];
-  constexpr int kGroupsPerThread = (kHRWords / kHRGroup + BLOCK - 1) / BLOCK;
+  __shared__ int s_pre[BLOCK];
+  __shared__ T s_val[NUM ? BLOCK : 1];
+  __shared__ int s_scan[2][BLOCK / 64];
   const int tid = threadIdx.x;
-  const int count = *R.count_of(bin);
-  const int* items = R.bin_items + (int64_t)bin * R.bin_stride;
+  const HeavyHead head = *R.heavy_head;
+  const int nparts = what == kHeavyBad ? 0 : head.parts;
+  const int row0 = what == kHeavyBad ? head.ordered : 0;
+  const int count = nparts + (what == kHeavyParts ? 0 : head.rows - row0);
+  const int* items = R.bin_items + (int64_t)kHeavyBin * R.bin_stride + row0;
   int* s_colbuf = reinterpret_cast<int*>(s_acc);
   __shared__ int s_idx;
-  // Rows are taken from a queue (largest first), so one block's share is not fixed in advance. The next row is
-  // fetched while the current one runs: its queue slot when the current row starts, then one dependent load per
-  // barrier of the current row (bin item, tile, A row bounds, each entry's A column and value, its B-row range). A
+  // Parts and rows are taken from a queue (largest first), so one block's share is not fixed in advance. The next one is
+  // fetched while the current one runs: its queue slot when the current one starts, then one dependent load per
+  // barrier (bin item, tile, A row bounds, each entry's A column and value, its B-row range). A
   // row then starts with its staging in registers instead of behind a chain of global round trips.
-  int nq = 0;        // thread 0: the next row's queue slot
-  int pst = 0;       // fetch steps done for the next row (uniform)
+  int nq = 0;        // thread 0: the next one's queue slot
+  int pst = 0;       // fetch steps done for it (uniform)
   int n_idx = 0, n_fr = 0, n_tix = 0, n_kk = 0, n_cap = 0;  // n_cap, n_off: thread 0 only
+  int n_lo = 0, n_hi = 0;  // its columns; n_hi 0: none (nothing to do)
+  bool n_skip = false;
   long long n_off = 0;
-  RP n_a0 = 0, n_a1 = 0, n_st = 0, n_len = 0;
+  RP n_a0 = 0, n_a1 = 0, n_st = 0;
+  int n_len = 0;
   T n_av = T(0);
   auto advance = [&](int upto) {  // all threads, uniform upto; a barrier separates steps 1 and 2
     if (pst < 1 && upto >= 1) {
@@ -1658,20 +2033,42 @@ __global__ __launch_bounds__(hr_block<MODE>()) void k_heavy_rank(RowsDev<T, RP> 
     }
     if (pst < 2 && upto >= 2) {
       n_idx = __builtin_amdgcn_readfirstlane(s_idx);
-      if (n_idx < count) n_fr = items[n_idx];
+      if (n_idx < count) n_fr = uniform(n_idx < nparts ? R.heavy_parts[n_idx].fr : items[n_idx - nparts]);
       pst = 2;
     }
     if (pst < 3 && upto >= 3) {
-      if (n_idx < count) n_tix = R.blk_tile[n_fr >> 8];
+      n_skip = false;
+      if (n_idx < count) {
+        n_tix = uniform((int)R.blk_tile[n_fr >> 8]);
+        if (n_idx < nparts) {
+          const HeavyPart& x = R.heavy_parts[n_idx];
+          n_lo = uniform(x.lo);
+          n_hi = uniform(x.hi);
+          n_skip = n_lo >= n_hi || (NUM && (x.nnz == 0 || x.off < 0));
+        }
+      }
       pst = 3;
     }
     if (pst < 4 && upto >= 4) {
       if (n_idx < count) {
         const TileDev<T, RP>& t = R.tiles[n_tix];
         const int64_t ni = n_fr - t.flat0;
-        n_a0 = t.a_rp[ni];
-        n_a1 = t.a_rp[ni + 1];
-        if (NUM && tid == 0) {  // only this block reads or rewrites the row's slot
+        n_a0 = uniform(t.a_rp[ni]);
+        n_a1 = uniform(t.a_rp[ni + 1]);
+        if (n_idx < nparts) {
+          if (NUM) {
+            n_skip = n_skip || R.heavy_parts[R.heavy_first[n_fr]].bad;
+            n_off = R.heavy_parts[n_idx].off;
+            if (MODE == 1) {  // the row may hash now that its count is known, or not fit
+              n_off += R.off[n_fr];
+              n_skip = n_skip || bin_for(R.nnz[n_fr], R.prod[n_fr], R.tn, t.n) != kHeavyBin;
+              if (!n_skip && R.off[n_fr] + R.nnz[n_fr] > R.out_limit) {
+                if (tid == 0) R.stats[3] = 1ull;
+                n_skip = true;
+              }
+            }
+          }
+        } else if (NUM && tid == 0) {  // only this block reads or rewrites the row's slot
           n_cap = R.cap[n_fr];
           n_off = R.off[n_fr];
         }
@@ -1690,25 +2087,37 @@ __global__ __launch_bounds__(hr_block<MODE>()) void k_heavy_rank(RowsDev<T, RP> 
       if (n_idx < count && n_a1 - n_a0 <= (RP)BLOCK && tid < (int)(n_a1 - n_a0)) {
         const TileDev<T, RP>& t = R.tiles[n_tix];
         n_st = t.b_rp[n_kk];
-        n_len = t.b_rp[n_kk + 1] - n_st;
+        n_len = (int)(t.b_rp[n_kk + 1] - n_st);
       }
       pst = 6;
     }
   };
   if (tid == 0) nq = (int)atomicAdd(R.heavy_queue, 1ull);
-  advance(6);  // the first row: the whole chain, unhidden
+  advance(6);  // the first one: the whole chain, unhidden
   for (;;) {
     if (n_idx >= count) break;
-    const int fr = n_fr;
-    const TileDev<T, RP> tile = R.tiles[n_tix];
-    const int64_t i = fr - tile.flat0;
+    const bool part = n_idx < nparts, skip = uniform((int)n_skip) != 0;
+    const int idx = n_idx, fr = n_fr;
+    TileDev<T, RP> tile = R.tiles[n_tix];
+    tile.a_col = uniform(tile.a_col);
+    tile.a_val = uniform(tile.a_val);
+    tile.b_rp = uniform(tile.b_rp);
+    tile.b_col = uniform(tile.b_col);
+    tile.b_val = uniform(tile.b_val);
+    tile.c_col = uniform(tile.c_col);
+    tile.c_val = uniform(tile.c_val);
+    tile.n = uniform(tile.n);
     const int W = (tile.n + 31) / 32;
     const int Wr = (W + kHRGroup - 1) / kHRGroup * kHRGroup;  // whole groups (the tail words stay zero)
-    for (int w = tid; w < Wr; w += BLOCK) s_bits[w] = 0u;
+    const int lo = part ? n_lo : 0, hi = part ? n_hi : INT_MAX;
+    const int w0 = lo >> 5, w1 = part ? hi >> 5 : Wr;  // the words in use: a part's, whole groups, or all
+    if (!skip)
+      for (int w = w0 + tid; w < w1; w += BLOCK) s_bits[w] = 0u;
     const RP a0 = n_a0, a1 = n_a1;
     const int na = (int)(a1 - a0);
     const bool one_chunk = na <= BLOCK;  // one entry per thread, staged once and kept in registers
-    const RP my_st = n_st, my_len = n_len;
+    RP my_st = n_st;
+    int my_len = n_len;
     const T my_av = n_av;
     const int my_cap = n_cap;
     const long long my_off = n_off;
@@ -1718,97 +2127,112 @@ __global__ __launch_bounds__(hr_block<MODE>()) void k_heavy_rank(RowsDev<T, RP> 
     n_len = 0;
     n_av = T(0);
     do {
-      // stage (start, length) of every entry from registers and run the product loop
-      auto run_staged = [&](RP st, RP len, auto&& f, auto num_tag) {
-        constexpr bool kNum = decltype(num_tag)::value;
-        if (tid < na) {
-          s_est[tid] = st;
-          if (kNum) s_eval[tid] = my_av;
-        }
-        long long tot;
-        const long long ex = block_excl_scan<BLOCK, long long>((long long)(tid < na ? len : 0), &tot, s_lscan);
-        if (tid < na) s_epre[tid] = (int)ex;
-        if (tid == 0) s_epre[na] = (int)tot;
-        __syncthreads();
-        enumerate_staged<BLOCK, kNum, 4>(tile, na, tot, tid, s_est, s_epre, s_eval, nullptr, f);
-        __syncthreads();
-      };
       __syncthreads();
-      auto set_bit = [&](int j, double) { atomicOr(&s_bits[j >> 5], 1u << (j & 31)); };
-      if (one_chunk) run_staged(my_st, my_len, set_bit, std::false_type{});
-      else for_each_product<BLOCK, BLOCK, false, T, RP>(tile, a0, a1, tid, s_est, s_epre, s_eval, s_lscan, nullptr,
-                                                        set_bit);
+      if (skip) break;
+      bool bad = false;  // MODE 0, parts: a product outside the part's columns
+      // Stage (start, length, value) of the row's entries, one per thread and BLOCK at a time, and run the product loop.
+      // One chunk: st and len are the caller's. More: each chunk is loaded, and cut to the columns [c_lo, c_hi)
+      // of a part.
+      auto run_row = [&](RP st, int len, int c_lo, int c_hi, auto&& f, auto num_tag) {
+        constexpr bool kNum = decltype(num_tag)::value;
+        for (RP c0 = a0; c0 < a1; c0 += BLOCK) {
+          const int ne = (int)((a1 - c0) < (RP)BLOCK ? (a1 - c0) : (RP)BLOCK);
+          T av = my_av;
+          if (!one_chunk) {
+            st = 0;
+            len = 0;
+            if (tid < ne) {
+              const int kk = glob(tile.a_col)[c0 + tid];
+              st = glob(tile.b_rp)[kk];
+              const RP l = glob(tile.b_rp)[kk + 1] - st;
+              len = (int)l;
+              if (kNum) av = glob(tile.a_val)[c0 + tid];
+              if (part) {
+                RP x, y;
+                hr_column_range(tile.b_col, st, l, c_lo, c_hi, &x, &y);
+                bad = bad || y < x;
+                st += x;
+                len = y > x ? (int)(y - x) : 0;
+              }
+            }
+          }
+          int tot;
+          const int ex = block_scan_dpp<BLOCK>(tid < ne ? len : 0, &tot, s_scan[0]);
+          if (tid < ne) {
+            s_delta[tid] = st - (RP)ex;
+            s_pre[tid] = ex;
+            if constexpr (kNum) s_val[tid] = av;
+          }
+          __syncthreads();
+          enumerate_waves<BLOCK, kNum, sizeof(T) + sizeof(RP) == 8 ? 4 : 2>(tile, ne, tot, tid, s_delta, s_pre, s_val, f);
+          __syncthreads();
+        }
+      };
+      if (part && one_chunk && tid < na) {  // the entry's share of its B row
+        RP x, y;
+        hr_column_range(tile.b_col, my_st, (RP)my_len, lo, hi, &x, &y);
+        bad = y < x;
+        my_st += x;
+        my_len = y > x ? (int)(y - x) : 0;
+      }
+      auto set_bit = [&](int j, T, T) {
+        atomicOr(&s_bits[j >> 5], 1u << (j & 31));
+        if (MODE == 0 && part) bad = bad || (unsigned)(j - lo) >= (unsigned)(hi - lo);
+      };
+      run_row(my_st, my_len, lo, hi, set_bit, std::false_type{});
+      if (MODE == 0 && part && bad) R.heavy_parts[R.heavy_first[fr]].bad = 1;
       advance(1);
       __syncthreads();
       advance(2);
-      // group prefixes, in order: thread t counts groups [t * kGroupsPerThread, (t + 1) * kGroupsPerThread)
-      const int ng = Wr / kHRGroup;
-      int gc[kGroupsPerThread];
-      long long c = 0;
-#pragma unroll
-      for (int q = 0; q < kGroupsPerThread; q++) {
-        const int g = tid * kGroupsPerThread + q;
-        int n1 = 0;
-        if (g < ng) {
-          const u32x4_t* p4 = reinterpret_cast<const u32x4_t*>(s_bits + g * kHRGroup);
-#pragma unroll
-          for (int v = 0; v < kHRGroup / 4; v++) {
-            const u32x4_t x = p4[v];
-            n1 += __popc(x.x) + __popc(x.y) + __popc(x.z) + __popc(x.w);
-          }
-        }
-        gc[q] = n1;
+      // group prefixes, in order: thread t counts `per` groups from g0 + t * per
+      const int g0 = w0 / kHRGroup, g1 = w1 / kHRGroup;
+      const int per = (g1 - g0 + BLOCK - 1) / BLOCK;
+      int c = 0;
+      for (int g = g0 + tid * per; g < min(g1, g0 + (tid + 1) * per); g++) {
+        const u32x4_t x = *reinterpret_cast<const u32x4_t*>(s_bits + g * kHRGroup);
+        const int n1 = __popc(x.x) + __popc(x.y) + __popc(x.z) + __popc(x.w);
+        if (NUM) s_gpre[g] = n1;
         c += n1;
       }
-      long long total;
-      long long run = block_excl_scan<BLOCK, long long>(c, &total, s_scan);
+      int total;
+      int run = block_scan_dpp<BLOCK>(c, &total, s_scan[1]);
       advance(3);
-      const int run0 = (int)run;
-#pragma unroll
-      for (int q = 0; q < kGroupsPerThread; q++) {
-        const int g = tid * kGroupsPerThread + q;
-        if (NUM && g < ng) s_gpre[g] = (int)run;
-        run += gc[q];
-      }
-      // A row whose columns fit one slice (most heavy rows) stages them here, by rank, from the words this thread
-      // just counted: no separate pass over the bitmap and no column search.
-      if (NUM && total <= (long long)kHRSlice) {
-        int r = run0;
-        for (int w = tid * kGroupsPerThread * kHRGroup; w < (tid + 1) * kGroupsPerThread * kHRGroup && w < Wr; w++) {
-          unsigned m = s_bits[w];
-          while (m) {
-            s_colbuf[r++] = w * 32 + (__ffs(m) - 1);
-            m &= m - 1;
-          }
-        }
-      }
       if (MODE == 0) {
         if (tid == 0) {
-          R.nnz[fr] = (int)total;
-          atomicAdd(&R.stats[1], 1ull);
+          if (part) {
+            R.heavy_parts[idx].nnz = total;
+          } else {
+            R.nnz[fr] = total;
+            atomicAdd(&R.stats[1], 1ull);
+          }
         }
         __syncthreads();
         break;
       }
+      for (int g = g0 + tid * per; g < min(g1, g0 + (tid + 1) * per); g++) {
+        const int n1 = s_gpre[g];
+        s_gpre[g] = run;
+        run += n1;
+      }
       if (tid == 0) {
-        long long b;
-        if (MODE == 1 || (MODE == 2 && total <= (long long)my_cap)) {
-          b = my_off;
-        } else {
-          b = (long long)atomicAdd(R.cursor, (unsigned long long)total);
-          R.off[fr] = b;
-        }
-        if (b + total > R.out_limit) {  // refused: nothing is written and, after this pass, the row holds 0 entries
-          R.stats[3] = 1ull;
-          b = -1;
-          if (MODE != 1) R.off[fr] = 0;
+        long long b = my_off;
+        if (!part) {
+          if (!(MODE == 1 || (MODE == 2 && total <= my_cap))) {
+            b = (long long)atomicAdd(R.cursor, (unsigned long long)total);
+            R.off[fr] = b;
+          }
+          if (b + total > R.out_limit) {  // refused: nothing is written and, after this pass, the row holds 0 entries
+            R.stats[3] = 1ull;
+            b = -1;
+            if (MODE != 1) R.off[fr] = 0;
+          }
+          R.nnz[fr] = (b < 0 && MODE != 1) ? 0 : total;
+          atomicAdd(&R.stats[1], 1ull);
         }
         s_base = b;
-        R.nnz[fr] = (b < 0 && MODE != 1) ? 0 : (int)total;
-        atomicAdd(&R.stats[1], 1ull);
       }
       __syncthreads();
-      const long long base = s_base;
+      const long long base = uniform(s_base);
       advance(4);
       if (base < 0) {  // refused: nothing is written
         __syncthreads();
@@ -1817,26 +2241,27 @@ __global__ __launch_bounds__(hr_block<MODE>()) void k_heavy_rank(RowsDev<T, RP> 
       // one rank slice at a time: columns (staged in LDS by rank, then stored with unit stride), then values. A
       // slice's first column and each entry's first B position in it are where the previous slice ended.
       RP my_lo = 0;
-      for (long long s0 = 0; s0 < total; s0 += kHRSlice) {
-        const int len = (int)(total - s0 < kHRSlice ? total - s0 : kHRSlice);
-        const bool whole = s0 == 0 && len == total;  // the columns are staged already (above)
-        int c_lo = 0, c_hi = INT_MAX;
+      for (int s0 = 0; s0 < total; s0 += kHRSlice) {
+        const int len = total - s0 < kHRSlice ? total - s0 : kHRSlice;
+        const bool whole = s0 == 0 && len == total;
+        int c_lo = lo, c_hi = hi;
         if (!whole) {
           if (tid == 0) {  // column range of the slice
-            s_crange[0] = s0 == 0 ? 0 : s_crange[1];
-            s_crange[1] = s0 + len >= total ? INT_MAX : hr_select(s_bits, s_gpre, ng, (int)(s0 + len));
+            s_crange[0] = s0 == 0 ? lo : s_crange[1];
+            s_crange[1] = s0 + len >= total ? hi : hr_select(s_bits, s_gpre, g0, g1, s0 + len);
           }
           __syncthreads();
-          c_lo = s_crange[0];
-          c_hi = s_crange[1];
+          c_lo = uniform(s_crange[0]);
+          c_hi = uniform(s_crange[1]);
         }
         const int w_lo = c_lo >> 5, w_hi = c_hi == INT_MAX ? W - 1 : (c_hi - 1) >> 5;
         // a wavefront takes 64 consecutive words (whole groups) at a time: each word's rank base is its group prefix
-        // plus the bits of the group's earlier words (a kHRGroup-lane scan of popcounts)
-        if (!whole)
+        // plus the bits of the group's earlier words (a kHRGroup-lane scan of popcounts). A lane per word keeps
+        // the lanes of a wavefront alike; 16 words per thread left one wavefront with all of a skewed row's dense words
+        // (20700 of 130000 cycles per row of an R-MAT square at scale 16).
         for (int wb = (w_lo & ~63) + (tid & ~63); wb <= w_hi; wb += BLOCK) {
           const int lane = tid & 63, w = wb + lane;
-          const unsigned full = w < W ? s_bits[w] : 0u;
+          const unsigned full = w >= w0 && w < w1 && w < W ? s_bits[w] : 0u;
           const int pc = __popc(full);
           int inc = pc;
 #pragma unroll
@@ -1848,43 +2273,38 @@ __global__ __launch_bounds__(hr_block<MODE>()) void k_heavy_rank(RowsDev<T, RP> 
           if (w == w_lo) m &= ~((1u << (c_lo & 31)) - 1u);
           if (c_hi != INT_MAX && w == (c_hi >> 5)) m &= (1u << (c_hi & 31)) - 1u;
           if (m) {
-            const int r0 = s_gpre[w / kHRGroup] + inc - pc - (int)s0;
+            int r = s_gpre[w / kHRGroup] + inc - pc - s0 + __popc(full & ((m & (0u - m)) - 1u));
             while (m) {
-              const int b = __ffs(m) - 1;
-              s_colbuf[r0 + __popc(full & ((1u << b) - 1u))] = w * 32 + b;
+              s_colbuf[r++] = w * 32 + (__ffs(m) - 1);
               m &= m - 1;
             }
           }
         }
         __syncthreads();
         if (s0 == 0) advance(5);
-        for (int t = tid; t < len; t += BLOCK) __builtin_nontemporal_store(s_colbuf[t], &tile.c_col[base + s0 + t]);
+        for (int t = tid; t < len; t += BLOCK) __builtin_nontemporal_store(s_colbuf[t], &glob(tile.c_col)[base + s0 + t]);
         __syncthreads();
         for (int t = tid; t < len; t += BLOCK) s_acc[t] = 0.0;
-        __syncthreads();
         if (s0 == 0) advance(6);
-        auto add = [&](int j, double v) {
-          if (whole || (j >= c_lo && j < c_hi)) atomicAdd(&s_acc[hr_rank(s_bits, s_gpre, j) - (int)s0], v);
+        auto add = [&](int j, T a, T b) {
+          if (whole || (j >= c_lo && j < c_hi))
+            atomicAdd(&s_acc[hr_rank(s_bits, s_gpre, j) - s0], (double)a * (double)b);
         };
-        if (one_chunk) {
-          RP st = my_st, ln = my_len;
-          if (!whole && tid < na) {  // the part of the entry's B row inside the slice's columns
-            const RP lo = my_lo;
-            const RP hi = c_hi == INT_MAX ? my_len : hr_lower_bound(tile.b_col, my_st, lo, my_len, c_hi);
-            st = my_st + lo;
-            ln = hi - lo;
-            my_lo = hi;
-          }
-          run_staged(st, ln, add, std::true_type{});
-        } else {
-          for_each_product<BLOCK, BLOCK, true, T, RP>(tile, a0, a1, tid, s_est, s_epre, s_eval, s_lscan, nullptr, add);
-          __syncthreads();
+        RP st = my_st;
+        int ln = my_len;
+        if (one_chunk && !whole && tid < na) {  // the part of the entry's B row inside the slice's columns
+          const RP x = my_lo;
+          const RP y = s0 + len >= total ? (RP)my_len : hr_lower_bound(tile.b_col, my_st, x, (RP)my_len, c_hi);
+          st = my_st + x;
+          ln = (int)(y - x);
+          my_lo = y;
         }
-        for (int t = tid; t < len; t += BLOCK) __builtin_nontemporal_store((T)s_acc[t], &tile.c_val[base + s0 + t]);
+        run_row(st, ln, c_lo, c_hi, add, std::true_type{});
+        for (int t = tid; t < len; t += BLOCK) __builtin_nontemporal_store((T)s_acc[t], &glob(tile.c_val)[base + s0 + t]);
         __syncthreads();
       }
     } while (false);
-    advance(6);  // rows that ended early (symbolic, refused) finish the next row's fetch here
+    advance(6);  // rows that ended early (symbolic, refused, skipped) finish the next row's fetch here
   }
 }
 

@@ -245,9 +245,11 @@ struct StagePlan : StageBase {
       if (counts[b] > 0) launched |= 1u << b;
     hipLaunchKernelGGL(k_check_bins, dim3(1), dim3(64), 0, s, (const int32_t*)F.R.bin_count, launched, F.R.stats + 3);
     BCLX_HIP(hipGetLastError());
+    if (counts[kHeavyBin] > 0) F.plan_heavy(s, mode_k);
     fork(s);
     int q = 0;
-    if (counts[kHeavyBin] > 0) F.run_bin(side[q++ % side.size()], mode_k, kHeavyBin, persistent ? -1 : counts[kHeavyBin]);
+    if (counts[kHeavyBin] > 0)
+      F.run_bin(side[q++ % side.size()], mode_k, kHeavyBin, persistent ? -1 : counts[kHeavyBin], true);
     for (int b = kEscBin0 + kEscBins - 1; b >= kEscBin0; b--) {
       if (counts[b] == 0) continue;
       F.run_bin(side[q++ % side.size()], mode_k, b, counts[b]);
