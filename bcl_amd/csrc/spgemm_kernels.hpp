@@ -828,10 +828,11 @@ __global__ __launch_bounds__(BLOCK) void k_hash(RowsDev<T, RP> R, int bin) {
 // Rows of a SUMMA-stage tile product are mostly output-dense (nnz(C_i) close to the products), where a hash table
 // costs two LDS slots per output entry plus a rank structure, and caps how many rows a CU holds. Here the products
 // of a row are expanded into registers as 32-bit keys (column << 13 | product index), sorted with a bitonic network
-// across the wavefront (registers and lane shuffles), and equal columns are summed in product order (the reference's
-// A-row order, in float64, rounded once). LDS holds only the float64 products (8 bytes per product) and the sorted
-// columns. The count is exact after the sort, so the predicted mode never overflows: a row that outgrows its slot
+// across the wavefront, and equal columns are summed in float64 in a fixed order and rounded once. LDS holds only the float64 products (8 bytes per product) and the sorted
+// keys. The count is exact after the sort, so the predicted mode never overflows: a row that outgrows its slot
 // is bump-allocated in the same pass.
+// Bound by VALU instructions (92 % busy in the kernel of 2048 to 4096 products before the sort kept neighbouring
+// positions in a lane).
 //   MODE 0 symbolic -> nnz[fr]; MODE 1 numeric at off[fr]; MODE 2 at off[fr] when nnz <= cap[fr], else
 //   bump-allocated; MODE 3 bump-allocated.
 // ------------------------------------------------------------------------------------------------------------
@@ -842,266 +843,12 @@ constexpr unsigned kEscKeyShift = 32 - kEscColBits;      // key = column << 13 |
 constexpr unsigned kEscIdxMask = (1u << kEscKeyShift) - 1u;
 constexpr unsigned kEscPad = 0xffffffffu;                 // sorts after every real key
 
-// Does sorted position k * 64 + lane start an output entry (a real key whose column differs from its
-// predecessor's)? Position 0 always does: the pad key's column field equals the largest column.
-template <int K>
-__device__ inline bool esc_head(const unsigned (&key)[K], int k, int lane) {
-  const unsigned up = (unsigned)__shfl_up((int)key[k], 1, 64);
-  const unsigned wrap = k > 0 ? (unsigned)__shfl((int)key[k > 0 ? k - 1 : 0], 63, 64) : kEscPad;
-  const unsigned prev = lane == 0 ? wrap : up;
-  return key[k] != kEscPad && ((k == 0 && lane == 0) || (prev >> kEscKeyShift) != (key[k] >> kEscKeyShift));
-}
-
-// For the K products x = x0 + k * 64 + lane of a wavefront, the staged entry e holding product t = x - base
-// (pre[e] <= t < pre[e + 1], pre has ne + 1 prefix counts): K branchless binary searches in lockstep. Products outside
-// the chunk get some valid e (the caller skips them).
-template <int K>
-__device__ inline void esc_lookup(const int* pre, int ne, int base, int lane, int x0, int (&lo)[K]) {
-  int top = 1;  // largest power of two < ne (0 when ne == 1)
-  while (top < ne) top <<= 1;
-  top >>= 1;
-#pragma unroll
-  for (int k = 0; k < K; k++) lo[k] = 0;
-  for (int step = top; step > 0; step >>= 1) {
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-      const int c = lo[k] + step;
-      if (c < ne && pre[c] <= x0 + k * 64 + lane - base) lo[k] = c;
-    }
-  }
-}
-
-// Compare-exchange of one bitonic stage whose partner is `d` lanes away (d < 64): keep min or max of the pair.
-// Value of lane (lane ^ D) of a wavefront. Distances 1, 2 and 8 are one DPP move (quad_perm [1,0,3,2], quad_perm
-// [2,3,0,1], row_ror:8), 4 is two DPP moves (row_shl:4 for lanes with bit 2 clear, row_shr:4 for the others), 16 is
-// a ds_swizzle in xor mode (within 32 lanes), 32 a bpermute.
-template <int D>
-__device__ inline unsigned lane_xor(unsigned v, int lane) {
-  const int x = (int)v;
-  if constexpr (D == 1) return (unsigned)__builtin_amdgcn_update_dpp(0, x, 0xB1, 0xF, 0xF, false);
-  else if constexpr (D == 2) return (unsigned)__builtin_amdgcn_update_dpp(0, x, 0x4E, 0xF, 0xF, false);
-  else if constexpr (D == 4) {
-    const int up = __builtin_amdgcn_update_dpp(0, x, 0x104, 0xF, 0xF, false);  // lane + 4
-    const int dn = __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false);  // lane - 4
-    return (unsigned)((lane & 4) ? dn : up);
-  } else if constexpr (D == 8) return (unsigned)__builtin_amdgcn_update_dpp(0, x, 0x128, 0xF, 0xF, false);
-  else if constexpr (D == 16) return (unsigned)__builtin_amdgcn_ds_swizzle(x, 0x401F);
-  else return (unsigned)__shfl_xor(x, D, 64);
-}
-
-template <int D>
-__device__ inline unsigned esc_xchg(unsigned v, bool keep_min, int lane) {
-  const unsigned o = lane_xor<D>(v, lane);
-  return keep_min ? min(v, o) : max(v, o);
-}
-
-// Bitonic sort, ascending, of the 64 * K keys of a wavefront; element e = k * 64 + lane lives in key[k].
-template <int K>
-__device__ inline void esc_sort(unsigned (&key)[K], int lane) {
-#pragma unroll
-  for (int size = 2; size <= 64 * K; size <<= 1) {
-#pragma unroll
-    for (int d = size >> 1; d > 0; d >>= 1) {
-      if (d >= 64) {
-        const int dk = d >> 6;
-#pragma unroll
-        for (int k = 0; k < K; k++) {
-          if ((k & dk) == 0) {
-            const bool asc = ((k * 64) & size) == 0;
-            const unsigned a = key[k], b = key[k | dk];
-            const bool sw = (a > b) == asc;
-            key[k] = sw ? b : a;
-            key[k | dk] = sw ? a : b;
-          }
-        }
-      } else {
-#pragma unroll
-        for (int k = 0; k < K; k++) {
-          const bool asc = (((k * 64) | lane) & size) == 0;
-          const bool lower = (lane & d) == 0;
-          const bool keep_min = asc == lower;
-          switch (d) {
-            case 1: key[k] = esc_xchg<1>(key[k], keep_min, lane); break;
-            case 2: key[k] = esc_xchg<2>(key[k], keep_min, lane); break;
-            case 4: key[k] = esc_xchg<4>(key[k], keep_min, lane); break;
-            case 8: key[k] = esc_xchg<8>(key[k], keep_min, lane); break;
-            case 16: key[k] = esc_xchg<16>(key[k], keep_min, lane); break;
-            default: key[k] = esc_xchg<32>(key[k], keep_min, lane); break;
-          }
-        }
-      }
-    }
-  }
-}
-
-// Half-cleaner stages at distances 32 * K .. 1 (ascending) over one wavefront's 64 * K keys, which merge a bitonic
-// sequence into sorted order: in-register stages for distances of 64 or more, lane exchanges below.
-template <int K>
-__device__ inline void esc_half_clean(unsigned (&key)[K], int lane) {
-#pragma unroll
-  for (int d = 32 * K; d > 0; d >>= 1) {
-    if (d >= 64) {
-      const int dk = d >> 6;
-#pragma unroll
-      for (int k = 0; k < K; k++) {
-        if ((k & dk) == 0) {
-          const unsigned a = key[k], b = key[k | dk];
-          key[k] = min(a, b);
-          key[k | dk] = max(a, b);
-        }
-      }
-    } else {
-      const bool keep_min = (lane & d) == 0;
-#pragma unroll
-      for (int k = 0; k < K; k++) {
-        switch (d) {
-          case 1: key[k] = esc_xchg<1>(key[k], keep_min, lane); break;
-          case 2: key[k] = esc_xchg<2>(key[k], keep_min, lane); break;
-          case 4: key[k] = esc_xchg<4>(key[k], keep_min, lane); break;
-          case 8: key[k] = esc_xchg<8>(key[k], keep_min, lane); break;
-          case 16: key[k] = esc_xchg<16>(key[k], keep_min, lane); break;
-          default: key[k] = esc_xchg<32>(key[k], keep_min, lane); break;
-        }
-      }
-    }
-  }
-}
-
-template <int K, int MODE, typename T, typename RP>
-__global__ __launch_bounds__(64 * kEscWaves) void k_esc(RowsDev<T, RP> R, int bin) {
-  constexpr int N = 64 * K;
-  constexpr bool NUM = MODE != 0;
-  __shared__ double s_val[kEscWaves][NUM ? N : 1];  // float64 products by product index
-  __shared__ unsigned s_key[kEscWaves][NUM ? N : 1];  // sorted keys
-  __shared__ int s_pre[kEscWaves][65];              // per chunk of A entries: products before each entry
-  __shared__ RP s_st[kEscWaves][64];                // B-row start of each entry
-  __shared__ T s_av[kEscWaves][64];                 // A value of each entry
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int count = *R.count_of(bin);
-  const int* items = R.bin_items + (int64_t)bin * R.bin_stride;
-  for (int idx = blockIdx.x * kEscWaves + w; idx < count; idx += gridDim.x * kEscWaves) {
-    const int fr = items[idx];
-    const TileDev<T, RP> tile = R.tiles[R.blk_tile[fr >> 8]];
-    const int64_t i = fr - tile.flat0;
-    const RP a0 = tile.a_rp[i], a1 = tile.a_rp[i + 1];
-    unsigned key[K];
-#pragma unroll
-    for (int k = 0; k < K; k++) key[k] = kEscPad;
-    // expand: product x (A-row order) -> key (column << 13 | x), float64 product -> s_val[x]
-    int base = 0;
-    for (RP c0 = a0; c0 < a1; c0 += 64) {
-      const int ne = (int)((a1 - c0) < (RP)64 ? (a1 - c0) : (RP)64);
-      int len = 0;
-      if (lane < ne) {
-        const int kk = tile.a_col[c0 + lane];
-        const RP st = tile.b_rp[kk];
-        len = (int)(tile.b_rp[kk + 1] - st);
-        s_st[w][lane] = st;
-        if (NUM) s_av[w][lane] = tile.a_val[c0 + lane];
-      }
-      int inc = len;
-#pragma unroll
-      for (int d = 1; d < 64; d <<= 1) {
-        const int t = __shfl_up(inc, d, 64);
-        if (lane >= d) inc += t;
-      }
-      const int total = __shfl(inc, 63, 64);
-      if (lane < ne) s_pre[w][lane] = inc - len;
-      if (lane == 0) s_pre[w][ne] = total;
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      int lo[K];  // entry e with s_pre[e] <= t < s_pre[e + 1], all K lookups in lockstep
-      esc_lookup<K>(s_pre[w], ne, base, lane, 0, lo);
-#pragma unroll
-      for (int k = 0; k < K; k++) {
-        const int x = k * 64 + lane;
-        const int t = x - base;
-        if (t >= 0 && t < total) {
-          const RP q = s_st[w][lo[k]] + (RP)(t - s_pre[w][lo[k]]);
-          key[k] = ((unsigned)tile.b_col[q] << kEscKeyShift) | (unsigned)x;
-          if (NUM) s_val[w][x] = (double)s_av[w][lo[k]] * (double)tile.b_val[q];
-        }
-      }
-      base += total;
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
-    esc_sort<K>(key, lane);
-    // compress: a sorted position starts an output entry when its column differs from the previous position's
-    int cnt = 0;
-#pragma unroll
-    for (int k = 0; k < K; k++) cnt += __popcll(__ballot(esc_head<K>(key, k, lane)));
-    if (MODE == 0) {
-      if (lane == 0) R.nnz[fr] = cnt;
-      continue;
-    }
-    long long o = 0;
-    if (lane == 0) {
-      if (MODE == 1 || (MODE == 2 && cnt <= R.cap[fr])) {
-        o = R.off[fr];
-      } else {
-        o = (long long)atomicAdd(R.cursor, (unsigned long long)cnt);
-        R.off[fr] = o;
-      }
-      if (o + cnt > R.out_limit) {  // refused: nothing is written and, after this pass, the row holds 0 entries
-        R.stats[3] = 1ull;
-        o = -1;
-        if (MODE != 1) R.off[fr] = 0;
-      }
-      R.nnz[fr] = (o < 0 && MODE != 1) ? 0 : cnt;
-    }
-    o = __shfl(o, 0, 64);
-#pragma unroll
-    for (int k = 0; k < K; k++) s_key[w][k * 64 + lane] = key[k];
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    if (o >= 0) {
-      int before = 0;
-#pragma unroll
-      for (int k = 0; k < K; k++) {
-        const bool head = esc_head<K>(key, k, lane);
-        const unsigned long long mask = __ballot(head);
-        if (head) {
-          // sum the run of equal columns in sorted order, i.e. in product (A-row) order
-          const unsigned col = key[k] >> kEscKeyShift;
-          double sum = s_val[w][key[k] & kEscIdxMask];
-          for (int p = k * 64 + lane + 1; p < N; p++) {
-            const unsigned kp = s_key[w][p];
-            if (kp == kEscPad || (kp >> kEscKeyShift) != col) break;
-            sum += s_val[w][kp & kEscIdxMask];
-          }
-          const long long pos = o + before + __popcll(mask & ((1ull << lane) - 1ull));
-          __builtin_nontemporal_store((int)col, &tile.c_col[pos]);
-          __builtin_nontemporal_store((T)sum, &tile.c_val[pos]);
-        }
-        before += __popcll(mask);
-      }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  }
-}
-
-// ------------------------------------------------------------------------------------------------------------
-// Rows of at most 32 (64) products, 8 (16) lanes each. The products are expanded four per lane as 32-bit keys (column
-// << 5 (6) | product index), sorted in registers (DPP exchanges: no LDS, no barrier), and equal columns are summed in
-// product (A-row) order, in float64, rounded once.
-// A hash row of this size costs a table clear, LDS atomics and a sort of its table in LDS; a one-wavefront ESC row
-// leaves half the lanes idle. Tiles up to 2^27 - 2 columns wide. Modes as in k_esc.
-// ------------------------------------------------------------------------------------------------------------
-
-constexpr int kSmallWaves = 4;  // wavefronts per block
-
 // A value moved between the lanes of a 16-lane DPP row, one VALU move (part of the using instruction where that allows
-// it): from lane ^ X (X = 1, 2, 3, 7 or 15), or from the lane D below (above); lanes without one get 0.
+// it): from lane ^ X (X = 1, 2, 3, 7, 8 or 15), or from the lane D below (above); lanes without one get 0.
 template <int X>
 __device__ inline unsigned dpp_xor(unsigned v) {
-  constexpr int ctrl = X == 1 ? 0xB1 : X == 2 ? 0x4E : X == 3 ? 0x1B : X == 7 ? 0x141 : 0x140;
-  static_assert(X == 1 || X == 2 || X == 3 || X == 7 || X == 15, "a quad permutation or a mirror");
+  constexpr int ctrl = X == 1 ? 0xB1 : X == 2 ? 0x4E : X == 3 ? 0x1B : X == 7 ? 0x141 : X == 8 ? 0x128 : 0x140;
+  static_assert(X == 1 || X == 2 || X == 3 || X == 7 || X == 8 || X == 15, "a quad permutation, a mirror or a rotation");
   return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, 0xF, 0xF, true);
 }
 template <int D>
@@ -1123,6 +870,401 @@ __device__ inline void cx(unsigned& a, unsigned& b) {
   b = max(a, b);
   a = lo;
 }
+
+// Compare-exchange of a wavefront's keys with lane ^ 16 or lane ^ 32 (half-cleaner: the lower lane keeps the minimum), two
+// slots at a time: swapping half of one with half of the other brings both keys of each pair into one lane, and swapping
+// again takes them home. Two instructions per key, none of them LDS.
+template <int X, int K>
+__device__ inline void swap_step(unsigned (&key)[K]) {
+  static_assert(X == 16 || X == 32, "the distances of the swap instructions");
+  auto swap = [](unsigned& a, unsigned& b) {
+    if constexpr (X == 16) {
+      const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+      a = r[0];
+      b = r[1];
+    } else {
+      const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+      a = r[0];
+      b = r[1];
+    }
+  };
+#pragma unroll
+  for (int q = 0; q < K; q += 2) {
+    swap(key[q], key[q + 1]);
+    cx(key[q], key[q + 1]);
+    swap(key[q], key[q + 1]);
+  }
+}
+
+// Half-cleaner at distance X lanes inside a 16-lane row; lim is ~0 in the upper lane of each pair.
+template <int X, int K>
+__device__ inline void dpp_step(unsigned (&key)[K], unsigned lim) {
+#pragma unroll
+  for (int q = 0; q < K; q++) {
+    // lane ^ 4 is the mirror of eight, then of four
+    const unsigned o = X == 4 ? dpp_xor<3>(dpp_xor<7>(key[q])) : dpp_xor<X == 4 ? 1 : X>(key[q]);
+    key[q] = min_or_max(key[q], o, lim);
+  }
+}
+
+// The same against the mirrored position (lane ^ X, slot K - 1 - q), the first stage of a merge of two ascending runs.
+template <int X, int K>
+__device__ inline void mirror_step(unsigned (&key)[K], unsigned lim) {
+  unsigned o[K];
+#pragma unroll
+  for (int q = 0; q < K; q++) o[q] = dpp_xor<X>(key[K - 1 - q]);
+#pragma unroll
+  for (int q = 0; q < K; q++) key[q] = min_or_max(key[q], o[q], lim);
+}
+
+template <int K>
+__device__ inline void lane_merge(unsigned (&key)[K]) {
+#pragma unroll
+  for (int d = K / 2; d > 0; d >>= 1)
+#pragma unroll
+    for (int q = 0; q < K; q++)
+      if ((q & d) == 0) cx(key[q], key[q + d]);
+}
+
+template <int K>
+__device__ inline void lane_sort(unsigned (&key)[K]) {
+  static_assert(K == 2 || K == 4 || K == 8, "slots per lane");
+  if constexpr (K == 2) {
+    cx(key[0], key[1]);
+  } else {
+#pragma unroll
+    for (int q = 0; q < K; q += 4) {
+      cx(key[q], key[q + 1]);
+      cx(key[q + 2], key[q + 3]);
+      cx(key[q], key[q + 2]);
+      cx(key[q + 1], key[q + 3]);
+      cx(key[q + 1], key[q + 2]);
+    }
+    if constexpr (K == 8) {  // odd-even merge of the two halves
+      cx(key[0], key[4]);
+      cx(key[1], key[5]);
+      cx(key[2], key[6]);
+      cx(key[3], key[7]);
+      cx(key[2], key[4]);
+      cx(key[3], key[5]);
+      cx(key[1], key[2]);
+      cx(key[3], key[4]);
+      cx(key[5], key[6]);
+    }
+  }
+}
+
+// Masks of the lanes that keep the maximum at each distance.
+struct LaneLimits {
+  unsigned l1, l2, l4, l8;
+  __device__ explicit LaneLimits(int lane)
+      : l1(lane & 1 ? ~0u : 0u), l2(lane & 2 ? ~0u : 0u), l4(lane & 4 ? ~0u : 0u), l8(lane & 8 ? ~0u : 0u) {}
+};
+
+// Sorts a bitonic sequence of the 64 * K keys of a wavefront: position x is slot x % K of lane x / K.
+template <int K>
+__device__ inline void esc_half_clean(unsigned (&key)[K], const LaneLimits& m) {
+  swap_step<32>(key);
+  swap_step<16>(key);
+  dpp_step<8>(key, m.l8);
+  dpp_step<4>(key, m.l4);
+  dpp_step<2>(key, m.l2);
+  dpp_step<1>(key, m.l1);
+  lane_merge(key);
+}
+
+// Ascending sort of the 64 * K keys of a wavefront: in, any order; out, position x is slot x % K of lane x / K. Bitonic;
+// K neighbours per lane leave 21 of the 45 stages of 512 keys crossing lanes (positions spread over the lanes: 39, in
+// LDS exchanges for two of the six distances): 71 instructions per key instead of about 185. Runs up to 16 lanes merge by
+// the mirrored position; the odd rows are reversed before runs of 16 lanes merge, and the upper 32 lanes sort
+// complemented keys, i.e. descending.
+template <int K>
+__device__ inline void esc_sort(unsigned (&key)[K], int lane, const LaneLimits& m) {
+  const unsigned flip = lane & 32 ? ~0u : 0u;
+#pragma unroll
+  for (int q = 0; q < K; q++) key[q] ^= flip;
+  lane_sort(key);
+  mirror_step<1>(key, m.l1);
+  lane_merge(key);
+  mirror_step<3>(key, m.l2);
+  dpp_step<1>(key, m.l1);
+  lane_merge(key);
+  mirror_step<7>(key, m.l4);
+  dpp_step<2>(key, m.l2);
+  dpp_step<1>(key, m.l1);
+  lane_merge(key);
+  mirror_step<15>(key, m.l8);
+  dpp_step<4>(key, m.l4);
+  dpp_step<2>(key, m.l2);
+  dpp_step<1>(key, m.l1);
+  lane_merge(key);
+  unsigned o[K];
+#pragma unroll
+  for (int q = 0; q < K; q++) o[q] = key[K - 1 - q];
+#pragma unroll
+  for (int q = 0; q < K; q++)  // row_mirror in rows 1 and 3
+    key[q] = (unsigned)__builtin_amdgcn_update_dpp((int)key[q], (int)o[q], 0x140, 0xA, 0xF, false);
+  swap_step<16>(key);
+  dpp_step<8>(key, m.l8);
+  dpp_step<4>(key, m.l4);
+  dpp_step<2>(key, m.l2);
+  dpp_step<1>(key, m.l1);
+  lane_merge(key);
+#pragma unroll
+  for (int q = 0; q < K; q++) key[q] ^= flip;
+  esc_half_clean(key, m);
+}
+
+// Expands a wavefront's share of a row's products, x0 + q * 64 + lane in A-row order, into keys (column << 13 | x), with the
+// float64 products in s_val[x]; slots past the row's products keep the pad key. 64 A entries at a time, one per lane. For
+// each 64 products the entries that start among them are counted by a ballot: up to eight are broadcast and compared per lane,
+// more are searched (a binary search per product took a third of the instructions the sort takes). Every wavefront of a row
+// walks the row's entries itself.
+template <int K, bool NUM, typename T, typename RP>
+__device__ inline void esc_expand(const TileDev<T, RP>& tile, RP a0, RP a1, int x0, int lane, unsigned (&key)[K],
+                                  double* s_val) {
+#pragma unroll
+  for (int q = 0; q < K; q++) key[q] = kEscPad;
+  int base = 0;
+  for (RP c0 = a0; c0 < a1 && base < x0 + 64 * K; c0 += 64) {
+    RP st = 0;
+    int len = 0;
+    T av = T(0);
+    if (c0 + lane < a1) {
+      const int kk = glob(tile.a_col)[c0 + lane];
+      st = glob(tile.b_rp)[kk];
+      len = (int)(glob(tile.b_rp)[kk + 1] - st);
+      if (NUM) av = glob(tile.a_val)[c0 + lane];
+    }
+    const int inc = wave_scan_dpp(len);
+    const int total = __builtin_amdgcn_readlane(inc, 63);
+    const int ex = inc - len;  // lanes past the row start at `total`: after every product
+    const RP delta = st - (RP)ex;
+    RP pos[K];
+    T a[K];
+#pragma unroll
+    for (int q = 0; q < K; q++) {
+      const int t0 = x0 + q * 64 - base, t = t0 + lane;  // products t of this chunk
+      pos[q] = 0;
+      a[q] = T(0);
+      if (t0 + 63 >= 0 && t0 < total) {  // uniform
+        const int before = __popcll(__ballot(ex <= t0));
+        const int in = __popcll(__ballot(ex <= t0 + 63)) - before;
+        int e = before - 1;  // the last entry that starts at or before t
+        if (in <= 8) {
+          for (int i = 0; i < in; i++) e += __builtin_amdgcn_readlane(ex, before + i) <= t ? 1 : 0;
+        } else {
+          e = 0;
+#pragma unroll
+          for (int step = 32; step > 0; step >>= 1)
+            if (__shfl(ex, e + step, 64) <= t) e += step;
+        }
+        e = e < 0 ? 0 : e;
+        pos[q] = (RP)__shfl(delta, e, 64) + (RP)t;
+        if (NUM) a[q] = __shfl(av, e, 64);
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < K; q++) {
+      const int x = x0 + q * 64 + lane, t = x - base;
+      if (t >= 0 && t < total) {
+        key[q] = ((unsigned)glob(tile.b_col)[pos[q]] << kEscKeyShift) | (unsigned)x;
+        if (NUM) s_val[x] = (double)a[q] * (double)glob(tile.b_val)[pos[q]];
+      }
+    }
+    base += total;
+  }
+}
+
+// What the wavefronts of a row (W of them) tell each other when it is compressed.
+template <int W>
+struct EscShare {
+  unsigned last[W];   // last key
+  int count[W];       // output entries
+  double lead[W];     // sum of the products before the first output entry (they end the last run of an earlier wavefront)
+  int stop[W];        // lead ends inside the wavefront
+  int open[W];        // its first position continues a run
+  long long o;
+};
+
+// Compresses a sorted row (wavefront w of W holds positions [w * 64 * K, ...), slot x % K of lane x / K) and writes it. A position
+// starts an output entry when it holds a product whose column differs from the previous position's. The runs of equal columns
+// are summed from their end to their start: in the lane, then over the lanes and wavefronts that a run goes on in (a segmented
+// suffix scan, skipped when no lane lies inside a run). A loop over each run's products in LDS took as many
+// dependent reads as the longest run has products, and all wavefronts of the row waited for the one with the hub
+// columns. Entries are staged in LDS by rank and stored with unit stride.
+template <int K, int W, int MODE, typename T, typename RP, typename SYNC>
+__device__ inline void esc_compress(const RowsDev<T, RP>& R, const TileDev<T, RP>& tile, int fr, unsigned (&key)[K], int w,
+                                    int lane, unsigned* s_key, double* s_val, EscShare<W>& sh, SYNC&& sync) {
+  constexpr bool NUM = MODE != 0;
+  unsigned prev = (unsigned)__shfl_up((int)key[K - 1], 1, 64);
+  if constexpr (W > 1) {
+    if (lane == 63) sh.last[w] = key[K - 1];
+    sync();
+    if (lane == 0 && w > 0) prev = sh.last[w - 1];
+  }
+  bool head[K], pad[K];
+  int mine = 0;
+#pragma unroll
+  for (int q = 0; q < K; q++) {
+    pad[q] = key[q] == kEscPad;
+    head[q] = !pad[q] && ((q == 0 && w == 0 && lane == 0) || (prev >> kEscKeyShift) != (key[q] >> kEscKeyShift));
+    prev = key[q];
+    mine += head[q] ? 1 : 0;
+  }
+  const int inc = wave_scan_dpp(mine);
+  const int wcnt = __builtin_amdgcn_readlane(inc, 63);
+  double v[NUM ? K : 1];
+  double carry = 0.0;       // sum of the lane's products before its first head, and on through later lanes
+  bool stop = true;         // carry ends
+  const bool open0 = !head[0] && !pad[0];
+  if constexpr (NUM) {
+#pragma unroll
+    for (int q = 0; q < K; q++) v[q] = pad[q] ? 0.0 : s_val[key[q] & kEscIdxMask];
+    stop = false;
+    bool in = open0;
+#pragma unroll
+    for (int q = 0; q < K; q++) {
+      in = in && !head[q] && !pad[q];
+      stop = stop || head[q] || pad[q];
+      if (in) carry += v[q];
+    }
+    for (int d = 1; d < 64; d <<= 1) {
+      if (__ballot(!stop) == 0ull) break;
+      const double c = __shfl_down(carry, d, 64);
+      const bool t = __shfl_down(stop ? 1 : 0, d, 64) != 0;
+      if (!stop && lane + d < 64) {
+        carry += c;
+        stop = t;
+      }
+    }
+  }
+  int before = 0, cnt = wcnt;
+  if constexpr (W > 1) {
+    if (lane == 0) {
+      sh.count[w] = wcnt;
+      if (NUM) {
+        sh.lead[w] = carry;
+        sh.stop[w] = stop;
+        sh.open[w] = open0;
+      }
+    }
+    sync();
+    cnt = 0;
+#pragma unroll
+    for (int q = 0; q < W; q++) {
+      if (q < w) before += sh.count[q];
+      cnt += sh.count[q];
+    }
+  }
+  if constexpr (MODE == 0) {
+    if (w == 0 && lane == 0) R.nnz[fr] = cnt;
+    sync();
+    return;
+  } else {
+    if (w == 0 && lane == 0) {
+      long long o;
+      if (MODE == 1 || (MODE == 2 && cnt <= R.cap[fr])) {
+        o = R.off[fr];
+      } else {
+        o = (long long)atomicAdd(R.cursor, (unsigned long long)cnt);
+        R.off[fr] = o;
+      }
+      if (o + cnt > R.out_limit) {  // refused: nothing is written and, after this pass, the row holds 0 entries
+        R.stats[3] = 1ull;
+        o = -1;
+        if (MODE != 1) R.off[fr] = 0;
+      }
+      R.nnz[fr] = (o < 0 && MODE != 1) ? 0 : cnt;
+      sh.o = o;
+    }
+    // what follows the lane's last position: the next lane's carry, or the next wavefronts'
+    double next = __shfl_down(carry, 1, 64);
+    bool cut = __shfl_down(open0 ? 1 : 0, 1, 64) == 0;
+    if (lane == 63) {
+      next = 0.0;
+      cut = true;
+      if constexpr (W > 1) {
+        bool go = w + 1 < W && sh.open[w + 1 < W ? w + 1 : w];
+        cut = !go;
+        for (int q = w + 1; q < W && go; q++) {
+          next += sh.lead[q];
+          go = !sh.stop[q];
+        }
+      }
+    }
+    if constexpr (W > 1) {  // a run through all later lanes of this wavefront continues in the next ones
+      const double far = __shfl(next, 63, 64);
+      const bool far_cut = __shfl(cut ? 1 : 0, 63, 64) != 0;
+      const bool through = __shfl_down(stop ? 1 : 0, 1, 64) == 0;  // the next lane's carry runs off the wavefront
+      if (lane < 63 && !cut && through && !far_cut) next += far;
+    }
+    int r = before + inc;  // one past the lane's last entry
+    T* s_out = reinterpret_cast<T*>(s_val);
+#pragma unroll
+    for (int q = K - 1; q >= 0; q--) {
+      next = cut ? v[q] : v[q] + next;
+      cut = head[q] || pad[q];
+      if (head[q]) {
+        r--;
+        s_key[r] = key[q] >> kEscKeyShift;
+        v[q] = next;
+      }
+    }
+    sync();  // every product is read: s_val takes the entries
+    r = before + inc;
+#pragma unroll
+    for (int q = K - 1; q >= 0; q--)
+      if (head[q]) s_out[--r] = (T)v[q];
+    sync();
+    const long long o = sh.o;
+    if (o >= 0) {
+      for (int x = w * 64 + lane; x < cnt; x += 64 * W) {
+        __builtin_nontemporal_store((int)s_key[x], &glob(tile.c_col)[o + x]);
+        __builtin_nontemporal_store(s_out[x], &glob(tile.c_val)[o + x]);
+      }
+    }
+    sync();
+  }
+}
+
+template <int K, int MODE, typename T, typename RP>
+__global__ __launch_bounds__(64 * kEscWaves) void k_esc(RowsDev<T, RP> R, int bin) {
+  constexpr int N = 64 * K;
+  constexpr bool NUM = MODE != 0;
+  __shared__ double s_val[kEscWaves][NUM ? N : 1];    // float64 products by product index, then the entries' values
+  __shared__ unsigned s_key[kEscWaves][NUM ? N : 1];  // the entries' columns
+  __shared__ EscShare<1> s_share[kEscWaves];
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const LaneLimits lim(lane);
+  auto wave_sync = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  const int count = *R.count_of(bin);
+  const int* items = R.bin_items + (int64_t)bin * R.bin_stride;
+  for (int idx = blockIdx.x * kEscWaves + w; idx < count; idx += gridDim.x * kEscWaves) {
+    const int fr = items[idx];
+    const TileDev<T, RP> tile = R.tiles[R.blk_tile[fr >> 8]];
+    const int64_t i = fr - tile.flat0;
+    unsigned key[K];
+    esc_expand<K, NUM>(tile, glob(tile.a_rp)[i], glob(tile.a_rp)[i + 1], 0, lane, key, s_val[w]);
+    esc_sort(key, lane, lim);
+    wave_sync();
+    esc_compress<K, 1, MODE>(R, tile, fr, key, 0, lane, s_key[w], s_val[w], s_share[w], wave_sync);
+  }
+}
+
+// ------------------------------------------------------------------------------------------------------------
+// Rows of at most 32 (64) products, 8 (16) lanes each. The products are expanded four per lane as 32-bit keys (column
+// << 5 (6) | product index), sorted in registers (DPP exchanges: no LDS, no barrier), and equal columns are summed in
+// product (A-row) order, in float64, rounded once.
+// A hash row of this size costs a table clear, LDS atomics and a sort of its table in LDS; a one-wavefront ESC row
+// leaves half the lanes idle. Tiles up to 2^27 - 2 columns wide. Modes as in k_esc.
+// ------------------------------------------------------------------------------------------------------------
+
+constexpr int kSmallWaves = 4;  // wavefronts per block
 
 // Ascending sort of the 4 * G keys of each row group (G = 8 or 16 lanes): in, any order; out, element x of the sorted
 // sequence is slot x % 4 of lane x / 4. Bitonic, with every comparator ascending (each merge first meets the mirrored
@@ -1417,10 +1559,10 @@ __global__ __launch_bounds__(64 * kSmallWaves, !ONE ? 6 : N == 32 ? 8 : 7) void 
 }
 
 // Sort-based rows of 512 * W products or fewer, W wavefronts per row: each wavefront expands and sorts 512 of the
-// row's products in registers (as the single-wavefront kernel does), the sorted runs are merged pairwise in place in
-// LDS (each key's merged position is its own index plus its rank in the partner run, found by binary search while
-// every key is still in place; ties go to the left run, so the pad keys fill the tail), and the block compresses the
-// sorted row. LDS: 12 bytes per product (key and float64 product) plus one staged chunk of A entries.
+// row's products in registers (as the single-wavefront kernel does), the sorted runs are merged pairwise by the rest of a
+// bitonic network, and the block compresses the sorted row. LDS: 12 bytes per product (key and float64 product). Rows of
+// 2048 to 4096 products of an R-MAT square at scale 16 (12 M products): symbolic 131 -> 77 us, numeric
+// 175 -> 110 us with the sort, the entry lookup and the compression above.
 constexpr int kEscChunk = 512;
 
 template <int W, int MODE, typename T, typename RP>
@@ -1428,155 +1570,53 @@ __global__ __launch_bounds__(64 * W, 6) void k_esc_block(RowsDev<T, RP> R, int b
   constexpr int N = kEscChunk * W;
   constexpr int K = kEscChunk / 64;
   constexpr bool NUM = MODE != 0;
-  __shared__ unsigned s_key[N];
+  typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+  __shared__ __align__(16) unsigned s_key[N];
   __shared__ double s_val[NUM ? N : 1];
-  __shared__ int s_pre[65];
-  __shared__ RP s_st[64];
-  __shared__ T s_av[64];
-  __shared__ int s_cnt[W];
-  __shared__ long long s_o;
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  __shared__ EscShare<W> s_share;
+  static_assert(K == 8, "two 16-byte accesses per lane");
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const LaneLimits lim(lane);
   const int count = *R.count_of(bin);
   const int* items = R.bin_items + (int64_t)bin * R.bin_stride;
   for (int idx = blockIdx.x; idx < count; idx += gridDim.x) {
     const int fr = items[idx];
     const TileDev<T, RP> tile = R.tiles[R.blk_tile[fr >> 8]];
     const int64_t i = fr - tile.flat0;
-    const RP a0 = tile.a_rp[i], a1 = tile.a_rp[i + 1];
     unsigned key[K];
-#pragma unroll
-    for (int k = 0; k < K; k++) key[k] = kEscPad;
-    // expand: wavefront 0 stages each chunk of 64 A entries; wavefront w takes products x in [w * 512, (w + 1) * 512)
-    int base = 0;
-    for (RP c0 = a0; c0 < a1; c0 += 64) {
-      const int ne = (int)((a1 - c0) < (RP)64 ? (a1 - c0) : (RP)64);
-      if (w == 0) {
-        int len = 0;
-        if (lane < ne) {
-          const int kk = tile.a_col[c0 + lane];
-          const RP st = tile.b_rp[kk];
-          len = (int)(tile.b_rp[kk + 1] - st);
-          s_st[lane] = st;
-          if (NUM) s_av[lane] = tile.a_val[c0 + lane];
-        }
-        int inc = len;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-          const int t = __shfl_up(inc, d, 64);
-          if (lane >= d) inc += t;
-        }
-        if (lane < ne) s_pre[lane] = inc - len;
-        if (lane == 63) s_pre[ne] = inc;
-      }
+    esc_expand<K, NUM>(tile, glob(tile.a_rp)[i], glob(tile.a_rp)[i + 1], w * kEscChunk, lane, key, s_val);
+    esc_sort(key, lane, lim);
+    // Merge: for each block size S = 1024 .. N, a mirror stage (position E against E ^ (S - 1)) and half-cleaners at
+    // distances S / 4 .. 1. Distances of 512 or more cross wavefronts and go through LDS, where a lane's eight keys are two
+    // 16-byte halves, each with neighbouring lanes side by side; shorter ones stay in registers and lanes.
+    // One stage across wavefronts: against wavefront w ^ dw, mirrored or not; the lower wavefront keeps the minimum.
+    auto cross = [&](int dw, auto mirror_tag, bool lower) {
+      constexpr bool mirrored = decltype(mirror_tag)::value;
+      u32x4* mine = reinterpret_cast<u32x4*>(s_key + w * kEscChunk);
+      const u32x4* other = reinterpret_cast<const u32x4*>(s_key + (w ^ dw) * kEscChunk);
+      mine[lane] = u32x4{key[0], key[1], key[2], key[3]};
+      mine[64 + lane] = u32x4{key[4], key[5], key[6], key[7]};
       __syncthreads();
-      const int total = s_pre[ne];
-      int lo[K];
-      esc_lookup<K>(s_pre, ne, base, lane, w * kEscChunk, lo);
+      const int l = mirrored ? 63 - lane : lane;
+      const u32x4 p = other[l], q = other[64 + l];
+      unsigned o[K];
 #pragma unroll
-      for (int k = 0; k < K; k++) {
-        const int x = w * kEscChunk + k * 64 + lane;
-        const int t = x - base;
-        if (t >= 0 && t < total) {
-          const RP q = s_st[lo[k]] + (RP)(t - s_pre[lo[k]]);
-          key[k] = ((unsigned)tile.b_col[q] << kEscKeyShift) | (unsigned)x;
-          if (NUM) s_val[x] = (double)s_av[lo[k]] * (double)tile.b_val[q];
-        }
+      for (int u = 0; u < 4; u++) {
+        o[u] = mirrored ? q[3 - u] : p[u];
+        o[4 + u] = mirrored ? p[3 - u] : q[u];
       }
-      base += total;
-      __syncthreads();
-    }
-    esc_sort<K>(key, lane);
-    // merge the wavefronts' sorted runs with the rest of a bitonic network: for each block size S = 1024 .. N, a
-    // mirror stage (position E against E ^ (S - 1)) and half-cleaners at distances S/4 .. 1. Distances of 512 or
-    // more cross wavefronts and go through LDS; shorter ones stay in registers and lanes.
-    const int E0 = w * kEscChunk + lane;  // position of key[k] is E0 + k * 64
-    // one compare-exchange stage across wavefronts: partner position E ^ d through LDS; mirror stages (d = S - 1)
-    // keep the minimum in the lower half of each S-block, half-cleaners in the lower half of each 2d-block
-    auto lds_stage = [&](int d, int S) {
 #pragma unroll
-      for (int k = 0; k < K; k++) s_key[E0 + k * 64] = key[k];
-      __syncthreads();
-#pragma unroll
-      for (int k = 0; k < K; k++) {
-        const int E = E0 + k * 64;
-        const unsigned o = s_key[E ^ d];
-        const bool lower = d == S - 1 ? (E & (S >> 1)) == 0 : (E & d) == 0;
-        key[k] = lower ? min(key[k], o) : max(key[k], o);
-      }
+      for (int u = 0; u < K; u++) key[u] = lower ? min(key[u], o[u]) : max(key[u], o[u]);
       __syncthreads();
     };
-#pragma unroll
-    for (int S = 2 * kEscChunk; S <= N; S <<= 1) {
-      lds_stage(S - 1, S);
-      for (int d = S >> 2; d >= kEscChunk; d >>= 1) lds_stage(d, S);
-      esc_half_clean<K>(key, lane);
+#pragma unroll 1
+    for (int s = 2; s <= W; s <<= 1) {
+      cross(s - 1, std::true_type{}, (w & (s >> 1)) == 0);
+#pragma unroll 1
+      for (int d = s >> 2; d > 0; d >>= 1) cross(d, std::false_type{}, (w & d) == 0);
+      esc_half_clean(key, lim);
     }
-#pragma unroll
-    for (int k = 0; k < K; k++) s_key[E0 + k * 64] = key[k];
-    __syncthreads();
-    // compress: wavefront w owns sorted positions [w * 512, (w + 1) * 512), as k * 64 + lane
-    int wcnt = 0;
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-      const int p = w * kEscChunk + k * 64 + lane;
-      const unsigned prev = p > 0 ? s_key[p - 1] : kEscPad;
-      const bool head = key[k] != kEscPad && (p == 0 || (prev >> kEscKeyShift) != (key[k] >> kEscKeyShift));
-      wcnt += __popcll(__ballot(head));
-    }
-    if (lane == 0) s_cnt[w] = wcnt;
-    __syncthreads();
-    int before = 0, cnt = 0;
-#pragma unroll
-    for (int q = 0; q < W; q++) {
-      if (q < w) before += s_cnt[q];
-      cnt += s_cnt[q];
-    }
-    if (MODE == 0) {
-      if (threadIdx.x == 0) R.nnz[fr] = cnt;
-      __syncthreads();
-      continue;
-    }
-    if (threadIdx.x == 0) {
-      long long o;
-      if (MODE == 1 || (MODE == 2 && cnt <= R.cap[fr])) {
-        o = R.off[fr];
-      } else {
-        o = (long long)atomicAdd(R.cursor, (unsigned long long)cnt);
-        R.off[fr] = o;
-      }
-      if (o + cnt > R.out_limit) {  // refused: nothing is written and, after this pass, the row holds 0 entries
-        R.stats[3] = 1ull;
-        o = -1;
-        if (MODE != 1) R.off[fr] = 0;
-      }
-      R.nnz[fr] = (o < 0 && MODE != 1) ? 0 : cnt;
-      s_o = o;
-    }
-    __syncthreads();
-    const long long o = s_o;
-    if (o >= 0) {
-#pragma unroll
-      for (int k = 0; k < K; k++) {
-        const int p = w * kEscChunk + k * 64 + lane;
-        const unsigned prev = p > 0 ? s_key[p - 1] : kEscPad;
-        const bool head = key[k] != kEscPad && (p == 0 || (prev >> kEscKeyShift) != (key[k] >> kEscKeyShift));
-        const unsigned long long mask = __ballot(head);
-        if (head) {
-          const unsigned col = key[k] >> kEscKeyShift;
-          double sum = s_val[key[k] & kEscIdxMask];
-          for (int p2 = p + 1; p2 < N; p2++) {
-            const unsigned kp = s_key[p2];
-            if (kp == kEscPad || (kp >> kEscKeyShift) != col) break;
-            sum += s_val[kp & kEscIdxMask];
-          }
-          const long long pos = o + before + __popcll(mask & ((1ull << lane) - 1ull));
-          __builtin_nontemporal_store((int)col, &tile.c_col[pos]);
-          __builtin_nontemporal_store((T)sum, &tile.c_val[pos]);
-        }
-        before += __popcll(mask);
-      }
-    }
-    __syncthreads();
+    esc_compress<K, W, MODE>(R, tile, fr, key, w, lane, s_key, s_val, s_share, [] { __syncthreads(); });
   }
 }
 
