@@ -7,7 +7,7 @@
 // as a tree of merge-path merges, and equal (row, column) pairs, now adjacent and in tile order, are summed in
 // float64 and rounded once. A counting merge sizes the rows, a scan places them, a second merge writes them.
 //
-// Measured: eight R-MAT scale 16 tiles (11.2 M entries, fp32) 11.0 ms through the general path, 0.91 ms here.
+// Measured: eight R-MAT scale 16 tiles (11.2 M entries, fp32) 11.0 ms through the general path, 0.81 ms here.
 //
 // Tiles whose columns are not strictly increasing within each row, and sums of more than kAccMaxTiles tiles (one lane
 // per tile sets a piece up), take the general path: one SpGEMM [T_1 T_2 ... T_K] * [I; I; ...; I], where the left operand stacks the tiles side by side
@@ -160,7 +160,8 @@ struct AccDev {
   int32_t* piece_cnt;    // entries of C per piece
   int32_t* npieces;      // pieces in use
   int32_t* bad;          // [0] set by the cut (descriptors disagree with the row_ptrs: nothing may use the pieces),
-                         // [1] set by the merge (columns not strictly increasing): the general path takes the sum
+                         // [1] set by the cut and the merge (columns not strictly increasing): the general path
+                         // takes the sum
 };
 
 // row weights: entries over all tiles, plus one (so a span of weights holds a bounded number of empty rows too)
@@ -224,7 +225,7 @@ __global__ __launch_bounds__(256) void k_acc_split(AccDev<T, RP> D) {
     const int* col = live ? D.tile[lane].col : nullptr;
     int64_t lo = live ? (int64_t)D.tile[lane].rp[pc.row] : 0;
     int64_t hi = live ? (int64_t)D.tile[lane].rp[pc.row + 1] : 0;
-    const int64_t first = lo;
+    const int64_t first = lo, last = hi;
     const int64_t len = wave_sum<long long>(hi - lo);
     const int64_t want = pc.q * ((len + pc.npieces - 1) / pc.npieces);
     int64_t clo = 0, chi = pc.q == 0 ? 1 : D.n;
@@ -244,16 +245,23 @@ __global__ __launch_bounds__(256) void k_acc_split(AccDev<T, RP> D) {
         hi = a;
       }
     }
-    if (live) D.bound[(int64_t)p * D.K + lane] = lo;
+    if (live) {
+      D.bound[(int64_t)p * D.K + lane] = lo;
+      // the merge looks at the order inside a piece: here, at the seam to the piece before
+      if (lo > first && lo < last && col[lo - 1] >= col[lo]) D.bad[1] = 1;
+    }
   }
 }
 
 // One workgroup per piece (blocks below nlong: long-row pieces, strided; then one block per span of short rows).
 // NUM false: entries of C per row (cnt) and per long-row piece; NUM true: the entries, at off[].
-// Bound by LDS reads of the merge tree (log2 K levels, about two 8-byte reads per entry and level) and the latency of
-// the piece's loads; five workgroups per CU (fp32) cover each other's.
+// Bound by VALU instructions, a third of them in the merge tree (log2 K levels, about two 8-byte LDS reads per entry and
+// level), with five workgroups per CU (fp32; four for the writing pass, three in fp64) to cover each other's loads: counting
+// pass of eight R-MAT scale 16 tiles 195 -> 157 us and writing pass 251 -> 231 us when the loads of a piece were put
+// in one batch.
 template <bool NUM, typename T, typename RP>
-__global__ __launch_bounds__(kAccThreads) void k_acc_merge(AccDev<T, RP> D, int nlong, int* c_col, T* c_val) {
+__global__ __launch_bounds__(kAccThreads, NUM ? (sizeof(T) == 8 ? 3 : 4) : 5) void k_acc_merge(AccDev<T, RP> D, int nlong,
+                                                                                               int* c_col, T* c_val) {
   __shared__ unsigned long long s_key[kAccCap];
   __shared__ T s_val[NUM ? kAccCap : 1];
   __shared__ unsigned s_mark[kAccCap];  // tile << 10 | local row of each slot; then entries per local row
@@ -264,36 +272,41 @@ __global__ __launch_bounds__(kAccThreads) void k_acc_merge(AccDev<T, RP> D, int 
   __shared__ unsigned s_scan[kAccThreads / 64 + 1];
   __shared__ long long s_base;
   const int tid = threadIdx.x, K = D.K;
-  if (D.bad[0]) return;  // written by an earlier kernel only
   const bool is_long = (int)blockIdx.x < nlong;
+  const int bad = D.bad[0];  // written by an earlier kernel only
   const int np = is_long ? *D.npieces : 1;
+  int row0 = 0, nrows = 1;
+  if (!is_long) {
+    const int64_t c = (int64_t)blockIdx.x - nlong;
+    row0 = D.chunk[2 * c];
+    nrows = D.chunk[2 * c + 1] - row0;
+  }
+  TileIn<T, RP> mine{};  // of tile tid
+  if (tid < K) mine = D.tile[tid];
+  if (bad || nrows <= 0) return;
   for (int p = is_long ? (int)blockIdx.x : 0; p < np; p += nlong > 0 && is_long ? nlong : 1) {
     // the piece's K runs: [beg, beg + len) of each tile, laid out one after the other in the slots
-    int row0, nrows;
     AccPiece pc{0, 0, 0};
     if (is_long) {
       pc = D.piece[p];
       row0 = pc.row;
-      nrows = 1;
-    } else {
-      const int64_t c = (int64_t)blockIdx.x - nlong;
-      row0 = D.chunk[2 * c];
-      nrows = D.chunk[2 * c + 1] - row0;
-      if (nrows <= 0) return;
     }
     if (tid < 64) {
       int64_t beg = 0, end = 0;
       if (tid < K) {
         if (is_long) {
           beg = D.bound[(int64_t)p * K + tid];
-          end = pc.q + 1 < pc.npieces ? D.bound[(int64_t)(p + 1) * K + tid] : (int64_t)D.tile[tid].rp[row0 + 1];
+          // the next piece is the row's, or another row's (or past the last): read with the rest, not after it
+          const int64_t next = D.bound[(int64_t)(p + 1 < np ? p + 1 : p) * K + tid];
+          end = (int64_t)mine.rp[row0 + 1];
+          if (pc.q + 1 < pc.npieces) end = next;
         } else {
-          beg = (int64_t)D.tile[tid].rp[row0];
-          end = (int64_t)D.tile[tid].rp[row0 + nrows];
+          beg = (int64_t)mine.rp[row0];
+          end = (int64_t)mine.rp[row0 + nrows];
         }
         s_beg[tid] = beg;
-        s_tcol[tid] = D.tile[tid].col;
-        if (NUM) s_tval[tid] = D.tile[tid].val;
+        s_tcol[tid] = mine.col;
+        if (NUM) s_tval[tid] = mine.val;
       }
       const bool back = end < beg;  // only possible when the row is not sorted
       const int len = back ? 0 : (int)(end - beg < kAccCap ? end - beg : kAccCap);
@@ -352,18 +365,30 @@ __global__ __launch_bounds__(kAccThreads) void k_acc_merge(AccDev<T, RP> D, int 
       }
     }
     __syncthreads();
+    // every load of the piece is issued before the first is used
+    int64_t at[kAccItems];
+    int tile[kAccItems], col[kAccItems];
+    T val[NUM ? kAccItems : 1];
+#pragma unroll
+    for (int v = 0; v < kAccItems; v++) {
+      const int s = v * kAccThreads + tid;
+      tile[v] = s < E ? (int)(s_mark[s] >> 10) : 0;
+      at[v] = s_beg[tile[v]] + (s - s_seg[tile[v]]);
+    }
+#pragma unroll
+    for (int v = 0; v < kAccItems; v++) {
+      if (v * kAccThreads + tid < E) {
+        col[v] = glob(s_tcol[tile[v]])[at[v]];
+        if (NUM) val[v] = glob(s_tval[tile[v]])[at[v]];
+      }
+    }
 #pragma unroll
     for (int v = 0; v < kAccItems; v++) {
       const int s = v * kAccThreads + tid;
       if (s < E) {
-        const unsigned mk = s_mark[s];
-        const int t = (int)(mk >> 10);
-        const int64_t q = s_beg[t] + (s - s_seg[t]);
-        const int c = s_tcol[t][q];
-        if (is_long && s == s_seg[t] && q > (int64_t)D.tile[t].rp[row0] && s_tcol[t][q - 1] >= c) D.bad[1] = 1;
-        s_key[s] = (unsigned long long)(mk & 1023u) << (31 + kAccSlotBits) |
-                   (unsigned long long)((unsigned)c & 0x7fffffffu) << kAccSlotBits | (unsigned)s;
-        if (NUM) s_val[s] = s_tval[t][q];
+        s_key[s] = (unsigned long long)(s_mark[s] & 1023u) << (31 + kAccSlotBits) |
+                   (unsigned long long)((unsigned)col[v] & 0x7fffffffu) << kAccSlotBits | (unsigned)s;
+        if (NUM) s_val[s] = val[v];
       }
     }
     __syncthreads();
