@@ -193,9 +193,12 @@ void FlatRows<T, RP>::bin(hipStream_t s, int src) {
 }
 
 template <typename T, typename RP>
-void FlatRows<T, RP>::scan(hipStream_t s, const int32_t* cnt, int64_t* off, int64_t off_add) {
+void FlatRows<T, RP>::scan(hipStream_t s, const int32_t* cnt, int64_t* off, int64_t off_add, bool with_report) {
+  reported = false;
   if (nflat <= kScanOneMax) {
-    hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(kScanBlock), 0, s, cnt, nflat, off, off_add, scan_total);
+    hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(1024), 0, s, cnt, nflat, off, off_add, scan_total,
+                       (const int32_t*)R.bin_count, with_report ? h->h_pinned : nullptr);
+    reported = with_report;
     BCLX_HIP(hipGetLastError());
     return;
   }
@@ -242,7 +245,8 @@ void scan_counts(hipStream_t s, const int32_t* cnt, int64_t n, int64_t* off, lon
     return;
   }
   if (n <= kScanOneMax) {
-    hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(kScanBlock), 0, s, cnt, n, off, (int64_t)0, total);
+    hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(1024), 0, s, cnt, n, off, (int64_t)0, total, (const int32_t*)nullptr,
+                       (int64_t*)nullptr);
     BCLX_HIP(hipGetLastError());
     return;
   }
@@ -436,8 +440,11 @@ void FlatRows<T, RP>::read_counts(hipStream_t s, int32_t* dst) {
 template <typename T, typename RP>
 int64_t FlatRows<T, RP>::report(hipStream_t s, int32_t* counts) {
   static_assert(kNumBins + 1 <= kPinnedCounts && kNumBins < 64, "one value per lane");
-  hipLaunchKernelGGL((k_report<T, RP>), dim3(1), dim3(64), 0, s, R, (const int64_t*)scan_total, h->h_pinned);
-  BCLX_HIP(hipGetLastError());
+  if (!reported) {
+    hipLaunchKernelGGL((k_report<T, RP>), dim3(1), dim3(64), 0, s, R, (const int64_t*)scan_total, h->h_pinned);
+    BCLX_HIP(hipGetLastError());
+  }
+  reported = false;
   BCLX_HIP(hipStreamSynchronize(s));
   for (int b = 0; b < kNumBins; b++) counts[b] = (int32_t)h->h_pinned[b];
   return h->h_pinned[kNumBins];
@@ -545,7 +552,7 @@ int64_t TwoPhase<T, RP>::symbolic() {
   if (small_rows) {
     F.run_bin(s, 0, kSmallBin, -1);
     F.run_bin(s, 0, kEscBin0, -1);
-    F.scan(s, F.R.nnz, F.R.off, 0);
+    F.scan(s, F.R.nnz, F.R.off, 0, true);
   }
   int64_t tot = F.report(s, counts);
   if (counts[kHeavyBin] > 0) F.prepare_heavy();
@@ -558,7 +565,7 @@ int64_t TwoPhase<T, RP>::symbolic() {
     more = true;
   }
   if (more) {
-    F.scan(s, F.R.nnz, F.R.off, 0);
+    F.scan(s, F.R.nnz, F.R.off, 0, true);
     int32_t again[kNumBins];
     tot = F.report(s, again);
   }

@@ -47,7 +47,8 @@ struct FlatRows {
   void analyze(hipStream_t s, bool do_bin, long long pred_min = -1, bool with_stats = true, bool cleared = false);
   void bin(hipStream_t s, int src);
   // exclusive scan of cnt over all flat rows into off (nflat + 1 entries), plus off_add; total -> *scan_total
-  void scan(hipStream_t s, const int32_t* cnt, int64_t* off, int64_t off_add);
+  // with_report: a one-launch scan also writes what report() waits for
+  void scan(hipStream_t s, const int32_t* cnt, int64_t* off, int64_t off_add, bool with_report = false);
   // planned: plan_heavy() ran before (the heavy bin)
   void run_bin(hipStream_t s, int mode, int b, int64_t count_hint, bool planned = false);
   // The heavy bin's small kernels (order, split and, in modes 2 and 3, counting and placing the parts). Callers that run
@@ -65,6 +66,7 @@ struct FlatRows {
   int64_t report(hipStream_t s, int32_t* counts);  // the bin counts and the last scan's total (synchronises s)
 
  private:
+  bool reported = false;  // the last scan wrote the report
   void layout(bool with_cap, bool pooled, bool* from_pool);
 };
 

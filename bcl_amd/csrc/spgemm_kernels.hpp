@@ -2619,29 +2619,71 @@ __global__ __launch_bounds__(kRowBlock) void k_compact(RowsDev<T, RP> R, const i
   }
 }
 
-// Scan of at most kScanOneMax counts by one workgroup: one launch instead of three (500 rows 2.7 us, 16384 rows 9.4 us;
-// the three took 6.7 and 8.3 us and two more gaps between launches).
-constexpr int64_t kScanOneMax = 8 * kScanTile;
-static __global__ __launch_bounds__(kScanBlock) void k_scan_one(const int32_t* cnt, int64_t n, int64_t* off,
-                                                                int64_t off_add, int64_t* total_out) {
-  __shared__ long long sm[kScanBlock / 64 + 1];
-  long long base = 0;
-  for (int64_t b = 0; b < n; b += kScanTile) {
-    const int64_t r0 = b + (int64_t)threadIdx.x * kScanPer;
-    long long v[kScanPer];
-    scan_load4(cnt, n, r0, v);
-    long long tot;
-    long long run = base + off_add + block_excl_scan<kScanBlock, long long>(v[0] + v[1] + v[2] + v[3], &tot, sm);
+// Scan of at most kScanOneMax counts by one workgroup: one launch instead of three. A wavefront takes 1024 neighbouring
+// counts, 64 per instruction, scans them by DPP, and the block meets at one barrier: 16384 rows 8.3 us (9.4 with four counts
+// per thread side by side, bound by the 8-byte stores of neighbouring lanes going to different lines; three launches
+// 8.3 and two more gaps between them). report (may be null): the bin counts and the total go to pinned host
+// memory, kNumBins + 1 values, as k_report writes them.
+constexpr int kScanOnePer = 16;
+constexpr int64_t kScanOneMax = 2 * 1024 * kScanOnePer;
+
+// Inclusive scan of one 64-bit value per lane of a wavefront, by DPP.
+__device__ inline long long wave_scan_dpp64(long long v) {
+  auto step = [&](auto ctrl, auto rows) {
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)v, decltype(ctrl)::value, decltype(rows)::value, 0xF, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(v >> 32), decltype(ctrl)::value, decltype(rows)::value, 0xF, false);
+    v += (long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo);
+  };
+  constexpr std::integral_constant<int, 0xF> all{};
+  step(std::integral_constant<int, 0x111>{}, all);  // row_shr:1, 2, 4, 8
+  step(std::integral_constant<int, 0x112>{}, all);
+  step(std::integral_constant<int, 0x114>{}, all);
+  step(std::integral_constant<int, 0x118>{}, all);
+  step(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xA>{});  // row_bcast:15 into rows 1 and 3
+  step(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xC>{});  // row_bcast:31 into rows 2 and 3
+  return v;
+}
+__device__ inline long long read_lane64(long long v, int lane) {
+  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)v, lane);
+  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(v >> 32), lane);
+  return (long long)(((unsigned long long)hi << 32) | lo);
+}
+
+static __global__ __launch_bounds__(1024) void k_scan_one(const int32_t* cnt, int64_t n, int64_t* off, int64_t off_add,
+                                                          int64_t* total_out, const int32_t* bin_count, int64_t* report) {
+  __shared__ long long s_wave[2][16];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  if (report && threadIdx.x < kNumBins) report[threadIdx.x] = bin_count[threadIdx.x * kCountStride];
+  long long base = off_add;
+  int turn = 0;
+  for (int64_t b = 0; b < n; b += 1024 * kScanOnePer, turn ^= 1) {
+    const int64_t r0 = b + w * 64 * kScanOnePer + lane;
+    int v[kScanOnePer];
 #pragma unroll
-    for (int q = 0; q < kScanPer; q++) {
-      if (r0 + q < n) off[r0 + q] = run;
-      run += v[q];
+    for (int q = 0; q < kScanOnePer; q++) v[q] = r0 + q * 64 < n ? cnt[r0 + q * 64] : 0;
+    long long ex[kScanOnePer], mine = 0;  // exclusive in the wavefront; its total so far
+#pragma unroll
+    for (int q = 0; q < kScanOnePer; q++) {
+      ex[q] = 0;
+      if (r0 - lane + q * 64 < n) {  // uniform
+        const long long inc = wave_scan_dpp64(v[q]);
+        ex[q] = mine + inc - v[q];
+        mine += read_lane64(inc, 63);
+      }
     }
-    base += tot;
+    if (lane == 0) s_wave[turn][w] = mine;
+    __syncthreads();
+    const long long waves = wave_scan_dpp64(lane < 16 ? s_wave[turn][lane] : 0ll);
+    const long long run = base + (w > 0 ? read_lane64(waves, w - 1) : 0ll);
+#pragma unroll
+    for (int q = 0; q < kScanOnePer; q++)
+      if (r0 + q * 64 < n) off[r0 + q * 64] = run + ex[q];
+    base += read_lane64(waves, 15);
   }
   if (threadIdx.x == 0) {
-    off[n] = base + off_add;
-    if (total_out) *total_out = base;
+    off[n] = base;
+    if (total_out) *total_out = base - off_add;
+    if (report) report[kNumBins] = base - off_add;
   }
 }
 
