@@ -10,12 +10,12 @@
 //      search; A's columns are sorted within each row) and writes that start and the segment length;
 //   2. one scan over the lengths of all tile columns, one column after the other, turns them into offsets; a tile's
 //      row_ptr is that scan restricted to its rows, minus the value at its first row;
-//   3. copy: work is split by entries (kSplitChunk per workgroup), so hub rows and short rows cost the same; a lane
+//   3. copy: work is split by entries plus rows (kSplitChunk per workgroup), so hub, short and empty rows cost the same; a lane
 //      finds its entry's row in a window of row offsets in LDS, its tile column by a division, and writes the entry to
 //      its tile at (row offset + position in the segment).
 // Bytes: A's row_ptr and col_idx are read twice (count, copy) and its values once; every tile is written once. Measured
 // on R-MAT scale 20 (15.7 M entries, 4 x 4 tiles), sizes and copy together: 1.82 ms with one wavefront per row and
-// one scan per tile column, 0.51 ms this way.
+// one scan per tile column, 0.43 ms this way.
 //
 // bclx_dense_binary_op is DMatrix's elementwise arithmetic on a tile (DMatrix::binary_op / binary_op_inplace,
 // bcl/containers/DMatrix.hpp:319-366, with operator+, -, *, / and += at :368-386): C = A op B per element, rows of
@@ -30,7 +30,8 @@
 namespace bclx {
 
 constexpr int kSplitMaxGridN = 256;            // tile columns of one split
-constexpr int kSplitChunk = 4096;              // entries of A per copying workgroup
+constexpr int kSplitChunk = 4096;              // entries plus rows of A per copying workgroup
+constexpr int kSplitWindow = 1024;             // rows whose offsets a copying workgroup holds at a time
 
 // Row i's segment of tile column tj: seg[tj * stride + i] = its first position within the row, cnt[...] its length.
 // A block takes 256 / gn whole rows, so a segment's end is its neighbour's start. Also clears the counts that pad a
@@ -76,23 +77,29 @@ struct SplitTile {
   int32_t ptr_width;
 };
 
+struct SplitChunk {
+  int64_t row, entry;  // where a chunk of A starts
+};
+
 // i / d, in 32 bits where the rows fit them
 __device__ inline int64_t row_div(int64_t i, int64_t d, int64_t m) {
   return m <= (int64_t)UINT32_MAX && d <= (int64_t)UINT32_MAX ? (int64_t)((uint32_t)i / (uint32_t)d) : i / d;
 }
 
 // The tiles' row_ptrs from the scanned offsets: one thread per (tile column, row). The threads of tile column 0 also
-// list, for each chunk of kSplitChunk entries of A, the row holding its first entry.
+// cut A into chunks of kSplitChunk entries plus rows: row i weighs its entries and one more; chunk[c] is the row
+// that weight c * kSplitChunk falls in and the entry it stands for.
 template <typename RP>
 __global__ __launch_bounds__(256) void k_split_rowptr(const RP* rp, const int64_t* off, int64_t stride, int64_t m,
                                                       int64_t tile_m, int gn, const SplitTile* tiles,
-                                                      int64_t* chunk_row) {
+                                                      SplitChunk* chunk, int64_t nchunks) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int tj = blockIdx.y;
   if (i >= m) return;
   if (tj == 0) {
     const int64_t a0 = (int64_t)rp[i], a1 = (int64_t)rp[i + 1];
-    for (int64_t c = (a0 + kSplitChunk - 1) / kSplitChunk; c * kSplitChunk < a1; c++) chunk_row[c] = i;
+    for (int64_t c = (a0 + i + kSplitChunk - 1) / kSplitChunk; c < nchunks && c * kSplitChunk <= a1 + i; c++)
+      chunk[c] = SplitChunk{i, c * kSplitChunk - i < a1 ? c * kSplitChunk - i : a1};
   }
   const int64_t ti = row_div(i, tile_m, m), first = ti * tile_m, li = i - first;
   const int64_t rows = (m - first) < tile_m ? (m - first) : tile_m;
@@ -108,37 +115,51 @@ __global__ __launch_bounds__(256) void k_split_rowptr(const RP* rp, const int64_
   }
 }
 
-// Copies A's entries [blockIdx * kSplitChunk, ...) to their tiles, walking windows of 256 row offsets from the chunk's
-// first row; unit-stride loads, four entries in flight per thread. An entry that would land outside its tile (columns
+// Copies a chunk of A's entries to their tiles, walking windows of its row offsets; unit-stride loads, four entries in flight
+// per thread. An entry that would land outside its tile (columns
 // of A not sorted within the row, or not below n) is not written and sets *bad.
+// Bound by the latency of a window (offsets, then entries, then stores): chunks of 4096 entries alone and windows of 256 rows
+// gave the workgroups on the sparse rows of an R-MAT matrix up to a hundred windows one after the other (16 M entries at
+// scale 20 into 4 x 4 tiles: 218 -> 120 us; 4 M rows with an entry in every 20th, 2 x 2 tiles, sizes and copy 1030 ->
+// 260 us). Staging each segment's place in LDS instead of reading it per entry
+// made no difference.
 template <typename RP, typename T>
 __global__ __launch_bounds__(256) void k_split_copy(const RP* rp, const int32_t* col, const T* val, int64_t m,
                                                     int64_t n, int64_t tile_m, uint32_t tile_n, int gn,
                                                     const int64_t* off, const int32_t* seg, int64_t stride,
-                                                    const SplitTile* tiles, const int64_t* chunk_row, int64_t total,
-                                                    int32_t* bad) {
-  __shared__ int64_t s_rp[257];
+                                                    const SplitTile* tiles, const SplitChunk* chunk, int64_t nchunks,
+                                                    int64_t total, int32_t* bad) {
+  __shared__ int s_rp[kSplitWindow + 1];  // offsets less the window's first entry, from -1 (before it) to kSplitChunk
+  __shared__ int64_t s_first, s_end;      // first and last offset
   const int tid = threadIdx.x;
-  const int64_t c0 = (int64_t)blockIdx.x * kSplitChunk;
-  if (c0 >= total) return;
-  const int64_t c1 = c0 + kSplitChunk < total ? c0 + kSplitChunk : total;
-  int64_t r0 = chunk_row[blockIdx.x];
-  int64_t e = c0;
-  while (e < c1 && r0 < m) {
-    const int64_t r = r0 + tid;
-    s_rp[tid] = (int64_t)rp[r < m ? r : m];
-    if (tid == 0) s_rp[256] = (int64_t)rp[r0 + 256 < m ? r0 + 256 : m];
+  const int64_t b = blockIdx.x;
+  // the chunk's rows [r0, r1] and entries [e, c1)
+  const SplitChunk from = chunk[b], to = b + 1 < nchunks ? chunk[b + 1] : SplitChunk{m - 1, total};
+  int64_t r0 = from.row, e = from.entry;
+  const int64_t r1 = to.row, c1 = to.entry;
+  while (e < c1 && r0 <= r1) {
+    const int rows = (int)(r1 - r0 + 1 < kSplitWindow ? r1 - r0 + 1 : kSplitWindow);
+    int top = 1;  // the largest power of two below the number of rows, or 0
+    while (top < rows) top <<= 1;
+    for (int r = tid; r <= top; r += 256) {
+      const int64_t p = (int64_t)rp[r0 + (r < rows ? r : rows)], d = p - e;
+      s_rp[r] = r >= rows || d > kSplitChunk ? kSplitChunk : d < -1 ? -1 : (int)d;
+      if (r == 0) s_first = p;
+      if (r == rows) s_end = p;
+    }
     __syncthreads();
-    const int64_t we = s_rp[256] < c1 ? s_rp[256] : c1;
+    const int64_t we = s_end < c1 ? s_end : c1, p0 = s_first;
+    top >>= 1;
     for (int64_t x0 = e; x0 < we; x0 += 4 * 256) {
-      int a[4];  // largest a with s_rp[a] <= x: four branchless searches in lockstep
+      int a[4];  // largest a with s_rp[a] <= x - e: four branchless searches in lockstep
 #pragma unroll
       for (int q = 0; q < 4; q++) a[q] = 0;
 #pragma unroll
-      for (int step = 128; step > 0; step >>= 1) {
+      for (int step = kSplitWindow / 2; step > 0; step >>= 1) {
+        if (step > top) continue;  // uniform
 #pragma unroll
         for (int q = 0; q < 4; q++)
-          if (s_rp[a[q] + step] <= x0 + q * 256 + tid) a[q] += step;
+          if (s_rp[a[q] + step] <= (int)(x0 - e) + q * 256 + tid) a[q] += step;
       }
       int c[4];
       T v[4];
@@ -159,7 +180,8 @@ __global__ __launch_bounds__(256) void k_split_copy(const RP* rp, const int32_t*
         }
         const int64_t i = r0 + a[q], ti = row_div(i, tile_m, m);
         const int64_t* o = off + (int64_t)tj * stride;
-        const int64_t at = x - s_rp[a[q]] - seg[(int64_t)tj * stride + i];  // position within the segment
+        const int64_t row = a[q] > 0 ? e + s_rp[a[q]] : p0;  // only the first row starts before the window's entries
+        const int64_t at = x - row - seg[(int64_t)tj * stride + i];  // position within the segment
         const int64_t oi = o[i], dst = oi - o[ti * tile_m] + at;
         const SplitTile& t = tiles[ti * gn + tj];
         if (at < 0 || oi + at >= o[i + 1] || dst < 0 || dst >= t.nnz) {
@@ -171,7 +193,7 @@ __global__ __launch_bounds__(256) void k_split_copy(const RP* rp, const int32_t*
       }
     }
     e = we > e ? we : e;
-    r0 += 256;
+    r0 += kSplitWindow;
     __syncthreads();
   }
 }
@@ -200,7 +222,7 @@ void split_grid(bclx_handle* h, const bclx_csr* A, int64_t tile_m, int64_t tile_
                o_off = ws.reserve(sizeof(int64_t) * (size_t)(L + 4)),
                o_part = ws.reserve(sizeof(long long) * (size_t)scan_partials(L)),
                o_tot = ws.reserve(sizeof(int64_t) * (size_t)(gm * gn + 1)),
-               o_chunk = ws.reserve(sizeof(int64_t) * (size_t)(A->nnz / kSplitChunk + 1)),
+               o_chunk = ws.reserve(sizeof(SplitChunk) * (size_t)((A->nnz + m) / kSplitChunk + 1)),
                o_tile = ws.reserve(sizeof(SplitTile) * (size_t)(gm * gn)), o_bad = ws.reserve(sizeof(int32_t));
   ScratchUse use(h, ws);
   int32_t* cnt = ws.at<int32_t>(o_cnt);
@@ -251,20 +273,21 @@ void split_grid(bclx_handle* h, const bclx_csr* A, int64_t tile_m, int64_t tile_
   const int64_t entries = nnz.back();
   DevBuf more_chunks;
   if (m > 0) {
-    int64_t* chunk_row = ws.at<int64_t>(o_chunk);
+    SplitChunk* chunk = ws.at<SplitChunk>(o_chunk);
     if (entries > A->nnz) {  // the descriptor's nnz is not what row_ptr says
-      more_chunks.alloc(sizeof(int64_t) * (size_t)(entries / kSplitChunk + 1));
-      chunk_row = more_chunks.as<int64_t>();
+      more_chunks.alloc(sizeof(SplitChunk) * (size_t)((entries + m) / kSplitChunk + 1));
+      chunk = more_chunks.as<SplitChunk>();
     }
+    const int64_t nchunks = (entries + m + kSplitChunk - 1) / kSplitChunk;
     SplitTile* dt = ws.at<SplitTile>(o_tile);
     BCLX_HIP(hipMemcpyAsync(dt, st.data(), sizeof(SplitTile) * st.size(), hipMemcpyHostToDevice, s));
     hipLaunchKernelGGL((k_split_rowptr<RP>), dim3(div_up(m, 256), (unsigned)gn), dim3(256), 0, s, rp, off, stride, m,
-                       tile_m, gn, dt, chunk_row);
+                       tile_m, gn, dt, chunk, nchunks);
     BCLX_HIP(hipGetLastError());
     if (entries > 0) {
-      hipLaunchKernelGGL((k_split_copy<RP, T>), dim3(div_up(entries, kSplitChunk)), dim3(256), 0, s, rp, A->col_idx,
+      hipLaunchKernelGGL((k_split_copy<RP, T>), dim3((unsigned)nchunks), dim3(256), 0, s, rp, A->col_idx,
                          static_cast<const T*>(A->vals), m, A->n, tile_m, (uint32_t)std::min<int64_t>(tile_n, UINT32_MAX),
-                         gn, off, seg, stride, dt, chunk_row, entries, bad);
+                         gn, off, seg, stride, dt, chunk, nchunks, entries, bad);
       BCLX_HIP(hipGetLastError());
     }
     BCLX_HIP(hipMemcpyAsync(&h_bad, bad, sizeof(int32_t), hipMemcpyDeviceToHost, s));
