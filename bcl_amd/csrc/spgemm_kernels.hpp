@@ -67,7 +67,8 @@ __host__ __device__ inline int bin_for(int64_t need, int64_t work, const BinTuni
   if (tn.esc_max > 0 && work <= kSmallMax && n < ((int64_t)1 << kSmallColBits) - 1) return kSmallBin;
   const bool esc_ok = n <= (1 << kEscColBits);
   if (esc_ok && work > tn.esc_min && work <= tn.esc_max && work <= kEscMaxProducts) return esc_bin(work);
-  if (need > (esc_ok && tn.heavy_need > kRankNeed ? kRankNeed : tn.heavy_need)) return kHeavyBin;
+  const bool rank = esc_ok && work > kEscMaxProducts;  // the rank-slice kernel takes it from kRankNeed on
+  if (need > (rank && tn.heavy_need > kRankNeed ? kRankNeed : tn.heavy_need)) return kHeavyBin;
   int64_t slots = need << tn.load_shift;
   int bn = 1;
   while (bn < 9 && bin_table(bn) < slots) bn++;
