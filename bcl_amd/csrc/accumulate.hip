@@ -308,10 +308,12 @@ __global__ __launch_bounds__(kAccThreads, NUM ? (sizeof(T) == 8 ? 3 : 4) : 5) vo
         s_tcol[tid] = mine.col;
         if (NUM) s_tval[tid] = mine.val;
       }
-      const bool back = end < beg;  // only possible when the row is not sorted
-      const int len = back ? 0 : (int)(end - beg < kAccCap ? end - beg : kAccCap);
+      // only possible when the row is not sorted or a row_ptr changed meanwhile (a run cut short would pass every check
+      // that follows, so it is refused here)
+      const bool refused = end < beg || end - beg > kAccCap;
+      const int len = refused ? 0 : (int)(end - beg);
       const int inc = wave_incl_scan(len);
-      if (__ballot(back) != 0ull && tid == 0) D.bad[1] = 1;
+      if (__ballot(refused) != 0ull && tid == 0) D.bad[1] = 1;
       if (tid < K) s_seg[tid] = inc - len;
       if (tid == 63) s_seg[K] = inc;
       if (NUM && is_long) {  // entries of the row's earlier pieces
@@ -326,7 +328,7 @@ __global__ __launch_bounds__(kAccThreads, NUM ? (sizeof(T) == 8 ? 3 : 4) : 5) vo
     for (int s = tid; s < kAccCap; s += kAccThreads) s_mark[s] = 0;
     __syncthreads();
     const int E = s_seg[K];
-    if (E > kAccCap) {  // only possible when a row is not sorted or a row_ptr changed meanwhile
+    if (E > kAccCap) {  // likewise: runs that fit one by one, but not together
       if (tid == 0) D.bad[1] = 1;
       return;
     }
