@@ -543,13 +543,13 @@ static bool accumulate_merge(bclx_handle* h, int K, const bclx_csr* tiles, bclx_
   D.n = n;
   D.nchunks = (total_in + m) / kAccTarget + 1;
   D.max_pieces = (int32_t)max_pieces;
-  Arena ws;  // in the handle's scratch: this call waits for the stream before it returns
+  Arena ws;  // in a CallWorkspace: this call waits for the stream before it returns
   const size_t o_woff = ws.reserve(sizeof(int64_t) * (m + 4)), o_cnt = ws.reserve(sizeof(int32_t) * (m + 4)),
                o_off = ws.reserve(sizeof(int64_t) * (m + 4)), o_chunk = ws.reserve(sizeof(int32_t) * 2 * D.nchunks),
                o_piece = ws.reserve(sizeof(AccPiece) * max_pieces), o_bound = ws.reserve(sizeof(int64_t) * max_pieces * K),
                o_pcnt = ws.reserve(sizeof(int32_t) * max_pieces), o_part = ws.reserve(sizeof(long long) * scan_partials(m)),
                o_flag = ws.reserve(2 * sizeof(int64_t) + sizeof(int32_t));
-  ScratchUse use(h, ws);
+  CallWorkspace use(h, ws);
   D.woff = ws.at<int64_t>(o_woff);
   D.cnt = ws.at<int32_t>(o_cnt);
   D.off = ws.at<int64_t>(o_off);
@@ -596,7 +596,7 @@ static bool accumulate_merge(bclx_handle* h, int K, const bclx_csr* tiles, bclx_
   C->m = m;
   C->n = n;
   C->nnz = nnz;
-  BCLX_HIP(hipStreamSynchronize(s));  // C is complete, and the handle's scratch free, on return
+  BCLX_HIP(hipStreamSynchronize(s));  // C is complete, and the workspace free, on return
   return true;
 }
 

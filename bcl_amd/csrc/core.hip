@@ -25,6 +25,47 @@ void dev_free(void* p, const AllocFns& how) {
   if (how.free) how.free(p, how.user);
   else (void)hipFree(p);
 }
+
+// hipSuccess: the stream is not being captured. hipErrorStreamCaptureImplicit: it is, or is the null stream beside one
+// that is: it may not be waited for, nor events recorded on it. Others: not a stream any more.
+static hipError_t stream_state(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  const hipError_t e = hipStreamIsCapturing(s, &st);
+  if (e != hipSuccess) (void)hipGetLastError();
+  return e == hipSuccess && st != hipStreamCaptureStatusNone ? hipErrorStreamCaptureImplicit : e;
+}
+
+void finish_dense(bclx_handle* h) {
+  if (!h->scratch_used) return;
+  if (h->scratch_stream == h->stream) (void)hipStreamSynchronize(h->stream);
+  else (void)hipEventSynchronize(h->scratch_left);
+}
+
+void leave_dense(bclx_handle* h) {
+  if (!h->scratch_used || h->scratch_stream != h->stream) return;
+  const hipError_t e = stream_state(h->stream);
+  if (e == hipSuccess && hipEventRecord(h->scratch_left, h->stream) == hipSuccess) return;
+  if (e != hipErrorStreamCaptureImplicit) {  // destroyed before it was left
+    (void)hipGetLastError();
+    (void)hipDeviceSynchronize();
+  }
+  h->scratch_used = false;
+}
+
+// Under capture nothing runs yet, so nothing is waited for: ordering a graph's launches is the caller's.
+char* dense_scratch(bclx_handle* h, size_t bytes) {
+  const bool runs = stream_state(h->stream) == hipSuccess;
+  if (runs && h->scratch_used) {
+    if (bytes > h->scratch.bytes) finish_dense(h);
+    else if (h->scratch_stream != h->stream) BCLX_HIP(hipStreamWaitEvent(h->stream, h->scratch_left, 0));
+  }
+  h->scratch.reserve(bytes);
+  if (runs) {
+    h->scratch_used = true;
+    h->scratch_stream = h->stream;
+  }
+  return h->scratch.as<char>();
+}
 }  // namespace bclx
 
 using namespace bclx;
@@ -53,6 +94,7 @@ bclx_status bclx_create(int device, void* stream, bclx_handle** out) {
     h->lds_per_block = lds > 0 ? (size_t)lds : 65536;
     init_noalloc_scratch(device);
     BCLX_HIP(hipHostMalloc(reinterpret_cast<void**>(&h->h_pinned), sizeof(int64_t) * kPinnedCounts, hipHostMallocDefault));
+    BCLX_HIP(hipEventCreateWithFlags(&h->scratch_left, hipEventDisableTiming));
     *out = h.release();
   });
 }
@@ -62,6 +104,7 @@ bclx_status bclx_destroy(bclx_handle* h) {
     if (!h) return;
     (void)hipSetDevice(h->device);
     (void)hipStreamSynchronize(h->stream);
+    finish_dense(h);
     delete h;
   });
 }
@@ -78,7 +121,9 @@ bclx_status bclx_set_allocator(bclx_handle* h, bclx_alloc_fn alloc, bclx_free_fn
 bclx_status bclx_set_stream(bclx_handle* h, void* stream) {
   return guarded([&] {
     BCLX_REQUIRE(h != nullptr, BCLX_ERR_INVALID, "null handle");
-    if (h->stream != static_cast<hipStream_t>(stream)) h->stream_changes++;
+    if (h->stream == static_cast<hipStream_t>(stream)) return;
+    leave_dense(h);
+    h->stream_changes++;
     h->stream = static_cast<hipStream_t>(stream);
   });
 }

@@ -636,8 +636,7 @@ static void direct_run(bclx_handle* h, DirectArgs D, int bk, int splits, bool ap
   splits = (int)std::max<int64_t>(1, (nk + D.kt_per_split - 1) / D.kt_per_split);
   const dim3 grid((unsigned)(D.tiles_m * D.tiles_n), 1, (unsigned)splits);
   if (splits > 1 || apart) {  // partial products into the workspace, scaled and added to C afterwards
-    h->scratch.reserve(sizeof(T) * (size_t)splits * (size_t)(D.M * D.N));
-    T* ws = h->scratch.as<T>();
+    T* ws = reinterpret_cast<T*>(dense_scratch(h, sizeof(T) * (size_t)splits * (size_t)(D.M * D.N)));
     const int64_t ldc = D.ldc;
     D.ldc = D.N;
     D.split_stride = D.M * D.N;
@@ -715,8 +714,7 @@ static void gemm_run(bclx_handle* h, bool ta, bool tb, int64_t m, int64_t n, int
   const size_t lo_a = MODE == 2 ? (size_t)Mp * Kp * 2 : 0, lo_b = MODE == 2 ? (size_t)Np * Kp * 2 : 0;
   const size_t off_b = (a_bytes + 255) / 256 * 256, off_la = off_b + (b_bytes + 255) / 256 * 256;
   const size_t off_lb = off_la + (lo_a + 255) / 256 * 256, total = off_lb + lo_b + 256;
-  h->scratch.reserve(total);
-  char* ws = h->scratch.as<char>();
+  char* ws = dense_scratch(h, total);
   E* Ap = reinterpret_cast<E*>(ws);
   E* Bp = reinterpret_cast<E*>(ws + off_b);
   uint16_t* Al = MODE == 2 ? reinterpret_cast<uint16_t*>(ws + off_la) : nullptr;

@@ -117,8 +117,14 @@ struct bclx_handle {
   hipStream_t stream = nullptr;
   int num_cus = 256;
   size_t lds_per_block = 65536;
-  // scratch reused across calls (grow-only)
+  // operands and partial sums of dense products (grow-only; dense_scratch()). A product may still run when its call
+  // returns: scratch_stream is where the last one was launched, and where the handle is on another stream by now,
+  // scratch_left was recorded there when it moved on.
   bclx::DevBuf scratch;
+  bool scratch_used = false;
+  hipStream_t scratch_stream = nullptr;
+  hipEvent_t scratch_left = nullptr;
+  bclx::DevBuf call_ws;  // CallWorkspace; hipMalloc'd handles only
   bclx::DevBuf dense_slots;  // heavy-row dense accumulators, kept zeroed between uses
   size_t dense_slot_doubles = 0;
   int dense_nslots = 0;
@@ -129,6 +135,7 @@ struct bclx_handle {
   unsigned stream_changes = 0;  // bclx_set_stream calls that changed the stream
   ~bclx_handle() {
     if (h_pinned) (void)hipHostFree(h_pinned);
+    if (scratch_left) (void)hipEventDestroy(scratch_left);
   }
 };
 
@@ -162,22 +169,34 @@ inline void set_device(bclx_handle* h) {
 
 inline unsigned div_up(int64_t a, int64_t b) { return (unsigned)((a + b - 1) / b); }
 
-// The handle's scratch for a call that waits for its stream before it returns: grown on demand, and given back at the
-// end of a call that grew it beyond kScratchKeep (so one large call does not hold its memory until bclx_destroy).
-constexpr size_t kScratchKeep = size_t(1) << 30;
-struct ScratchUse {
+// Device memory of a call that waits for its stream before it returns, so nothing of the call still uses it then, on any
+// stream. Kept by the handle for the next such call, up to kCallKeep bytes; a handle with a caller's allocator keeps
+// nothing.
+constexpr size_t kCallKeep = size_t(1) << 30;
+struct CallWorkspace {
   bclx_handle* h;
-  size_t before;
-  ScratchUse(bclx_handle* h_, Arena& ws) : h(h_), before(h_->scratch.bytes) {
-    h->scratch.reserve(ws.used);
-    ws.use_external(h->scratch.p, h->scratch.bytes);
+  DevBuf own;
+  CallWorkspace(bclx_handle* h_, Arena& ws) : h(h_) {
+    DevBuf& b = h->alloc.alloc ? own : h->call_ws;
+    b.reserve(ws.used);
+    ws.use_external(b.p, b.bytes);
   }
-  ~ScratchUse() {
-    if (h->scratch.bytes <= kScratchKeep || h->scratch.bytes <= before) return;
+  ~CallWorkspace() {
+    if (!own.p && h->call_ws.bytes <= kCallKeep) return;
     (void)hipStreamSynchronize(h->stream);
-    h->scratch.release();
+    if (!own.p) h->call_ws.release();
   }
+  CallWorkspace(const CallWorkspace&) = delete;
+  CallWorkspace& operator=(const CallWorkspace&) = delete;
 };
+
+// The handle's scratch for a dense product on its stream: what an earlier product left running on another stream
+// (bclx_set_stream in between) comes first.
+char* dense_scratch(bclx_handle* h, size_t bytes);
+// Waits for the dense products that still use the scratch.
+void finish_dense(bclx_handle* h);
+// The handle is about to leave its stream.
+void leave_dense(bclx_handle* h);
 
 // Looks up, once per device and with that device current, the address of the fixed scratch array that
 // bclx_spgemm_noalloc works in.

@@ -217,14 +217,14 @@ void split_grid(bclx_handle* h, const bclx_csr* A, int64_t tile_m, int64_t tile_
   const int64_t m = A->m;
   const int64_t stride = m / 4 * 4 + 4;  // a tile column's counts, padded with zeros: off[tj * stride + m] is its end
   const int64_t L = stride * gn;
-  Arena ws;  // in the handle's scratch: this call waits for the stream before it returns
+  Arena ws;  // in a CallWorkspace: this call waits for the stream before it returns
   const size_t o_cnt = ws.reserve(sizeof(int32_t) * (size_t)L), o_seg = ws.reserve(sizeof(int32_t) * (size_t)L),
                o_off = ws.reserve(sizeof(int64_t) * (size_t)(L + 4)),
                o_part = ws.reserve(sizeof(long long) * (size_t)scan_partials(L)),
                o_tot = ws.reserve(sizeof(int64_t) * (size_t)(gm * gn + 1)),
                o_chunk = ws.reserve(sizeof(SplitChunk) * (size_t)((A->nnz + m) / kSplitChunk + 1)),
                o_tile = ws.reserve(sizeof(SplitTile) * (size_t)(gm * gn)), o_bad = ws.reserve(sizeof(int32_t));
-  ScratchUse use(h, ws);
+  CallWorkspace use(h, ws);
   int32_t* cnt = ws.at<int32_t>(o_cnt);
   int32_t* seg = ws.at<int32_t>(o_seg);
   int64_t* off = ws.at<int64_t>(o_off);
@@ -294,7 +294,7 @@ void split_grid(bclx_handle* h, const bclx_csr* A, int64_t tile_m, int64_t tile_
   } else {  // one row of tiles with no rows: each row_ptr is {0}
     for (int t = 0; t < gm * gn; t++) BCLX_HIP(hipMemsetAsync(tiles[t].row_ptr, 0, (size_t)tiles[t].ptr_width, s));
   }
-  BCLX_HIP(hipStreamSynchronize(s));  // the tiles are complete, and the handle's scratch free, on return
+  BCLX_HIP(hipStreamSynchronize(s));  // the tiles are complete, and the workspace free, on return
   BCLX_REQUIRE(h_bad == 0, BCLX_ERR_INVALID, "A's columns must be sorted within each row and below A->n");
 }
 

@@ -70,6 +70,8 @@ BCLX_API const char* bclx_last_error(void);
 /* Handle on `device` ordered on `stream` (a hipStream_t; NULL = the default stream). */
 BCLX_API bclx_status bclx_create(int device, void* stream, bclx_handle** out);
 BCLX_API bclx_status bclx_destroy(bclx_handle* h);
+/* Calls from here on are ordered on `stream`. A dense product still running on the stream that is left keeps its operands:
+ * a later one waits for it on the GPU before it uses the handle's scratch. */
 BCLX_API bclx_status bclx_set_stream(bclx_handle* h, void* stream);
 BCLX_API bclx_status bclx_synchronize(bclx_handle* h);
 
@@ -78,7 +80,9 @@ BCLX_API bclx_status bclx_synchronize(bclx_handle* h);
  * BCLX_ERR_ALLOC); free(ptr, user) releases it. Both NULL: hipMalloc / hipFree (the default). Replaces BCL's
  * Allocator template parameter (bcl/containers/sequential/CSRMatrix.hpp:32-36, rebound for the index arrays at
  * :41-42; bcl_allocator, bcl/core/alloc.hpp:60-105). Buffers are freed through the allocator that made them, so its
- * functions must stay valid until every plan made under them is destroyed. */
+ * functions must stay valid until every plan made under them is destroyed, and the handle where it ran dense products or
+ * wide heavy rows under them: their scratch stays with the handle. Sums and splits leave nothing behind in a handle with a
+ * caller's allocator; without one it keeps their workspace (up to 1 GiB) for the next call. */
 typedef void* (*bclx_alloc_fn)(size_t bytes, void* user);
 typedef void (*bclx_free_fn)(void* ptr, void* user);
 BCLX_API bclx_status bclx_set_allocator(bclx_handle* h, bclx_alloc_fn alloc, bclx_free_fn free_fn, void* user);
