@@ -10,7 +10,8 @@
 // Measured: eight R-MAT scale 16 tiles (11.2 M entries, fp32) 11.0 ms through the general path, 0.81 ms here.
 //
 // Tiles whose columns are not strictly increasing within each row, and sums of more than kAccMaxTiles tiles (one lane
-// per tile sets a piece up), take the general path: one SpGEMM [T_1 T_2 ... T_K] * [I; I; ...; I], where the left operand stacks the tiles side by side
+// per tile sets a piece up), and sums written over their own tiles, take the general path: one SpGEMM
+// [T_1 T_2 ... T_K] * [I; I; ...; I], where the left operand stacks copies of the tiles side by side
 // (row i of it is the concatenation of row i of every tile, tile t's columns shifted by t * n) and the right operand
 // stacks K identities. Every product is x * 1 (exact), so the two-phase SpGEMM returns exactly the union pattern,
 // sorted, with each entry summed in float64 and rounded once.
@@ -588,6 +589,14 @@ static bool accumulate_merge(bclx_handle* h, int K, const bclx_csr* tiles, bclx_
     BCLX_REQUIRE(C->nnz >= nnz, BCLX_ERR_INVALID, "C arrays smaller than the sum's entries");
     BCLX_REQUIRE(C->ptr_width == 8 || nnz <= INT32_MAX, BCLX_ERR_OVERFLOW,
                  "nnz(C) = " + std::to_string(nnz) + " does not fit an int32 row_ptr; request ptr_width 8");
+    // pieces are written while others still read their tiles
+    auto over = [&](const void* out, size_t bytes) {
+      return std::any_of(tiles, tiles + K, [&](const bclx_csr& x) {
+        return share_memory(out, bytes, x.row_ptr, sizeof(RP) * (m + 1)) ||
+               share_memory(out, bytes, x.col_idx, sizeof(int) * x.nnz) || share_memory(out, bytes, x.vals, sizeof(T) * x.nnz);
+      });
+    };
+    if (over(C->col_idx, sizeof(int) * nnz) || over(C->vals, sizeof(T) * nnz)) return false;
     hipLaunchKernelGGL((k_acc_merge<true, T, RP>), dim3(grid), dim3(kAccThreads), 0, s, D, nlong, C->col_idx,
                        static_cast<T*>(C->vals));
     BCLX_HIP(hipGetLastError());

@@ -167,6 +167,12 @@ inline void set_device(bclx_handle* h) {
   g_alloc = h->alloc;
 }
 
+// Do two arrays (n bytes each; none where n is 0) have memory in common?
+inline bool share_memory(const void* a, size_t na, const void* b, size_t nb) {
+  const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+  return na > 0 && nb > 0 && x < y + nb && y < x + na;
+}
+
 inline unsigned div_up(int64_t a, int64_t b) { return (unsigned)((a + b - 1) / b); }
 
 // Device memory of a call that waits for its stream before it returns, so nothing of the call still uses it then, on any
