@@ -46,6 +46,7 @@ template <typename T, typename RP>
 static void spgemm_noalloc(bclx_handle* h, const bclx_csr* A, const bclx_csr* B, bclx_csr* C) {
   const int64_t cap = C->nnz;
   TwoPhase<T, RP> W(h, make_tile<T, RP>(A, B), BinTuning{}, scratch_on(h->device), kScratchBytes);
+  W.reads(A, B);
   const int64_t nnz = W.symbolic();
   if (nnz > cap) {
     C->nnz = nnz;  // what a retry needs

@@ -4,6 +4,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <iterator>
 
 namespace bclx {
 
@@ -582,12 +583,17 @@ void TwoPhase<T, RP>::numeric(int* c_col, T* c_val, int64_t c_cap, void* row_ptr
   hipStream_t s = h->stream;
   F.tiles[0].c_col = c_col;
   F.tiles[0].c_val = c_val;
+  // row_ptr is written by the launch that sets C's arrays; last, where it is one of the operands' arrays
+  const bool last = std::any_of(std::begin(inputs), std::end(inputs), [&](const Range& x) {
+    return share_memory(row_ptr, (size_t)ptr_width * (m + 1), x.p, x.bytes);
+  });
   const unsigned g = div_up(m + 1, 256);
+  const int64_t now = last ? -1 : m;
   if (ptr_width == 8)
-    hipLaunchKernelGGL((k_begin_numeric<int64_t, T, RP>), dim3(g), dim3(256), 0, s, F.R, m, static_cast<int64_t*>(row_ptr),
+    hipLaunchKernelGGL((k_begin_numeric<int64_t, T, RP>), dim3(g), dim3(256), 0, s, F.R, now, static_cast<int64_t*>(row_ptr),
                        c_col, c_val);
   else
-    hipLaunchKernelGGL((k_begin_numeric<int32_t, T, RP>), dim3(g), dim3(256), 0, s, F.R, m, static_cast<int32_t*>(row_ptr),
+    hipLaunchKernelGGL((k_begin_numeric<int32_t, T, RP>), dim3(g), dim3(256), 0, s, F.R, now, static_cast<int32_t*>(row_ptr),
                        c_col, c_val);
   BCLX_HIP(hipGetLastError());
   F.R.out_limit = c_cap;
@@ -599,6 +605,12 @@ void TwoPhase<T, RP>::numeric(int* c_col, T* c_val, int64_t c_cap, void* row_ptr
     F.read_counts(s, counts);
   }
   for (int b = 1; b < kNumBins; b++) F.run_bin(s, 1, b, counts[b]);
+  if (!last) return;
+  if (ptr_width == 8)
+    hipLaunchKernelGGL(k_rowptr<int64_t>, dim3(g), dim3(256), 0, s, F.R.off, (int64_t)0, m, static_cast<int64_t*>(row_ptr));
+  else
+    hipLaunchKernelGGL(k_rowptr<int32_t>, dim3(g), dim3(256), 0, s, F.R.off, (int64_t)0, m, static_cast<int32_t*>(row_ptr));
+  BCLX_HIP(hipGetLastError());
 }
 
 template struct TwoPhase<float, int32_t>;
@@ -616,7 +628,10 @@ struct PlanBase {
 template <typename T, typename RP>
 struct TwoPhasePlan : PlanBase {
   TwoPhase<T, RP> tp;
-  TwoPhasePlan(bclx_handle* h, const bclx_csr* A, const bclx_csr* B) : tp(h, make_tile<T, RP>(A, B), BinTuning{}, nullptr, 0, true) {}
+  TwoPhasePlan(bclx_handle* h, const bclx_csr* A, const bclx_csr* B)
+      : tp(h, make_tile<T, RP>(A, B), BinTuning{}, nullptr, 0, true) {
+    tp.reads(A, B);
+  }
   int64_t symbolic() override { return tp.symbolic(); }
   void numeric(bclx_csr* C) override {
     BCLX_REQUIRE(C && C->row_ptr, BCLX_ERR_INVALID, "C or C->row_ptr is null");

@@ -105,6 +105,19 @@ struct TwoPhase {
   TwoPhase(const TwoPhase&) = delete;
   TwoPhase& operator=(const TwoPhase&) = delete;
   int64_t symbolic();
+  // A's and B's arrays, where the caller's row_ptr may be one of them
+  struct Range {
+    const void* p = nullptr;
+    size_t bytes = 0;
+  } inputs[6];
+  void reads(const bclx_csr* A, const bclx_csr* B) {
+    int q = 0;
+    for (const bclx_csr* x : {A, B}) {
+      inputs[q++] = {x->row_ptr, (size_t)(x->m + 1) * sizeof(RP)};
+      inputs[q++] = {x->col_idx, (size_t)x->nnz * sizeof(int)};
+      inputs[q++] = {x->vals, (size_t)x->nnz * sizeof(T)};
+    }
+  }
   // writes col/val into c_col/c_val (capacity c_cap entries) and row_ptr (m+1 entries of 4 or 8 bytes)
   void numeric(int* c_col, T* c_val, int64_t c_cap, void* row_ptr, int ptr_width);
 };

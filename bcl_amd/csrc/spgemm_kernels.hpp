@@ -2707,7 +2707,7 @@ __global__ void k_report(RowsDev<T, RP> R, const int64_t* total, int64_t* out) {
   if (threadIdx.x == kNumBins) out[kNumBins] = *total;
 }
 
-// One launch before the numeric pass: C's row_ptr, and the arrays its entries go to.
+// One launch before the numeric pass: C's row_ptr (m < 0: not yet), and the arrays its entries go to.
 template <typename OUT, typename T, typename RP>
 __global__ void k_begin_numeric(RowsDev<T, RP> R, int64_t m, OUT* rp, int* c_col, T* c_val) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
