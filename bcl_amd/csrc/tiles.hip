@@ -88,7 +88,8 @@ __device__ inline int64_t row_div(int64_t i, int64_t d, int64_t m) {
 
 // The tiles' row_ptrs from the scanned offsets: one thread per (tile column, row). The threads of tile column 0 also
 // cut A into chunks of kSplitChunk entries plus rows: row i weighs its entries and one more; chunk[c] is the row
-// that weight c * kSplitChunk falls in and the entry it stands for.
+// that weight c * kSplitChunk falls in and the entry it stands for. The entries are counted from rp[0] on: A may be rows
+// of a larger matrix, with its col_idx and vals.
 template <typename RP>
 __global__ __launch_bounds__(256) void k_split_rowptr(const RP* rp, const int64_t* off, int64_t stride, int64_t m,
                                                       int64_t tile_m, int gn, const SplitTile* tiles,
@@ -97,9 +98,9 @@ __global__ __launch_bounds__(256) void k_split_rowptr(const RP* rp, const int64_
   const int tj = blockIdx.y;
   if (i >= m) return;
   if (tj == 0) {
-    const int64_t a0 = (int64_t)rp[i], a1 = (int64_t)rp[i + 1];
+    const int64_t e0 = (int64_t)rp[0], a0 = (int64_t)rp[i] - e0, a1 = (int64_t)rp[i + 1] - e0;
     for (int64_t c = (a0 + i + kSplitChunk - 1) / kSplitChunk; c < nchunks && c * kSplitChunk <= a1 + i; c++)
-      chunk[c] = SplitChunk{i, c * kSplitChunk - i < a1 ? c * kSplitChunk - i : a1};
+      chunk[c] = SplitChunk{i, e0 + (c * kSplitChunk - i < a1 ? c * kSplitChunk - i : a1)};
   }
   const int64_t ti = row_div(i, tile_m, m), first = ti * tile_m, li = i - first;
   const int64_t rows = (m - first) < tile_m ? (m - first) : tile_m;
@@ -128,13 +129,13 @@ __global__ __launch_bounds__(256) void k_split_copy(const RP* rp, const int32_t*
                                                     int64_t n, int64_t tile_m, uint32_t tile_n, int gn,
                                                     const int64_t* off, const int32_t* seg, int64_t stride,
                                                     const SplitTile* tiles, const SplitChunk* chunk, int64_t nchunks,
-                                                    int64_t total, int32_t* bad) {
+                                                    int32_t* bad) {
   __shared__ int s_rp[kSplitWindow + 1];  // offsets less the window's first entry, from -1 (before it) to kSplitChunk
   __shared__ int64_t s_first, s_end;      // first and last offset
   const int tid = threadIdx.x;
   const int64_t b = blockIdx.x;
   // the chunk's rows [r0, r1] and entries [e, c1)
-  const SplitChunk from = chunk[b], to = b + 1 < nchunks ? chunk[b + 1] : SplitChunk{m - 1, total};
+  const SplitChunk from = chunk[b], to = b + 1 < nchunks ? chunk[b + 1] : SplitChunk{m - 1, (int64_t)rp[m]};
   int64_t r0 = from.row, e = from.entry;
   const int64_t r1 = to.row, c1 = to.entry;
   while (e < c1 && r0 <= r1) {
@@ -203,7 +204,7 @@ template <typename RP>
 __global__ void k_split_totals(const RP* rp, const int64_t* off, int64_t ostride, int64_t m, int64_t tile_m, int gm,
                                int gn, int64_t* tot) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t == gm * gn) tot[t] = (int64_t)rp[m];
+  if (t == gm * gn) tot[t] = (int64_t)rp[m] - (int64_t)rp[0];
   if (t >= gm * gn) return;
   const int ti = t / gn, tj = t - ti * gn;
   const int64_t r0 = (int64_t)ti * tile_m, r1 = (r0 + tile_m) < m ? (r0 + tile_m) : m;
@@ -287,7 +288,7 @@ void split_grid(bclx_handle* h, const bclx_csr* A, int64_t tile_m, int64_t tile_
     if (entries > 0) {
       hipLaunchKernelGGL((k_split_copy<RP, T>), dim3((unsigned)nchunks), dim3(256), 0, s, rp, A->col_idx,
                          static_cast<const T*>(A->vals), m, A->n, tile_m, (uint32_t)std::min<int64_t>(tile_n, UINT32_MAX),
-                         gn, off, seg, stride, dt, chunk, nchunks, entries, bad);
+                         gn, off, seg, stride, dt, chunk, nchunks, bad);
       BCLX_HIP(hipGetLastError());
     }
     BCLX_HIP(hipMemcpyAsync(&h_bad, bad, sizeof(int32_t), hipMemcpyDeviceToHost, s));
