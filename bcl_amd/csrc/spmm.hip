@@ -25,7 +25,7 @@ namespace bclx {
 
 constexpr int kSpmmThreads = 256;
 
-// Largest r in [0, m) with rp[r] <= e (e < rp[m]): one wavefront, 64 probes a round.
+// Largest r in [0, m) with rp[r] <= e, 0 if there is none: one wavefront, 64 probes a round.
 template <typename RP>
 __device__ inline int64_t spmm_row_of(const RP* rp, int64_t m, int64_t e, int lane) {
   int64_t lo = 0, len = m;
@@ -33,7 +33,7 @@ __device__ inline int64_t spmm_row_of(const RP* rp, int64_t m, int64_t e, int la
     const int64_t step = (len + 63) / 64;
     const int64_t q = lo + lane * step;
     const bool le = q < lo + len && (int64_t)rp[q] <= e;
-    const int k = __popcll(__ballot(le)) - 1;  // rp is monotone: the probes at or before e come first
+    const int hits = (int)__popcll(__ballot(le)), k = hits > 0 ? hits - 1 : 0;  // rp is monotone: hits come first
     const int64_t end = lo + len;
     lo += k * step;
     len = step < end - lo ? step : end - lo;
@@ -61,7 +61,9 @@ __global__ __launch_bounds__(kSpmmThreads) void k_spmm(const RP* __restrict__ rp
   typedef VT cvec_t __attribute__((ext_vector_type(VEC), aligned(sizeof(VT))));
   __shared__ int s_col[PADDED];
   __shared__ VT s_val[PADDED];
-  __shared__ uint16_t s_row[PADDED];  // per entry: first slot of its row in the block << 1 | shared
+  // per entry: first slot of its row in the block << 1 | shared. Entries of no row (rp may start above 0 or end below nnz)
+  // count as a shared row that is not listed in s_shared.
+  __shared__ uint16_t s_row[PADDED];
   __shared__ int s_id[EPB];           // at a row's first slot: the row, relative to the block's first
   __shared__ VT s_sum[GROUPS + 1][COLS];  // sums of the rows that several groups share
   __shared__ int s_shared[GROUPS + 1];    // those rows << 1 | crosses the block's ends, or -1
@@ -78,7 +80,7 @@ __global__ __launch_bounds__(kSpmmThreads) void k_spmm(const RP* __restrict__ rp
     const int x = q * kSpmmThreads + tid;
     s_col[slot(x)] = x < cnt ? col[e0 + x] : 0;
     s_val[slot(x)] = x < cnt ? val[e0 + x] : VT(0);
-    s_row[slot(x)] = 0;
+    s_row[slot(x)] = x == 0 ? 1 : 0;
   }
   if (tid < U) s_col[PADDED - U + tid] = 0;  // read, not used, by the last group
   for (int x = tid; x < (GROUPS + 1) * COLS; x += kSpmmThreads) s_sum[x / COLS][x % COLS] = VT(0);
@@ -100,6 +102,7 @@ __global__ __launch_bounds__(kSpmmThreads) void k_spmm(const RP* __restrict__ rp
       s_id[first] = (int)(r - r0);
       if (sh) s_shared[place(first)] = (int)(r - r0) << 1 | (cross ? 1 : 0);
     }
+    if (r == m - 1 && e > 0 && e < cnt) s_row[slot((int)e)] = (uint16_t)(e << 1 | 1);
     if (__syncthreads_or(r < m && e >= cnt)) break;
   }
   {
