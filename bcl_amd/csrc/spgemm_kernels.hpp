@@ -1641,9 +1641,10 @@ __global__ __launch_bounds__(64 * W, 6) void k_esc_block(RowsDev<T, RP> R, int b
 //   k_heavy_rank<0> counts each part's entries (symbolic: and the whole rows')
 //   k_heavy_place   sums a row's parts and, in modes 2 and 3, gives them their places in C
 //   k_heavy_rank    the parts (largest pieces) first, then the whole rows, from one queue
-// A part finds its share of each B row by binary search. Nothing else needs a B row's columns sorted, so the counting pass
-// checks each product's column against the part's range: the parts' shares tile every B row, so if all
-// columns are inside, nothing is missed. Otherwise the row runs whole.
+// A part finds its share of each B row by binary search, and so does a slice of a row or part of several slices. B rows
+// should be sorted, but nothing is lost where they are not: the counting pass checks each product's column against the
+// part's range, and the numeric pass against the slice's. Shares tile every B row (or part of it), so if all columns are
+// inside, nothing is missed. Otherwise the row runs whole, or its slices again over all of its products.
 // R-MAT square at scale 16 (122 M products): symbolic 0.53 -> 0.20 ms, numeric 1.76 -> 0.62 ms with the parts, the
 // product loop of enumerate_waves and a word of the bitmap per lane when the columns are written. Bound now by LDS latency and
 // atomics with one workgroup of 16 wavefronts per CU.
@@ -2040,6 +2041,7 @@ __global__ __launch_bounds__(hr_block<MODE>()) void k_heavy_rank(RowsDev<T, RP> 
   __shared__ __align__(16) double s_acc[NUM ? kHRSlice : 1];  // a slice's columns (as int), then its values
   __shared__ long long s_base;
   __shared__ int s_crange[2];
+  __shared__ int s_outside;  // a product of a slice's share is not in the slice's columns
   __shared__ RP s_delta[BLOCK];
   // product prefixes of one staged chunk fit 32 bits: at most BLOCK entries, each a B row of at most 2^19 columns
   __shared__ int s_pre[BLOCK];
@@ -2271,6 +2273,7 @@ __global__ __launch_bounds__(hr_block<MODE>()) void k_heavy_rank(RowsDev<T, RP> 
           atomicAdd(&R.stats[1], 1ull);
         }
         s_base = b;
+        s_outside = 0;
       }
       __syncthreads();
       const long long base = uniform(s_base);
@@ -2282,6 +2285,7 @@ __global__ __launch_bounds__(hr_block<MODE>()) void k_heavy_rank(RowsDev<T, RP> 
       // one rank slice at a time: columns (staged in LDS by rank, then stored with unit stride), then values. A
       // slice's first column and each entry's first B position in it are where the previous slice ended.
       RP my_lo = 0;
+      bool search = one_chunk || part;  // each slice finds its share of the B rows (uniform)
       for (int s0 = 0; s0 < total; s0 += kHRSlice) {
         const int len = total - s0 < kHRSlice ? total - s0 : kHRSlice;
         const bool whole = s0 == 0 && len == total;
@@ -2330,19 +2334,25 @@ __global__ __launch_bounds__(hr_block<MODE>()) void k_heavy_rank(RowsDev<T, RP> 
         auto add = [&](int j, T a, T b) {
           if (whole || (j >= c_lo && j < c_hi))
             atomicAdd(&s_acc[hr_rank(s_bits, s_gpre, j) - s0], (double)a * (double)b);
+          else
+            s_outside = 1;
         };
         RP st = my_st;
         int ln = my_len;
-        if (one_chunk && !whole && tid < na) {  // the part of the entry's B row inside the slice's columns
+        if (search && one_chunk && !whole && tid < na) {  // the part of the entry's B row inside the slice's columns
           const RP x = my_lo;
           const RP y = s0 + len >= total ? (RP)my_len : hr_lower_bound(tile.b_col, my_st, x, (RP)my_len, c_hi);
           st = my_st + x;
           ln = (int)(y - x);
           my_lo = y;
         }
-        run_row(st, ln, c_lo, c_hi, add, std::true_type{});
+        run_row(st, ln, search ? c_lo : lo, search ? c_hi : hi, add, std::true_type{});
         for (int t = tid; t < len; t += BLOCK) __builtin_nontemporal_store((T)s_acc[t], &glob(tile.c_val)[base + s0 + t]);
         __syncthreads();
+        if (!whole && search && s0 + len >= total && uniform(s_outside)) {  // an unsorted B row: all slices again
+          search = false;
+          s0 = -kHRSlice;
+        }
       }
     } while (false);
     advance(6);  // rows that ended early (symbolic, refused, skipped) finish the next row's fetch here
