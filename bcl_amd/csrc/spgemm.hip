@@ -95,6 +95,7 @@ void FlatRows<T, RP>::layout(bool with_cap, bool pooled, bool* from_pool) {
   R.bin_count = A.at<int32_t>(o_bc);
   R.bin_items = A.at<int32_t>(o_bi);
   R.bin_stride = nflat;
+  R.rank_kernel = (max_n + 31) / 32 <= kHRWords;
   R.ovf_count = A.at<int32_t>(o_oc);
   R.ovf_items = A.at<int32_t>(o_oi);
   R.pred_count = R.ovf_count + 1;
@@ -288,7 +289,7 @@ void launch_esc_block(const RowsDev<T, RP>& R, hipStream_t s, int mode, int b, u
 
 template <typename T, typename RP>
 void FlatRows<T, RP>::plan_heavy(hipStream_t s, int mode) {
-  if ((max_n + 31) / 32 > kHRWords) return;  // the wide-tile kernel runs every row whole
+  if (!R.rank_kernel) return;  // the wide-tile kernel runs every row whole
   if (mode == 1) {
     hipLaunchKernelGGL((k_order_heavy<false, T, RP>), dim3(1), dim3(1024), 0, s, R);  // the symbolic pass split them
   } else {
@@ -356,7 +357,7 @@ void FlatRows<T, RP>::run_bin(hipStream_t s, int mode, int b, int64_t count_hint
     }
     return;
   }
-  if (b == kHeavyBin && (max_n + 31) / 32 <= kHRWords) {
+  if (b == kHeavyBin && R.rank_kernel) {
     if (!planned) plan_heavy(s, mode);
     // persistent: the parts of split rows and the whole rows are taken from a queue
     const unsigned cus = (unsigned)h->num_cus;
@@ -469,7 +470,7 @@ void FlatRows<T, RP>::prepare_heavy() {
   // The rank-slice kernel keeps everything in LDS. The global dense fallback (tiles wider than 2^19 columns) needs
   // one accumulator of max_n doubles per resident workgroup, and a zeroed bitmap per workgroup when the tile is too
   // wide for an LDS bitmap; the kernel leaves both zeroed behind every row.
-  if ((max_n + 31) / 32 <= kHRWords) return;
+  if (R.rank_kernel) return;
   ensure_dense_slots(h, h->num_cus, (size_t)max_n);
   const int64_t words = (max_n + 31) / 32;
   if (heavy_lds_bitmap()) {

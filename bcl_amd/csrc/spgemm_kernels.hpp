@@ -38,8 +38,9 @@ __host__ __device__ constexpr int bin_group(int b) {
   return b == 1 ? 16 : b == 2 ? 32 : b <= 5 ? 64 : b == 6 ? 256 : b <= 8 ? 512 : 1024;
 }
 
-// Tiles at most 2^19 columns wide: rows of more than 4096 products that need more entries than this run in the
-// rank-slice kernel of the heavy bin, whatever heavy_need allows to hash. 20000 rows of 6400 products: 3190 entries
+// Where every tile of the batch is at most 2^19 columns wide: rows of more than 4096 products that need more entries than
+// this run in the rank-slice kernel of the heavy bin, whatever heavy_need allows to hash. (One wider tile gives the batch's
+// heavy rows to the wide-tile kernel, whose accumulator is in HBM.) 20000 rows of 6400 products: 3190 entries
 // 2.1 ms there and 7.8 ms hashed, 1918 entries 2.1 and 4.3 ms, 998 entries 2.1 and 1.95 ms; rows of 90000 products with
 // 1500 entries 2.3 and 3.3 ms; R-MAT square at scale 16 1.79 and 2.34 ms.
 constexpr int kRankNeed = 1024;
@@ -61,13 +62,14 @@ __host__ __device__ inline int esc_bin(int64_t work) {
 }
 
 // n: the tile's width. Rows of at most 32 products sort in registers (tiles narrower than 2^27 - 1 columns); longer
-// rows sort in the ESC bins when the columns fit their packed key (n <= 2^19). esc_max = 0 turns both off.
-__host__ __device__ inline int bin_for(int64_t need, int64_t work, const BinTuning& tn, int64_t n) {
+// rows sort in the ESC bins when the columns fit their packed key (n <= 2^19). esc_max = 0 turns both off. rank_kernel: the
+// batch's heavy rows run in the rank-slice kernel.
+__host__ __device__ inline int bin_for(int64_t need, int64_t work, const BinTuning& tn, int64_t n, bool rank_kernel) {
   if (work <= 0) return 0;
   if (tn.esc_max > 0 && work <= kSmallMax && n < ((int64_t)1 << kSmallColBits) - 1) return kSmallBin;
   const bool esc_ok = n <= (1 << kEscColBits);
   if (esc_ok && work > tn.esc_min && work <= tn.esc_max && work <= kEscMaxProducts) return esc_bin(work);
-  const bool rank = esc_ok && work > kEscMaxProducts;  // the rank-slice kernel takes it from kRankNeed on
+  const bool rank = rank_kernel && work > kEscMaxProducts;  // the rank-slice kernel takes it from kRankNeed on
   if (need > (rank && tn.heavy_need > kRankNeed ? kRankNeed : tn.heavy_need)) return kHeavyBin;
   int64_t slots = need << tn.load_shift;
   int bn = 1;
@@ -161,6 +163,7 @@ struct RowsDev {
   HeavyPart* heavy_parts;           // kMaxHeavyParts
   int32_t* heavy_first;             // per row of the heavy bin: its first part, -1 if it is not split
   unsigned long long* stats;   // [0] products [1] heavy rows [2] overflow rows [3] capacity exceeded [4] predicted
+  bool rank_kernel;            // every tile fits the rank-slice kernel (k_heavy_rank), which then runs the heavy bin
   long long out_limit;         // entries available in the output arrays; writes beyond it are refused
   BinTuning tn;
 };
@@ -336,7 +339,7 @@ __global__ __launch_bounds__(kRowBlock) void k_analyze(RowsDev<T, RP> R, int64_t
     }
     if (in[s]) R.prod[fr] = valid[s] ? prod[s] : 0;
     ub0[s] = prod[s] < (long long)tp[s]->n ? prod[s] : (long long)tp[s]->n;
-    b0[s] = valid[s] ? bin_for(ub0[s], prod[s], R.tn, tp[s]->n) : 0;
+    b0[s] = valid[s] ? bin_for(ub0[s], prod[s], R.tn, tp[s]->n, R.rank_kernel) : 0;
     if (with_stats && b0[s] == kHeavyBin) atomicAdd(&R.stats[5], 1ull);
     pr[s] = false;
   }
@@ -417,7 +420,7 @@ __global__ __launch_bounds__(kRowBlock) void k_analyze_long(RowsDev<T, RP> R, in
     if (lane == 0) {
       R.prod[fr] = prod;
       const long long ub0 = prod < (long long)t->n ? prod : (long long)t->n;
-      const int b0 = bin_for(ub0, prod, R.tn, t->n);
+      const int b0 = bin_for(ub0, prod, R.tn, t->n, R.rank_kernel);
       if (with_stats) {
         atomicAdd(&R.stats[0], (unsigned long long)prod);
         if (b0 == kHeavyBin) atomicAdd(&R.stats[5], 1ull);
@@ -452,7 +455,7 @@ __global__ __launch_bounds__(kRowBlock) void k_bin(RowsDev<T, RP> R, int src) {
   if (valid) {
     const long long work = R.prod[fr];
     const long long need = src == 0 ? (long long)R.nnz[fr] : (long long)R.cap[fr];
-    b = (need == 0 && src == 0) ? 0 : bin_for(need, work, R.tn, tile.n);
+    b = (need == 0 && src == 0) ? 0 : bin_for(need, work, R.tn, tile.n, R.rank_kernel);
   }
   int pos = 0;
   if (b > 0) pos = atomicAdd(&s_bcount[b], 1);
@@ -2104,7 +2107,7 @@ __global__ __launch_bounds__(hr_block<MODE>()) void k_heavy_rank(RowsDev<T, RP> 
             n_off = R.heavy_parts[n_idx].off;
             if (MODE == 1) {  // the row may hash now that its count is known, or not fit
               n_off += R.off[n_fr];
-              n_skip = n_skip || bin_for(R.nnz[n_fr], R.prod[n_fr], R.tn, t.n) != kHeavyBin;
+              n_skip = n_skip || bin_for(R.nnz[n_fr], R.prod[n_fr], R.tn, t.n, true) != kHeavyBin;
               if (!n_skip && R.off[n_fr] + R.nnz[n_fr] > R.out_limit) {
                 if (tid == 0) R.stats[3] = 1ull;
                 n_skip = true;

@@ -63,7 +63,7 @@ __global__ __launch_bounds__(256) void k_bin_predicted(RowsDev<T, RP> R) {
     if (idx < cnt) {
       fr = R.pred_items[idx];
       const TileDev<T, RP> tile = R.tiles[R.blk_tile[fr >> 8]];
-      b = bin_for(R.cap[fr], R.prod[fr], R.tn, tile.n);
+      b = bin_for(R.cap[fr], R.prod[fr], R.tn, tile.n, R.rank_kernel);
       pos = atomicAdd(&s_cnt[b], 1);
     }
     __syncthreads();
@@ -84,7 +84,7 @@ __global__ __launch_bounds__(256) void k_ovf_bin(RowsDev<T, RP> R) {
     const TileDev<T, RP> tile = R.tiles[R.blk_tile[fr >> 8]];
     const long long prod = R.prod[fr];
     const long long ub = prod < (long long)tile.n ? prod : (long long)tile.n;
-    const int b = bin_for(ub, prod, R.tn, tile.n);
+    const int b = bin_for(ub, prod, R.tn, tile.n, R.rank_kernel);
     const int pos = atomicAdd(R.count_of(b), 1);
     R.bin_items[(int64_t)b * R.bin_stride + pos] = fr;
   }

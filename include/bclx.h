@@ -134,8 +134,8 @@ typedef struct {
   const int32_t* h_tuning;   /* optional BCLX_TUNING_LEN binning knobs (autotuned), NULL = defaults:
                               *   [0] work_per_lane (64)  lanes per row >= products / work_per_lane
                               *   [1] heavy_need (4096)   rows needing more slots use the heavy accumulator (rows of
-                              *                         more than 4096 products on tiles up to 2^19 columns:
-                              *                         from 1024 on)
+                              *                         more than 4096 products, where all tiles of the stage
+                              *                         have at most 2^19 columns: from 1024 on)
                               *   [2] load_shift (1)      hash slots >= need << load_shift
                               *   [3] esc_min (32)        rows with esc_min < products <= esc_max are sorted
                               *   [4] esc_max (4096)      instead of hashed (0 turns sorting off; max 4096)
