@@ -92,17 +92,16 @@ __global__ __launch_bounds__(kSpmmThreads) void k_spmm(const RP* __restrict__ rp
   __syncthreads();
   // rows of the entries: shared when the row has entries in another block or more than one group's run here
   const int64_t r0 = s_first;
-  for (int64_t w = r0; w < m; w += kSpmmThreads) {
-    const int64_t r = w + tid;
-    const int64_t b = r < m ? (int64_t)rp[r] - e0 : cnt, e = r < m ? (int64_t)rp[r + 1] - e0 : cnt;
+  for (int64_t w = r0; w <= m; w += kSpmmThreads) {
+    const int64_t r = w + tid;  // row m: the entries after the last row, which are not listed
+    const int64_t b = r <= m ? (int64_t)rp[r] - e0 : cnt, e = r < m ? (int64_t)rp[r + 1] - e0 : cnt;
     if (b < cnt && e > b && e > 0) {
       const int first = b > 0 ? (int)b : 0;
-      const bool cross = b < 0 || e > cnt, sh = cross || e - b > RUN;
+      const bool cross = b < 0 || e > cnt, sh = cross || e - b > RUN || r == m;
       s_row[slot(first)] = (uint16_t)(first << 1 | (sh ? 1 : 0));
       s_id[first] = (int)(r - r0);
-      if (sh) s_shared[place(first)] = (int)(r - r0) << 1 | (cross ? 1 : 0);
+      if (sh && r < m) s_shared[place(first)] = (int)(r - r0) << 1 | (cross ? 1 : 0);
     }
-    if (r == m - 1 && e > 0 && e < cnt) s_row[slot((int)e)] = (uint16_t)(e << 1 | 1);
     if (__syncthreads_or(r < m && e >= cnt)) break;
   }
   {
