@@ -258,15 +258,16 @@ static void scale_rows(bclx_handle* h, VT* C, int64_t m, int64_t n, int64_t ldc,
 
 template <typename RP, typename VT, typename BT, int LPE, int VEC>
 static void spmm_launch(bclx_handle* h, const bclx_csr* A, const BT* B, int64_t ldb, VT* C, int64_t ldc, int64_t n,
-                        VT alpha, bool fresh) {
+                        VT alpha, bool fresh, bool whole_lines) {
   const RP* rp = static_cast<const RP*>(A->row_ptr);
   const int64_t slices = (n + LPE * VEC - 1) / (LPE * VEC);
   constexpr int64_t kMaxY = 32768;  // grid rows of one launch
   // 2048 entries per block (fp64: 1024, the same LDS) where that gives every CU four blocks (one, for narrow products,
   // whose groups' runs are short), else 512. Measured, us, 512 against 2048: 200 K rows of 9, fp32, 1 column 21.6 / 15.3,
-  // 64 columns 72 / 68; 20 K rows of 9, 64 columns 15 / 34.
+  // 64 columns 72 / 68; 20 K rows of 9, 64 columns 15 / 34. Always 512 where wide rows of B are not whole lines
+  // (100 K rows of 32, fp32, 33 columns 95 / 115, 129 columns 393 / 411; fp64, 33 columns 162 / 169).
   constexpr int kLarge = sizeof(VT) == 8 ? 1024 : 2048;
-  const bool large = (A->nnz / kLarge) * slices >= (LPE <= 4 ? 1 : 4) * (int64_t)h->num_cus;
+  const bool large = whole_lines && (A->nnz / kLarge) * slices >= (LPE <= 4 ? 1 : 4) * (int64_t)h->num_cus;
   const int epb = large ? kLarge : 512;
   if (fresh) {
     hipLaunchKernelGGL((k_spmm_clear<RP, VT>), dim3(div_up(A->m, 256)), dim3(256), 0, h->stream, rp, A->m, A->nnz, epb, C,
@@ -298,7 +299,8 @@ static void spmm_impl(bclx_handle* h, const bclx_csr* A, const void* Bv, int64_t
     if (fresh) scale_rows<VT>(h, C, A->m, n, ldc, VT(0));
     return;
   }
-#define BCLX_SPMM(LPE, VEC) spmm_launch<RP, VT, BT, LPE, VEC>(h, A, B, ldb, C, ldc, n, alpha, fresh)
+#define BCLX_SPMM(LPE, VEC) spmm_launch<RP, VT, BT, LPE, VEC>(h, A, B, ldb, C, ldc, n, alpha, fresh, true)
+#define BCLX_SPMM_LINES(LPE, VEC) spmm_launch<RP, VT, BT, LPE, VEC>(h, A, B, ldb, C, ldc, n, alpha, fresh, lines)
   // Slices of 256 bytes of a B row where rows are whole 128-byte lines: half as many lanes idle at odd widths and a
   // smaller B to gather from at a time (fp32 x 128 columns: 899 us against 1036 with 512-byte slices). Where rows are
   // not, a slice's ends share lines with its neighbours, and 512-byte slices gather fewer lines (fp32 x 100 columns, 200 K
@@ -318,8 +320,8 @@ static void spmm_impl(bclx_handle* h, const bclx_csr* A, const void* Bv, int64_t
     else if (n > 1) BCLX_SPMM(2, 1);
     else BCLX_SPMM(1, 1);
   } else if constexpr (sizeof(BT) == 4) {
-    if (n > 64 && !lines) BCLX_SPMM(32, 4);
-    else if (n > 32 && !vec16) BCLX_SPMM(32, 2);
+    if (n > 64 && !lines) BCLX_SPMM_LINES(32, 4);
+    else if (n > 32 && !vec16) BCLX_SPMM_LINES(32, 2);
     else if (n > 32) BCLX_SPMM(16, 4);
     else if (n > 16 && !vec16) BCLX_SPMM(16, 2);
     else if (n > 16) BCLX_SPMM(8, 4);
@@ -328,13 +330,17 @@ static void spmm_impl(bclx_handle* h, const bclx_csr* A, const void* Bv, int64_t
     else if (n > 1) BCLX_SPMM(2, 2);
     else BCLX_SPMM(1, 1);
   } else {
-    if (n > 32 && !lines) BCLX_SPMM(32, 2);
+    // fp64 rows that are not whole lines: slices of 1024 bytes where the last one is more than half used, else of 512
+    // (200 K rows of 9, x 127 columns 361 us against 415, x 145 columns 506 against 478)
+    if (n > 64 && !lines && (n - 1) % 128 >= 64) BCLX_SPMM_LINES(32, 4);
+    else if (n > 32 && !lines) BCLX_SPMM_LINES(32, 2);
     else if (n > 16) BCLX_SPMM(16, 2);
     else if (n > 8) BCLX_SPMM(8, 2);
     else if (n > 4) BCLX_SPMM(4, 2);
     else if (n > 1) BCLX_SPMM(2, 2);
     else BCLX_SPMM(1, 1);
   }
+#undef BCLX_SPMM_LINES
 #undef BCLX_SPMM
 }
 
