@@ -114,6 +114,10 @@ bclx_status bclx_set_allocator(bclx_handle* h, bclx_alloc_fn alloc, bclx_free_fn
     BCLX_REQUIRE(h != nullptr, BCLX_ERR_INVALID, "null handle");
     BCLX_REQUIRE((alloc == nullptr) == (free_fn == nullptr), BCLX_ERR_INVALID,
                  "give both allocator functions, or neither (hipMalloc / hipFree)");
+    // what the handle keeps for later calls, and no call or plan uses now, goes back to the allocator it came from
+    BCLX_HIP(hipSetDevice(h->device));
+    h->call_ws.release();
+    if (!h->plan_ws_busy) h->plan_ws.release();
     h->alloc = AllocFns{alloc, free_fn, user};
   });
 }

@@ -81,8 +81,9 @@ BCLX_API bclx_status bclx_synchronize(bclx_handle* h);
  * Allocator template parameter (bcl/containers/sequential/CSRMatrix.hpp:32-36, rebound for the index arrays at
  * :41-42; bcl_allocator, bcl/core/alloc.hpp:60-105). Buffers are freed through the allocator that made them, so its
  * functions must stay valid until every plan made under them is destroyed, and the handle where it ran dense products or
- * wide heavy rows under them: their scratch stays with the handle. Sums and splits leave nothing behind in a handle with a
- * caller's allocator; without one it keeps their workspace (up to 1 GiB) for the next call. */
+ * wide heavy rows under them: their scratch stays with the handle. A handle without a caller's allocator keeps the
+ * workspace of its last spgemm plan (up to 4 GiB) and of its last sum or split (up to 1 GiB) for the next one; this call
+ * gives both back (but for a plan that still exists), also where it sets the allocator that is set. */
 typedef void* (*bclx_alloc_fn)(size_t bytes, void* user);
 typedef void (*bclx_free_fn)(void* ptr, void* user);
 BCLX_API bclx_status bclx_set_allocator(bclx_handle* h, bclx_alloc_fn alloc, bclx_free_fn free_fn, void* user);
@@ -92,7 +93,8 @@ BCLX_API bclx_status bclx_set_allocator(bclx_handle* h, bclx_alloc_fn alloc, bcl
  * nnz(C). numeric: fills caller-allocated C (row_ptr m+1 of C->ptr_width, col_idx/vals of nnz) with sorted
  * columns and values accumulated in float64 and rounded once to C->dtype. A and B must share dtype and
  * ptr_width. C->ptr_width 4 fails with BCLX_ERR_OVERFLOW when nnz(C) > 2^31 - 1. The handle keeps the device workspace
- * of the last plan (up to 4 GiB) for the next one until bclx_destroy, unless it has a caller's allocator. */
+ * of the last plan (up to 4 GiB) for the next one until bclx_destroy or bclx_set_allocator, unless it has a caller's
+ * allocator. */
 BCLX_API bclx_status bclx_spgemm_symbolic(bclx_handle* h, const bclx_csr* A, const bclx_csr* B,
                                           bclx_spgemm_plan** plan, int64_t* nnz_c);
 BCLX_API bclx_status bclx_spgemm_numeric(bclx_spgemm_plan* plan, bclx_csr* C);
