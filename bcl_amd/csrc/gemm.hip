@@ -48,24 +48,17 @@ constexpr int kGThreads = 256;
 // C tile of block b. XCD-aware: block b runs on XCD b % 8, so each XCD is given a contiguous run of the order below.
 // The order walks groups of kTileGroup tile rows column by column, so the blocks an XCD runs at one time cover a
 // near-square patch of C and share their A and B panels in that XCD's L2 (a row-major order would share one A
-// panel and stream every B panel through L2; measured 8% slower on the BF16 8192^3 product). GROUPED = false keeps
-// the row-major order.
+// panel and stream every B panel through L2; measured 8% slower on the BF16 8192^3 product).
 constexpr int kTileGroup = 4;
-template <bool GROUPED>
 __device__ inline void gemm_tile_of(int b, int tiles_m, int tiles_n, int& tm, int& tn) {
   const int T = tiles_m * tiles_n;
   if (T % 8 == 0) b = (b % 8) * (T / 8) + (b / 8);
-  if constexpr (GROUPED) {
-    const int per_group = kTileGroup * tiles_n;
-    const int first = (b / per_group) * kTileGroup;
-    const int rows = tiles_m - first < kTileGroup ? tiles_m - first : kTileGroup;
-    const int r = b % per_group;
-    tm = first + r % rows;
-    tn = r / rows;
-  } else {
-    tm = b / tiles_n;
-    tn = b % tiles_n;
-  }
+  const int per_group = kTileGroup * tiles_n;
+  const int first = (b / per_group) * kTileGroup;
+  const int rows = tiles_m - first < kTileGroup ? tiles_m - first : kTileGroup;
+  const int r = b % per_group;
+  tm = first + r % rows;
+  tn = r / rows;
 }
 
 __device__ inline uint16_t f32_to_bf16_rne(float x) {
@@ -184,7 +177,7 @@ __global__ __launch_bounds__(kGThreads, TM * TN > 4 ? 2 : 1) void k_gemm(const t
   __shared__ __align__(16) E Bs[NSPLIT][BN * LDK];
 
   int tm, tn;
-  gemm_tile_of<true>(blockIdx.x, tiles_m, tiles_n, tm, tn);
+  gemm_tile_of(blockIdx.x, tiles_m, tiles_n, tm, tn);
   const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -413,7 +406,7 @@ __global__ __launch_bounds__(kGThreads, 2) void k_gemm_direct(DirectArgs D, cons
   __shared__ __align__(16) E As[NSPLIT][BM * LDK];
   __shared__ __align__(16) E Bs[NSPLIT][BN * LDK];
   int tm, tn;
-  gemm_tile_of<true>(blockIdx.x, D.tiles_m, D.tiles_n, tm, tn);
+  gemm_tile_of(blockIdx.x, D.tiles_m, D.tiles_n, tm, tn);
   const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
@@ -517,7 +510,7 @@ __global__ __launch_bounds__(kGThreads, 3) void k_gemm_f64_direct(DirectArgs D, 
   __shared__ __align__(16) double As[BM * LDK];
   __shared__ __align__(16) double Bs[BM * LDK];
   int tm, tn;
-  gemm_tile_of<true>(blockIdx.x, D.tiles_m, D.tiles_n, tm, tn);
+  gemm_tile_of(blockIdx.x, D.tiles_m, D.tiles_n, tm, tn);
   const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BM;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
