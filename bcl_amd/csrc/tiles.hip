@@ -14,7 +14,7 @@
 //      finds its entry's row in a window of row offsets in LDS, its tile column by a division, and writes the entry to
 //      its tile at (row offset + position in the segment).
 // Bytes: A's row_ptr and col_idx are read twice (count, copy) and its values once; every tile is written once. Measured
-// on R-MAT scale 20 (15.7 M entries, 4 x 4 tiles), sizes and copy together: 1.82 ms with one wavefront per row and
+// on R-MAT scale 20 (16.1 M entries, 4 x 4 tiles), sizes and copy together: 1.82 ms with one wavefront per row and
 // one scan per tile column, 0.43 ms this way.
 //
 // bclx_dense_binary_op is DMatrix's elementwise arithmetic on a tile (DMatrix::binary_op / binary_op_inplace,
