@@ -47,6 +47,7 @@ void leave_dense(bclx_handle* h) {
   if (e == hipSuccess && hipEventRecord(h->scratch_left, h->stream) == hipSuccess) return;
   if (e != hipErrorStreamCaptureImplicit) {  // destroyed before it was left
     (void)hipGetLastError();
+    (void)hipSetDevice(h->device);
     (void)hipDeviceSynchronize();
   }
   h->scratch_used = false;
